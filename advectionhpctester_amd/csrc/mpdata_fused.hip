@@ -48,10 +48,7 @@ hipError_t Fused<T>::step(const Geo& g, const T* x, T* xout, const T* u1, const 
     choose_tiling<T>(g, cfg, cl);
     if (iters == 3) {
         if (!sc || !sc->x2 || !sc->ul[0] || !sc->ul[1] || !sc->ul[2]) return hipErrorInvalidValue;
-        e = launch_three<T, false>(g, o, cfg, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
-        if (e != hipSuccess) return e;
-        k_copy_untouched_halo<T><<<256, 256, 0, s>>>(g, x, xout);
-        return hipGetLastError();
+        return launch_three<T, false>(g, o, cfg, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
     }
     switch (cfg) {
         case 1: e = launch2<T, 32, 16, 4>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
@@ -60,9 +57,7 @@ hipError_t Fused<T>::step(const Geo& g, const T* x, T* xout, const T* u1, const 
         case 4: e = launch2<T, 16, 32, 2>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
         default: e = launch2<T, 32, 32, 4>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
     }
-    if (e != hipSuccess) return e;
-    k_copy_untouched_halo<T><<<256, 256, 0, s>>>(g, x, xout);
-    return hipGetLastError();
+    return e;
 }
 
 // 32x16 tiles at 2 waves per SIMD (140 VGPRs, no spill), one workgroup
@@ -149,14 +144,11 @@ hipError_t FusedBatch<T>::step(const void* table, int n, int nitem, int cfg, lon
     hipError_t e = hipErrorInvalidValue;
     switch (cfg) {
 #define LAUNCH(c, rx, ry, mb) \
-    case c: e = launch_batch<T, rx, ry, mb>(table, n, nitem, shared, s); break;
+    case c: e = launch_batch<T, rx, ry, mb>(table, n, nitem, shared, max_halo, s); break;
         MPDATA_BATCH_CONFIGS(LAUNCH)
 #undef LAUNCH
     }
-    if (e != hipSuccess) return e;
-    const int bx = (int)std::min<long long>(64, (max_halo + 255) / 256);
-    k_copy_untouched_halo_batch<T><<<dim3(std::max(bx, 1), n), 256, 0, s>>>((const Member<T>*)table);
-    return hipGetLastError();
+    return e;
 }
 
 // Batch tiling for n members on one grid (configuration numbers of

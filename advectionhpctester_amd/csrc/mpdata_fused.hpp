@@ -150,7 +150,7 @@ struct BatchMember {
 };
 
 // The fused step over many domains of different shapes in one persistent
-// launch (plus one halo-copy launch).  The caller packs a descriptor table
+// launch (the halo copy included).  The caller packs a descriptor table
 // on the host (pack), copies it to device memory and launches with it.
 template <typename T>
 struct FusedBatch;

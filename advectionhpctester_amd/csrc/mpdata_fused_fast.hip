@@ -19,20 +19,13 @@ hipError_t FusedFast<T>::step(const Geo& g, const T* x, T* xout, const T* u1, co
     choose_tiling<T>(g, cfg, cl);
     if (iters == 3) {
         if (!sc || !sc->x2 || !sc->ul[0] || !sc->ul[1] || !sc->ul[2]) return hipErrorInvalidValue;
-        const hipError_t e =
-            launch_three<T, true>(g, o, cfg, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
-        if (e != hipSuccess) return e;
-        k_copy_untouched_halo<T><<<256, 256, 0, s>>>(g, x, xout);
-        return hipGetLastError();
+        return launch_three<T, true>(g, o, cfg, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
     }
     // the two tilings the chooser picks (32x32 lanes, 32x16 lanes at four
     // waves per SIMD); the tuning overrides of the exact build are not built
-    const hipError_t e =
-        cfg == 0 ? launch2<T, 32, 32, 4, true>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
-                 : launch2<T, 32, 16, 4, true>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
-    if (e != hipSuccess) return e;
-    k_copy_untouched_halo<T><<<256, 256, 0, s>>>(g, x, xout);
-    return hipGetLastError();
+    return cfg == 0
+               ? launch2<T, 32, 32, 4, true>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
+               : launch2<T, 32, 16, 4, true>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
 }
 
 template <typename T>
@@ -41,14 +34,11 @@ hipError_t FusedBatchFast<T>::step(const void* table, int n, int nitem, int cfg,
     hipError_t e = hipErrorInvalidValue;
     switch (cfg) {
 #define LAUNCH(c, rx, ry, mb) \
-    case c: e = launch_batch<T, rx, ry, mb, true>(table, n, nitem, shared, s); break;
+    case c: e = launch_batch<T, rx, ry, mb, true>(table, n, nitem, shared, max_halo, s); break;
         MPDATA_BATCH_CONFIGS(LAUNCH)
 #undef LAUNCH
     }
-    if (e != hipSuccess) return e;
-    const int bx = (int)std::min<long long>(64, (max_halo + 255) / 256);
-    k_copy_untouched_halo_batch<T><<<dim3(std::max(bx, 1), n), 256, 0, s>>>((const Member<T>*)table);
-    return hipGetLastError();
+    return e;
 }
 
 template <typename T>

@@ -776,14 +776,77 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     }
 }
 
+// Halo cells of x_out that the step does not define keep their x_in values:
+// the z-halo planes and the x/y halo cells outside the edge copies (all x/y
+// halo cells of a periodic direction, which the step leaves alone).  Cell q
+// of the three halo slabs -> its offset, or -1 for an edge copy (written by
+// the step itself).  32-bit: the arrays have below 2^31 elements.
+__device__ __forceinline__ int untouched_halo_cell(const Geo& g, uint32_t q, uint32_t nz_slab,
+                                                   uint32_t ny_slab) {
+    const uint32_t ih = g.ih, nx = g.np + 2 * ih, ny = g.mp + 2 * ih;
+    int i, j, k;
+    bool copy = true;
+    if (q < nz_slab) {
+        const uint32_t layer = q / (nx * ny), r = q - layer * (nx * ny), row = r / nx;
+        k = layer < ih ? 1 - (int)ih + (int)layer : g.lp + 1 + (int)(layer - ih);
+        i = (int)(r - row * nx) + 1 - (int)ih;
+        j = (int)row + 1 - (int)ih;
+    } else if (q < nz_slab + ny_slab) {
+        const uint32_t r = q - nz_slab, tt = r / nx, row = tt % (2 * ih);
+        i = (int)(r - tt * nx) + 1 - (int)ih;
+        k = (int)(tt / (2 * ih)) + 1;
+        j = row < ih ? 1 - (int)ih + (int)row : g.mp + 1 + (int)(row - ih);
+        copy = g.py || !((j == 0 || j == g.mp + 1) && i >= 1 && i <= g.np);
+    } else {
+        const uint32_t r = q - nz_slab - ny_slab, tt = r / (2 * ih), col = r - tt * (2 * ih);
+        k = (int)(tt / (uint32_t)g.mp) + 1;
+        j = (int)(tt - (uint32_t)(k - 1) * (uint32_t)g.mp) + 1;
+        i = col < ih ? 1 - (int)ih + (int)col : g.np + 1 + (int)(col - ih);
+        copy = g.px || !(i == 0 || i == g.np + 1);
+    }
+    return copy ? (int)off_raw<SCAL>(g, i, j, k) : -1;
+}
+
+// Block b of nb copies its share of them.  The step kernels are launched with
+// a few blocks more than they have places for work items (halo_blocks), which
+// do this and nothing else: they run on what the items leave idle, where a
+// kernel of its own came after them (13 us of 1.67 ms at 512x512x256, 4 us
+// and a launch of 28 us at 59^3).
+template <typename T>
+__device__ __forceinline__ void copy_untouched_halo(const Geo& g, const T* __restrict__ x,
+                                                    T* __restrict__ xo, uint32_t b, uint32_t nb) {
+    const uint32_t ih = g.ih, nx = g.np + 2 * ih, ny = g.mp + 2 * ih;
+    const uint32_t nz_slab = 2 * ih * nx * ny;        // k outside 1..lp
+    const uint32_t ny_slab = 2 * ih * nx * g.lp;      // k in 1..lp, j outside 1..mp
+    const uint32_t nx_slab = 2 * ih * g.mp * g.lp;    // k, j inside, i outside 1..np
+    const uint32_t total = nz_slab + ny_slab + nx_slab;
+    for (uint32_t q = b * blockDim.x + threadIdx.x; q < total; q += nb * blockDim.x) {
+        const int c = untouched_halo_cell(g, q, nz_slab, ny_slab);
+        if (c >= 0) xo[c] = x[c];
+    }
+}
+inline long long halo_cells(const Geo& g) {
+    const long long ih = g.ih, nx = g.np + 2 * ih, ny = g.mp + 2 * ih;
+    return 2 * ih * (nx * ny + nx * g.lp + (long long)g.mp * g.lp);
+}
+// blocks of nt threads for `cells` halo cells: four cells a thread, at most a
+// quarter of the chip's CUs
+inline int halo_blocks(long long cells, int nt) {
+    return (int)std::max(1LL, std::min(64LL, (cells + 4LL * nt - 1) / (4LL * nt)));
+}
+
 template <typename T, int RX, int RY, int MINB, bool FAST = false, int PASS = 0>
 __global__ void __launch_bounds__(RX * RY, MINB)
-k_fused_gauge2(Geo g, Off o, int ntx, int nty, int nchunk, int clen,
+k_fused_gauge2(Geo g, Off o, int nitemwg, int ntx, int nty, int nchunk, int clen,
                const T* __restrict__ x, const T* __restrict__ u1, const T* __restrict__ u2,
                const T* __restrict__ u3, const T* __restrict__ rhr, const T* __restrict__ h,
                const T* __restrict__ bcx, const T* __restrict__ bcy, T* __restrict__ xo,
                PassIO<T> pio) {
     __shared__ FusedLds<T, RX, RY> L;
+    if (blockIdx.x >= (unsigned)nitemwg) {
+        copy_untouched_halo<T>(g, x, xo, blockIdx.x - nitemwg, gridDim.x - nitemwg);
+        return;
+    }
     const int ntile = ntx * nty;
     // Work-item order: workgroups are dealt to the XCDs round-robin
     // (blockIdx % NXCD), each with its own L2.  The workgroups of one XCD
@@ -792,11 +855,10 @@ k_fused_gauge2(Geo g, Off o, int ntx, int nty, int nchunk, int clen,
     // the halo columns in that L2.  (A split into equal contiguous plane
     // ranges per workgroup balances the tail better but loses this
     // alignment and measured slower.)
-    const int nxcd = gridDim.x >= NXCD ? NXCD : 1;
-    const int per_xcd = gridDim.x / nxcd;                 // workgroups per XCD
+    const int nxcd = nitemwg >= NXCD ? NXCD : 1;
+    const int per_xcd = nitemwg / nxcd;                   // workgroups per XCD
     const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
-    const int nwg = per_xcd * nxcd;                       // workgroups that take items
-    if (blockIdx.x >= nwg) return;
+    if ((int)blockIdx.x >= per_xcd * nxcd) return;
     const int tiles_per_xcd = (ntile + nxcd - 1) / nxcd;
     for (int r = slot; ; r += per_xcd) {
         const int chunk = r / tiles_per_xcd, tix = r - chunk * tiles_per_xcd;
@@ -833,58 +895,6 @@ k_fused_gauge_rec(Geo g, Off o, int ntx, int nty, int nchunk, int clen, const T*
         const int k0 = 1 + chunk * clen, k1 = min(g.lp, k0 + clen - 1);
         fused_item<T, RX, RY, false, false, 0, true>(g, o, ntx, tile, k0, k1, x, u1, u2, u3, rhr,
                                                      h, bcx, bcy, xo, L, nullptr, nullptr, &tp);
-    }
-}
-
-// Halo cells of x_out that the step does not define keep their x_in values:
-// the z-halo planes and the x/y halo cells outside the edge copies (all x/y
-// halo cells of a periodic direction, which the step leaves alone).  Cell q
-// of the three halo slabs -> its offset, or -1 for an edge copy (written by
-// the step itself).
-__device__ __forceinline__ long long untouched_halo_cell(const Geo& g, long long q,
-                                                         long long nz_slab, long long ny_slab) {
-    const int ih = g.ih;
-    const long long nx = g.np + 2 * ih, ny = g.mp + 2 * ih;
-    int i, j, k;
-    bool copy = true;
-    if (q < nz_slab) {
-        long long r = q % (nx * ny);
-        int layer = (int)(q / (nx * ny));
-        k = layer < ih ? 1 - ih + layer : g.lp + 1 + (layer - ih);
-        i = (int)(r % nx) + 1 - ih;
-        j = (int)(r / nx) + 1 - ih;
-    } else if (q < nz_slab + ny_slab) {
-        long long r = q - nz_slab;
-        i = (int)(r % nx) + 1 - ih;
-        long long tt = r / nx;
-        int row = (int)(tt % (2 * ih));
-        k = (int)(tt / (2 * ih)) + 1;
-        j = row < ih ? 1 - ih + row : g.mp + 1 + (row - ih);
-        copy = g.py || !((j == 0 || j == g.mp + 1) && i >= 1 && i <= g.np);
-    } else {
-        long long r = q - nz_slab - ny_slab;
-        int col = (int)(r % (2 * ih));
-        long long tt = r / (2 * ih);
-        j = (int)(tt % g.mp) + 1;
-        k = (int)(tt / g.mp) + 1;
-        i = col < ih ? 1 - ih + col : g.np + 1 + (col - ih);
-        copy = g.px || !(i == 0 || i == g.np + 1);
-    }
-    return copy ? off_raw<SCAL>(g, i, j, k) : -1;
-}
-
-template <typename T>
-__global__ void k_copy_untouched_halo(Geo g, const T* __restrict__ x, T* __restrict__ xo) {
-    const int ih = g.ih;
-    const long long nx = g.np + 2 * ih, ny = g.mp + 2 * ih;
-    const long long nz_slab = 2ll * ih * nx * ny;      // k outside 1..lp
-    const long long ny_slab = 2ll * ih * nx * g.lp;    // k in 1..lp, j outside 1..mp
-    const long long nx_slab = 2ll * ih * g.mp * g.lp;  // k, j inside, i outside 1..np
-    const long long total = nz_slab + ny_slab + nx_slab;
-    for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < total;
-         q += (long long)gridDim.x * blockDim.x) {
-        const long long c = untouched_halo_cell(g, q, nz_slab, ny_slab);
-        if (c >= 0) xo[c] = x[c];
     }
 }
 
@@ -1052,8 +1062,10 @@ hipError_t launch2(const Geo& g, const Off& o, int clen, const T* x, T* xout, co
     if (e != hipSuccess) return e;
     const int grid = persistent_grid(nitem, (long long)(ntx * nty + NXCD - 1) / NXCD * nchunk, ncu,
                                      per_cu);
-    k_fused_gauge2<T, RX, RY, MINB, FAST, PASS><<<grid, RX * RY, 0, s>>>(
-        g, o, ntx, nty, nchunk, clen, x, u1, u2, u3, rhr, h, bcx, bcy, xout, pio);
+    // PASS 1 writes an intermediate, whose halo nothing reads
+    const int hb = PASS == 1 ? 0 : halo_blocks(halo_cells(g), RX * RY);
+    k_fused_gauge2<T, RX, RY, MINB, FAST, PASS><<<grid + hb, RX * RY, 0, s>>>(
+        g, o, grid, ntx, nty, nchunk, clen, x, u1, u2, u3, rhr, h, bcx, bcy, xout, pio);
     return hipGetLastError();
 }
 
@@ -1175,13 +1187,20 @@ size_t sched_offset(int n) {
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
 __global__ void __launch_bounds__(RX * RY, MINB)
 k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int shared,
-                     BatchSched* __restrict__ sc) {
+                     BatchSched* __restrict__ sc, int nitemwg) {
     __shared__ FusedLds<T, RX, RY> L;
     __shared__ int s_w;
-    const int nxcd = gridDim.x >= NXCD ? NXCD : 1;
-    const int per_xcd = gridDim.x / nxcd;
+    if (blockIdx.x >= (unsigned)nitemwg) {
+        for (int q = 0; q < nmem; q++) {
+            const Member<T>& m = mem[q];
+            copy_untouched_halo<T>(m.g, m.x, m.xo, blockIdx.x - nitemwg, gridDim.x - nitemwg);
+        }
+        return;
+    }
+    const int nxcd = nitemwg >= NXCD ? NXCD : 1;
+    const int per_xcd = nitemwg / nxcd;
     const int xcd = blockIdx.x % nxcd;
-    if (blockIdx.x >= per_xcd * nxcd) return;
+    if ((int)blockIdx.x >= per_xcd * nxcd) return;
     int w0, w1;  // this XCD's run
     if (nxcd == 1) {
         w0 = 0;
@@ -1240,24 +1259,6 @@ k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int
     if (threadIdx.x == 0 && atomicAdd(&sc->done[xcd], 1) == per_xcd - 1) {
         atomicExch(&sc->next[xcd], 0);
         atomicExch(&sc->done[xcd], 0);
-    }
-}
-
-// Halo copies of every member (blockIdx.y = member).
-template <typename T>
-__global__ void k_copy_untouched_halo_batch(const Member<T>* __restrict__ mem) {
-    const Member<T>& m = mem[blockIdx.y];
-    const Geo g = m.g;
-    const int ih = g.ih;
-    const long long nx = g.np + 2 * ih, ny = g.mp + 2 * ih;
-    const long long nz_slab = 2ll * ih * nx * ny;
-    const long long ny_slab = 2ll * ih * nx * g.lp;
-    const long long nx_slab = 2ll * ih * g.mp * g.lp;
-    const long long total = nz_slab + ny_slab + nx_slab;
-    for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < total;
-         q += (long long)gridDim.x * blockDim.x) {
-        const long long c = untouched_halo_cell(g, q, nz_slab, ny_slab);
-        if (c >= 0) m.xo[c] = m.x[c];
     }
 }
 
@@ -1365,7 +1366,8 @@ int pack_members(const BatchMember<T>* bm, int n, int clen, Member<T>* out) {
     X(5, 32, 32, 4)
 
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
-hipError_t launch_batch(const void* table, int n, int nitem, int shared, hipStream_t s) {
+hipError_t launch_batch(const void* table, int n, int nitem, int shared, long long max_halo,
+                        hipStream_t s) {
     int dev = 0, ncu = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -1376,8 +1378,9 @@ hipError_t launch_batch(const void* table, int n, int nitem, int shared, hipStre
     const int grid = persistent_grid(nitem, ((long long)nitem + NXCD - 1) / NXCD, ncu, per_cu);
     BatchSched* sc = reinterpret_cast<BatchSched*>(
         reinterpret_cast<char*>(const_cast<void*>(table)) + sched_offset<T>(n));
-    k_fused_gauge2_batch<T, RX, RY, MINB, FAST><<<grid, RX * RY, 0, s>>>(
-        (const Member<T>*)table, n, nitem, shared, sc);
+    const int hb = halo_blocks(max_halo * n, RX * RY);
+    k_fused_gauge2_batch<T, RX, RY, MINB, FAST><<<grid + hb, RX * RY, 0, s>>>(
+        (const Member<T>*)table, n, nitem, shared, sc, grid);
     return hipGetLastError();
 }
 

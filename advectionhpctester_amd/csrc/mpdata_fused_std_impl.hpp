@@ -610,18 +610,21 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
 template <typename T, int RX, int RY, int MINB, bool NONOS, bool PER, bool TAPE = false,
           bool FAST = false>
 __global__ void __launch_bounds__(RX * RY, MINB)
-k_fused_std(Geo g, Off o, int ntx, int nty, int nchunk, int clen, const T* __restrict__ x,
+k_fused_std(Geo g, Off o, int nitemwg, int ntx, int nty, int nchunk, int clen, const T* __restrict__ x,
             const T* __restrict__ u1, const T* __restrict__ u2, const T* __restrict__ u3,
             const T* __restrict__ rhr, const T* __restrict__ h, const T* __restrict__ bcx,
             const T* __restrict__ bcy, T* __restrict__ xo, StdTape<T> tp) {
     __shared__ StdLds<T, RX, RY> L;
+    if (blockIdx.x >= (unsigned)nitemwg) {
+        copy_untouched_halo<T>(g, x, xo, blockIdx.x - nitemwg, gridDim.x - nitemwg);
+        return;
+    }
     // work-item order of k_fused_gauge2: contiguous tile runs per XCD
     const int ntile = ntx * nty;
-    const int nxcd = gridDim.x >= NXCD ? NXCD : 1;
-    const int per_xcd = gridDim.x / nxcd;
+    const int nxcd = nitemwg >= NXCD ? NXCD : 1;
+    const int per_xcd = nitemwg / nxcd;
     const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
-    const int nwg = per_xcd * nxcd;
-    if (blockIdx.x >= nwg) return;
+    if ((int)blockIdx.x >= per_xcd * nxcd) return;
     const int tiles_per_xcd = (ntile + nxcd - 1) / nxcd;
     for (int r = slot; ; r += per_xcd) {
         const int chunk = r / tiles_per_xcd, tix = r - chunk * tiles_per_xcd;
@@ -651,8 +654,10 @@ hipError_t launch_std(const Geo& g, const Off& o, int clen, const T* x, T* xout,
     if (e != hipSuccess) return e;
     const int grid = persistent_grid(nitem, (long long)(ntx * nty + NXCD - 1) / NXCD * nchunk, ncu,
                                      per_cu);
-    k_fused_std<T, RX, RY, MINB, NONOS, PER, TAPE, FAST><<<grid, RX * RY, 0, s>>>(
-        g, o, ntx, nty, nchunk, clen, x, u1, u2, u3, rhr, h, bcx, bcy, xout, tp);
+    // a recorded step leaves the halo of its output alone
+    const int hb = TAPE ? 0 : halo_blocks(halo_cells(g), RX * RY);
+    k_fused_std<T, RX, RY, MINB, NONOS, PER, TAPE, FAST><<<grid + hb, RX * RY, 0, s>>>(
+        g, o, grid, ntx, nty, nchunk, clen, x, u1, u2, u3, rhr, h, bcx, bcy, xout, tp);
     return hipGetLastError();
 }
 
@@ -696,9 +701,7 @@ hipError_t std_step(const Geo& g, int nonos, const T* x, T* xout, const T* u1, c
         cfg == 0
             ? launch_std_any<T, 32, 32, 4, FAST>(g, o, cl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
             : launch_std_any<T, 32, 16, 4, FAST>(g, o, cl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
-    if (e != hipSuccess) return e;
-    k_copy_untouched_halo<T><<<256, 256, 0, s>>>(g, x, xout);
-    return hipGetLastError();
+    return e;
 }
 
 }  // namespace

@@ -474,7 +474,7 @@ int mpdata_ce_advection_oop_f32(mpdata_ctx *ctx, int alg_choice, int liner, int 
  * No counterpart in the reference (its batching is many fields on one grid,
  * advection_CEtimestep_twostep_GPUBC.f90).  n members of different shapes
  * (ih = 1, open walls), each advanced by the fused gauge step (2 iterations,
- * limiter on) in ONE persistent launch per step (plus one halo-copy launch);
+ * limiter on) in ONE persistent launch per step (the halo copy included);
  * a time loop can be captured into a HIP graph and launched once.  Results
  * are bit-identical to mpdata_step_oop_* on each member. */
 typedef struct mpdata_ens mpdata_ens;

@@ -160,3 +160,33 @@ def test_fused_standard_rejects_three_iterations(mp):
         with pytest.raises(mp.MpdataError) as e:
             d.step(x, *u, one, one, bcx, bcx, variant=STANDARD, iters=3)
         assert e.value.code == 4
+
+
+@pytest.mark.parametrize("variant,ibc", [("gauge", (0, 0, 0)), ("standard", (0, 0, 0)),
+                                         ("standard", (1, 0, 1)), ("standard", (1, 1, 1))])
+@pytest.mark.parametrize("dims", [(3, 3, 3, 1), (4, 3, 3, 3), (33, 29, 5, 2), (300, 210, 9, 1)])
+def test_fused_output_halo(mp, variant, ibc, dims):
+    """Every halo cell of the output, from less than one block of them to
+    many blocks: the input's value, but for the edge copies of open x/y walls,
+    which are the input's interior neighbours (exact copies: no tolerance)."""
+    n, m, l, ih = dims
+    c = _case(dims, sum(dims), np.float64)
+    with mp.Domain(*dims, ibc=ibc) as d:
+        t = {k: to_dev(v) for k, v in c.items()}
+        xo = torch.full_like(t["x"], float("nan"))
+        d.set_path(mp.PATH_FUSED)
+        print(f"output halo {variant} dims={dims} ibc={ibc}", flush=True)
+        d.step_oop(t["x"], xo, t["u1"], t["u2"], t["u3"], t["rhr"], t["h"], t["bcx"], t["bcy"],
+                   variant=mp.GAUGE if variant == "gauge" else STANDARD)
+        got = to_host(xo)
+    want = c["x"].copy()
+    ks = js = is_ = slice(ih, -ih)
+    if not ibc[0]:
+        want[ks, js, ih - 1] = c["x"][ks, js, ih]
+        want[ks, js, ih + n] = c["x"][ks, js, ih + n - 1]
+    if not ibc[1]:
+        want[ks, ih - 1, is_] = c["x"][ks, ih, is_]
+        want[ks, ih + m, is_] = c["x"][ks, ih + m - 1, is_]
+    want[ks, js, is_] = got[ks, js, is_]
+    assert not np.isnan(got).any()
+    assert bits_equal(want, got), describe_diff(want, got)
