@@ -43,21 +43,18 @@ hipError_t Fused<T>::step(const Geo& g, const T* x, T* xout, const T* u1, const 
                           const T* u3, const T* rhr, const T* h, const T* bcx, const T* bcy,
                           hipStream_t s, int iters, const FusedScratch<T>* sc) {
     const Off o = make_off(g);
-    hipError_t e = hipSuccess;
-    int cfg = 0, cl = 64;
-    choose_tiling<T>(g, cfg, cl);
+    const Tiling tl = choose_tiling<T>(g);
     if (iters == 3) {
         if (!sc || !sc->x2 || !sc->ul[0] || !sc->ul[1] || !sc->ul[2]) return hipErrorInvalidValue;
-        return launch_three<T, false>(g, o, cfg, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
+        return launch_three<T, false>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
     }
-    switch (cfg) {
-        case 1: e = launch2<T, 32, 16, 4>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
-        case 2: e = launch2<T, 32, 16, 2>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
-        case 3: e = launch2<T, 64, 16, 4>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
-        case 4: e = launch2<T, 16, 32, 2>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
-        default: e = launch2<T, 32, 32, 4>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s); break;
+    switch (tl.cfg) {
+        case 1: return launch2<T, 32, 16, 4>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+        case 2: return launch2<T, 32, 16, 2>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+        case 3: return launch2<T, 64, 16, 4>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+        case 4: return launch2<T, 16, 32, 2>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+        default: return launch2<T, 32, 32, 4>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
     }
-    return e;
 }
 
 // 32x16 tiles at 2 waves per SIMD (140 VGPRs, no spill), one workgroup
@@ -73,25 +70,14 @@ hipError_t Fused<T>::record(const Geo& g, const T* x, T* xout, const T* u1, cons
     constexpr int RX = 32, RY = 16, MINB = 2;
     if (g.px || g.py || g.pz || g.ih != 1) return hipErrorInvalidValue;
     const Off o = make_off(g);
-    const int env_clen = fused_chunk_env();
-    int clen = env_clen > 0 ? env_clen : chunk_by_rounds<RX, RY>(g, k_fused_gauge_rec<T, RX, RY, MINB>);
-    if (clen > g.lp) clen = g.lp;
-    const int ntx = (g.np + RX - 5) / (RX - 4), nty = (g.mp + RY - 5) / (RY - 4);
-    const int nchunk = (g.lp + clen - 1) / clen;
-    int dev = 0, ncu = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fused_gauge_rec<T, RX, RY, MINB>,
-                                                         RX * RY, 0);
+    long long slots = 0;
+    const hipError_t e = resident(k_fused_gauge_rec<T, RX, RY, MINB>, RX * RY, 0, slots);
     if (e != hipSuccess) return e;
-    const int grid = persistent_grid((long long)ntx * nty * nchunk,
-                                     (long long)(ntx * nty + NXCD - 1) / NXCD * nchunk, ncu, per_cu);
+    const March m = plan_march<RX, RY>(g, slots, fused_chunk_env());
     // xout: the interior and the edge copies; the other halo cells are left
     // alone (the recorded step defines only the interior)
-    k_fused_gauge_rec<T, RX, RY, MINB><<<grid, RX * RY, 0, s>>>(g, o, ntx, nty, nchunk, clen, x,
-                                                                 u1, u2, u3, rhr, h, bcx, bcy,
-                                                                 xout, tp);
+    k_fused_gauge_rec<T, RX, RY, MINB><<<m.nwg, RX * RY, 0, s>>>(g, o, m, x, u1, u2, u3, rhr, h,
+                                                                  bcx, bcy, xout, tp);
     return hipGetLastError();
 }
 

@@ -15,17 +15,16 @@ hipError_t FusedFast<T>::step(const Geo& g, const T* x, T* xout, const T* u1, co
                               const T* u3, const T* rhr, const T* h, const T* bcx, const T* bcy,
                               hipStream_t s, int iters, const FusedScratch<T>* sc) {
     const Off o = make_off(g);
-    int cfg = 0, cl = 64;
-    choose_tiling<T>(g, cfg, cl);
+    const Tiling tl = choose_tiling<T>(g);
     if (iters == 3) {
         if (!sc || !sc->x2 || !sc->ul[0] || !sc->ul[1] || !sc->ul[2]) return hipErrorInvalidValue;
-        return launch_three<T, true>(g, o, cfg, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
+        return launch_three<T, true>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, *sc, s);
     }
     // the two tilings the chooser picks (32x32 lanes, 32x16 lanes at four
     // waves per SIMD); the tuning overrides of the exact build are not built
-    return cfg == 0
-               ? launch2<T, 32, 32, 4, true>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
-               : launch2<T, 32, 16, 4, true>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+    return tl.cfg == 0
+               ? launch2<T, 32, 32, 4, true>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
+               : launch2<T, 32, 16, 4, true>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
 }
 
 template <typename T>

@@ -56,11 +56,24 @@ __device__ __forceinline__ int mirror(int i, int n) { return i == 0 ? 2 : (i == 
 // per-lane 64-bit address arithmetic.
 template <typename T>
 __device__ __forceinline__ T ldo(const T* p, uint32_t off) {
-    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + off);
+    typedef const __attribute__((address_space(1))) char* G;
+    return *(const __attribute__((address_space(1))) T*)((G)p + off);
 }
 template <typename T>
 __device__ __forceinline__ void sto(T* p, uint32_t off, T v) {
-    *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + off) = v;
+    typedef __attribute__((address_space(1))) char* G;
+    *(__attribute__((address_space(1))) T*)((G)p + off) = v;
+}
+
+// A value that is the same in every lane, in scalar registers: the compiler
+// cannot tell where it comes from memory that the kernel might write.
+template <typename S>
+__device__ __forceinline__ S uniform(const S& s) {
+    static_assert(sizeof(S) % 4 == 0, "copied by words");
+    struct W { int w[sizeof(S) / 4]; } b = __builtin_bit_cast(W, s);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(S) / 4); i++) b.w[i] = __builtin_amdgcn_readfirstlane(b.w[i]);
+    return __builtin_bit_cast(S, b);
 }
 
 // The value held by lane l-1 of the wave (DPP wave_shr:1; lane 0, which has
@@ -117,29 +130,40 @@ __device__ __forceinline__ T div_(T a, T b) {
 // the TX x TY output tile (TX=RX-4, TY=RY-4) plus a 2-cell ring.  Thread t
 // owns region position (t % RX, t / RX) for the whole k-march, so every value
 // a position needs only at its own column (x, u, h, rhr of the planes around
-// K, its xant, V3, pair sums) lives in a register queue, and only values
-// read by in-plane neighbours go through LDS:
+// K, its xant, V3) lives in a register queue, and values read by in-plane
+// neighbours go through LDS:
 //   sx   x on planes K and K+1 with a 3-cell ring (inflow halo values)
 //   sxa  xant, planes K-2 .. K
-//   sv1, sv2   V1 and V2, planes K-2 and K-1
-//   scp, scn   cp and cn, planes K-2 and K-1
+//   sv1, sv2   V1 and V2: plane K-1 from B on, K-2 until then
+//   scp, scn   cp and cn: plane K-1 from C on, K-2 until then
 //   sf1, sf2   limited x/y face fluxes of plane K-2
-//   e_*  (1024-thread tilings) h, u1, u3 of each column on plane K-1
-// The z cross terms of V1 and V2 use pair sums formed one plane at a time:
+//   e_*  h, u1, u3 of each column on plane K-1
+//   rr, hh  a thread's own r and h until the update two planes on
+// The z cross terms of V1 and V2 use pair sums:
 // rat4(xa(i-1,k-1), xa(i,k-1), xa(i-1,k+1), xa(i,k+1)) =
 //   ((xa(i,k+1)+xa(i-1,k+1)) - (xa(i,k-1)+xa(i-1,k-1)))*0.25,
 // the same operations in the same order as the reference.
 //
 // Two barriers per plane: stage A reads the x plane that the previous step
 // wrote and writes the next one; B reads the xant A wrote; C/D read the V
-// that B wrote.  A slot of a ring is rewritten only after a barrier that
-// every reader of its previous plane has passed (three xant slots, because
-// A of plane K runs while slower threads may still be in C of plane K-1,
-// reading xant K-2).
+// that B wrote.  A slot is rewritten only after a barrier that every other
+// thread's reads of its previous plane precede; a thread's own later reads of
+// it come before its write in program order.
 //
-// The grid is persistent: workgroups loop over (tile, k-chunk) work items,
-// a chunk of output planes [k0,k1] recomputing xant from k0-2 and cp,cn,V
-// from k0-1.  Inputs of plane K+1 are loaded while plane K is computed.
+// The grid is persistent: workgroups loop over (tile, k-range) work items, a
+// range of output planes [k0,k1] recomputing xant from k0-2 and cp,cn,V from
+// k0-1.  Inputs of plane K+1 are loaded while plane K is computed.
+//
+// What bounds it: not HBM (512x512x256 moves 5 GB in 1.3 ms) but the chain of
+// a plane.  Four waves per SIMD, all of one workgroup and so in the same
+// stage, hide little of a wait, and the registers (128) leave no room for
+// more.  So nothing waits inside a step but the two barriers: all loads of a
+// step are issued together after B and waited for once, before A; the store
+// of a plane is issued right after that wait; h and rhr of the plane being
+// updated are kept, not loaded again; V, the bounds and cp/cn are formed
+// straight-line by every lane, so that their LDS reads go out together.
+// Together with the scalar plane pointers, 512x512x256 went from 1.66 to
+// 1.31 ms (fast build) and 256x256x128 from 294 to 233 us (exact build).
 // ---------------------------------------------------------------------------
 template <typename T>
 struct XSrc {  // where one sx cell comes from: x, bcx, bcy or nothing
@@ -147,26 +171,23 @@ struct XSrc {  // where one sx cell comes from: x, bcx, bcy or nothing
     int base, stride;
 };
 
-// Whether a tiling passes the j-1 column inputs of V2 through LDS (the
-// 1024-thread tilings, one workgroup per CU, have the room; the 512-thread
-// ones run two workgroups per CU and load them).
-template <int RX, int RY>
-struct XJ { static constexpr bool value = RX * RY >= 1024; };
-
 // LDS of one workgroup of the fixed-position kernel.
 template <typename T, int RX, int RY>
 struct FusedLds {
-    static constexpr int NE = XJ<RX, RY>::value ? RY * RX : 1;
     T sx[2][RY + 2][RX + 2];
     T sxa[3][RY][RX];
-    T sv1[2][RY][RX];
-    T sv2[2][RY][RX];
-    T scp[2][RY][RX];
-    T scn[2][RY][RX];
+    T sv1[RY][RX];
+    T sv2[RY][RX];
+    T scp[RY][RX];
+    T scn[RY][RX];
     T sf1[RY][RX];  // limited flux through the left x-face, plane K-2
     T sf2[RY][RX];  // limited flux through the lower y-face, plane K-2
     // h, u1 (face i), u3 (faces P, P+1) of each source column on plane P
-    T e_h[NE], e_u1[NE], e_u3a[NE], e_u3b[NE];
+    T e_h[RY * RX], e_u1[RY * RX], e_u3a[RY * RX], e_u3b[RY * RX];
+    // r (FAST: r/h) of planes K-2..K and h of plane K-2 of the own column, for
+    // the update (a thread's own values, kept here for want of registers)
+    T rr[3][RY][RX];
+    T hh[RY][RX];
 };
 static_assert(sizeof(FusedLds<double, 32, 32>) <= 160 * 1024, "LDS of one CU");
 
@@ -250,8 +271,6 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     const bool do_v2 = in_dom && gj >= 2 && li >= -1 && li <= TX && lj >= -1;
     const bool do_c = in_dom && li >= -1 && li <= TX && lj >= -1 && lj <= TY;
     const bool do_d = in_dom && li >= 0 && li < TX && lj >= 0 && lj < TY;
-    // left/lower face fluxes: every x-face and y-face of a tile cell
-    const bool do_f = li >= 0 && li <= TX && lj >= 0 && lj <= TY;
     // upwind source cell: itself in the domain, the mirror image on the
     // one-cell halo ring (cp_scnd_last_to_halo_xy_fulld), clamped beyond
     const int ai = clampi(mirror(gi, np), 1, np), aj = clampi(mirror(gj, mp), 1, mp);
@@ -269,6 +288,9 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     // x-neighbour availability for the in-plane max/min (edge copies
     // duplicate the centre and do not change it)
     const bool nxm = gi > 1, nxp = gi < np, nym = gj > 1, nyp = gj < mp;
+    // the position past the last column holds a mirrored column's u1: its
+    // element of e_u1 is the last column's face n+1 instead
+    const bool wall_e = gi == np + 1, last_e = gi == np && pi < RX - 1;
     // tape ownership: x/y halo cells of xant and the wall faces n+1 belong to
     // the tile whose output range touches them
     bool own_fx = false, own_fy = false, own_s = false;
@@ -292,7 +314,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     // register queues of the source column; during step K they hold
     //   xq1..3 = x(K-1..K+1), u1a0/1 = u1(i,K-1..K), u1b0/1 = u1(i+1,K-1..K),
     //   u2a/u2b likewise at j and j+1, u3q0..2 = faces K-1..K+1,
-    //   hq1..2 = h(K-1..K), rq2 = rhr(K), v3q1..2 = V3 faces K-2..K-1,
+    //   hq1..2 = h(K-1..K), rq2 = rhr(K),
     //   xmx0/xmn0 = bounds of x for the limiter on plane K-1 (xmx1/xmn1:
     //   plane K, formed in A).
     // The column's own xant of planes K-2..K comes from sxa: the slot of
@@ -314,11 +336,13 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     u3q[2] = ldo(pl(u3, SXY, fc(Ks + 1)), so);
     hq[0] = ldo(pl(h, SXY, kc(Ks - 1)), so); hq[1] = ldo(pl(h, SXY, kc(Ks)), so);
     T rq2 = T(0);
-    if constexpr (!DENS && PASS != 2) rq2 = ldo(pl(rhr, SXY, kc(Ks)), so);
+    if constexpr (!DENS) rq2 = ldo(pl(rhr, SXY, kc(Ks)), so);
     // PASS 2: the previous pass's result on plane K (stage A's xant)
     T xaq = T(0);
     if constexpr (PASS == 2) xaq = ldo(pl(pio->xa, SXY, kc(Ks)), so);
-    T v3q[2] = {T(0), T(0)};
+    // V3 of face K-1 during step K; face lp stays past the top (stage B forms
+    // no face there), and the tape takes face K-2 too
+    T v3q2 = T(0), v3q1 = T(0);
     T xmx[2] = {T(0), T(0)}, xmn[2] = {T(0), T(0)};
     T f3c = T(0);  // limited flux through the upper z-face of the last output plane
 
@@ -326,6 +350,21 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     // after every LDS read of the previous one
     sx[0][pj + 1][pi + 1] = in_dom ? xq[1] : ld(own, Ks);
     if (t < NRING) sx[0][rsj][rsi] = ld(ring, Ks);
+    // x of plane K+1 for the LDS: ring cell, and the own cell where it is
+    // not in the queue (positions outside the domain); loaded a step ahead
+    // (a null source keeps the zero)
+    T xr = T(0), xown = T(0);
+    const bool ring_on = t < NRING && ring.p, own_on = !in_dom && own.p;
+    const uint32_t rstr = uint32_t(ring.stride) * uint32_t(sizeof(T)),
+                   ostr = uint32_t(own.stride) * uint32_t(sizeof(T));
+    const char* rp = ring_on ? (const char*)(ring.p + ring.base) + (uint64_t)rstr * (uint32_t)Ks : nullptr;
+    const char* op = own_on ? (const char*)(own.p + own.base) + (uint64_t)ostr * (uint32_t)Ks : nullptr;
+    auto ld_halo = [&](int k) __attribute__((always_inline)) {  // k >= 1
+        rp += rstr; op += ostr;
+        if (ring_on) xr = ldo((const T*)rp, 0);
+        if (own_on) xown = ldo((const T*)op, 0);
+    };
+    if (Ks + 1 <= Alast) ld_halo(Ks + 1);
     __syncthreads();
 
     // The tile arrays from sv2 on lie beyond the 64 KiB that a ds
@@ -338,14 +377,64 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     constexpr int MID = (int)offsetof(LT, sv2);
     constexpr int HI = (int)offsetof(LT, e_h) - RX * SZ;  // e arrays are read one row back
     uint32_t lmid = uint32_t(MID + t * SZ), lhi = uint32_t(HI + t * SZ);
-    asm volatile("" : "+v"(lmid), "+v"(lhi));
+    uint32_t lsx = uint32_t(offsetof(LT, sx) + ((saj - 1) * SW + (sai - 1)) * SZ);
+    asm volatile("" : "+v"(lmid), "+v"(lhi), "+v"(lsx));
     char* const lds0 = reinterpret_cast<char*>(&L);
     // array `arr` at ring slot s, offset (db rows, da columns) from the lane
 #define LMID(arr, s, db, da) \
     (*reinterpret_cast<T*>(lds0 + lmid + ((int)offsetof(LT, arr) - MID + (s) * PLN + ((db) * RX + (da)) * SZ)))
+// x of the plane in ring slot s, row db and column da of the 3x3 neighbourhood
+// of the source column; for a position in the domain its own
+#define LSX(s, db, da) \
+    (*reinterpret_cast<T*>(lds0 + lsx + ((s) * (SW * SH) + (db) * SW + (da)) * SZ))
 #define LHI(arr, r) (*reinterpret_cast<T*>(lds0 + lhi + ((int)offsetof(LT, arr) - HI + (r) * SZ)))
 
+    auto dif4 = [](T z0, T z1, T z2, T z3) { return (z3 + z2) - (z1 + z0); };
+    // Pseudo-velocity of a face between x1 and x2 with advector a and h of
+    // the two cells summed to h2: s1, s2 the sums of the cross advectors and
+    // d1, d2 the cross differences of x (both times 4; one pair at the lids).
+    // FAST: the powers of two folded, and every contraction written out, so
+    // that all tilings round alike.
+    auto vface = [](T x1, T x2, T a, T h2, T s1, T d1, auto... s2d2) __attribute__((always_inline)) {
+        if constexpr (FAST) {
+            T cr = s1 * d1;
+            if constexpr (sizeof...(s2d2) == 2) {
+                const T q2[2] = {s2d2...};
+                cr = fma_(q2[0], q2[1], cr);
+            }
+            const T q = a * rcp_nr(h2);
+            return fma_(q * cr, T(-0.0625), (x2 - x1) * fma_(-q, a, T(0.5) * T(fabs(a))));
+        } else {
+            const T hm = T(1) / (T(0.5) * h2);
+            T cr = s1 * (d1 * T(0.25));
+            if constexpr (sizeof...(s2d2) == 2) {
+                const T q2[2] = {s2d2...};
+                cr = cr + q2[0] * (q2[1] * T(0.25));
+            }
+            return vdyf(x1, x2, a, hm) - T(0.125) * a * hm * (cr);
+        }
+    };
+    auto lflux = [](T v, T c_c, T n_m, T c_m, T n_c) {
+        if constexpr (TAPE) return gflux(v, c_c, n_m, c_m, n_c);
+        else return pp(v) * min2(c_c, n_m) - pn(v) * min2(c_m, n_c);  // capped in C
+    };
     uint32_t so_k = so, fo_k = fo;
+    // planes of the newest queue slots, and the planes' sizes in bytes
+    const uint32_t SB8 = SXY * SZ, FB8 = FXY * SZ, YB8 = YXY * SZ;
+    const T* qx = uniform(pl(x, SXY, kc(Ks + 1)));
+    const T* qu1 = uniform(pl(u1, FXY, kc(Ks)));
+    const T* qu2 = uniform(pl(u2, YXY, kc(Ks)));
+    const T* qu3 = uniform(pl(u3, SXY, fc(Ks + 1)));
+    const T* qh = uniform(pl(h, SXY, kc(Ks)));
+    const T* qr = DENS ? nullptr : uniform(pl(rhr, SXY, kc(Ks)));
+    const T* qxa = PASS == 2 ? uniform(pl(pio->xa, SXY, kc(Ks))) : nullptr;
+    auto adv = [](auto* p, uint32_t d) {
+        // uniform() also keeps it one pointer, not an induction per unrolled step
+        return (decltype(p))((uintptr_t)uniform(p) + d);
+    };
+    T* qxo = uniform(pl(xo, SXY, Ks - 4));  // plane K-3 during step K
+    T xst = T(0);                           // the new x of that plane
+    const bool edge_d = do_d && (gi == 1 || gi == np || gj == 1 || gj == mp);
     auto step = [&](auto phase, int K) __attribute__((always_inline)) {
         constexpr int PH = decltype(phase)::value;
         // K opaque: every plane-dependent quantity is formed within the
@@ -364,32 +453,39 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         T& u2a0 = u2a[Q2a]; T& u2a1 = u2a[Q2b]; T& u2b0 = u2b[Q2a]; T& u2b1 = u2b[Q2b];
         T& u3q0 = u3q[Q3a]; T& u3q1 = u3q[Q3b]; T& u3q2 = u3q[Q3c];
         T& hq1 = hq[Q2a]; T& hq2 = hq[Q2b];
-        T& v3q1 = v3q[Q2a]; T& v3q2 = v3q[Q2b];
         T& xmx0 = xmx[Q2a]; T& xmn0 = xmn[Q2a]; T& xmx1 = xmx[Q2b]; T& xmn1 = xmn[Q2b];
         // the column offsets are opaque to the optimiser at each plane, so
         // loads keep the saddr form (plane pointer + offset) instead of
         // becoming per-lane 64-bit pointer inductions
         asm volatile("" : "+v"(so_k), "+v"(fo_k));
         const uint32_t so = so_k, fo = fo_k;
-        const bool A_on = K <= Alast, An_on = K + 1 <= Alast;
-        // h and rhr of the output plane K-2 for D (cache hits), loaded before
-        // this step's loads of plane K+1: a wait for them then does not wait
-        // for those too (loads complete in issue order for s_waitcnt).  h of
-        // plane K-1 for C is the queue's.
-        const T hQ = ldo(pl(h, SXY, kc(K - 2)), so);
-        T rQ = T(0);
-        if constexpr (!DENS) rQ = ldo(pl(rhr, SXY, kc(K - 2)), so);
+        const bool A_on = K <= Alast;
+        // Everything loaded for this step is needed now; waited for here, so
+        // that the stores below are not waited for before the next step does
+        // the same (loads and stores share one in-order counter: a store in
+        // stage D, with the wait for the loads right after it, exposed its
+        // whole latency on every plane).
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        // x of the last output plane, K-3, and the edge copies of x at level
+        // n around plane K
+        qxo = adv(qxo, SB8);
+        if (do_d && K - 3 >= k0 && K - 3 <= k1) sto(qxo, so, xst);
+        if (edge_d && K >= k0 && K <= k1) {
+            T* const xok = pl(xo, SXY, K);
+            if (gi == 1) sto(xok - 1, so, xq2);
+            if (gi == np) sto(xok + 1, so, xq2);
+            if (gj == 1) sto(xok - o.sx, so, xq2);
+            if (gj == mp) sto(xok + o.sx, so, xq2);
+        }
+        // plane K+1 into the LDS slot that stage A of plane K-1 read
+        if (K + 1 <= Alast) {
+            sx[E1][pj + 1][pi + 1] = in_dom ? xq3 : xown;
+            if (t < NRING) sx[E1][rsj][rsi] = xr;
+        }
         const T hP = hq1;
         // Temporaries of a step that are read only under the condition
         // that sets them are left unset rather than zeroed: a default value
         // would cost a register move per step on every path.
-        // x of plane K+1 for the LDS: ring cell, and the own cell where it
-        // is not in the queue (positions outside the domain)
-        T xr, xown;
-        if (An_on) {
-            if (t < NRING) xr = ld(ring, K + 1);
-            if (!in_dom) xown = ld(own, K + 1);
-        }
         // neighbour-column inputs of V1/V2 on plane P=K-1.  Column
         // (gi-1, gj) is the source column of the lane to the left wherever
         // V1 is formed (gi >= 2 in the domain, so the left position is in
@@ -405,26 +501,15 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         const int P = K - 1;
         const bool BC_on = P >= max(1, k0 - 1) && P <= min(lp, k1 + 1);
         const int Pc = kc(P);
-        const T nv1_h = from_left_lane(hq1);
-        const T nv1_u2a = from_left_lane(u2a0);
-        const T nv1_u2b = from_left_lane(u2b0);
-        const T nv1_u3a = from_left_lane(u3q0);
-        const T nv1_u3b = from_left_lane(u3q1);
-        // column (gi, gj-1)
-        T nv2_h, nv2_u1a, nv2_u1b, nv2_u3a, nv2_u3b;  // read under BC_on && do_v2
-        if constexpr (XJ<RX, RY>::value) {
-            if (BC_on) {
-                LHI(e_h, 0) = hq1;  // element e = t
-                LHI(e_u1, 0) = u1a0;
-                LHI(e_u3a, 0) = u3q0;
-                LHI(e_u3b, 0) = u3q1;
-            }
-        } else {
-            nv2_h = ldo(pl(h, SXY, Pc) - o.sx, so);
-            nv2_u1a = ldo(pl(u1, FXY, Pc) - o.fx, fo);
-            nv2_u1b = ldo(pl(u1, FXY, Pc) - o.fx + 1, fo);
-            nv2_u3a = ldo(pl(u3, SXY, Pc) - o.sx, so);
-            nv2_u3b = ldo(pl(u3, SXY, Pc + 1) - o.sx, so);
+        const T hx = from_left_lane(hq1) + hq1;
+        const T s2x = from_left_lane(u2a0 + u2b0) + u2b0 + u2a0;
+        const T s3x = from_left_lane(u3q0 + u3q1) + u3q1 + u3q0;
+        if (BC_on) {
+            LHI(e_h, 0) = hq1;  // element e = t
+            if (!wall_e) LHI(e_u1, 0) = u1a0;
+            if (last_e) LHI(e_u1, 1) = u1b0;
+            LHI(e_u3a, 0) = u3q0;
+            LHI(e_u3b, 0) = u3q1;
         }
 
         // ---- A: xant on plane K ------------------------------------------
@@ -435,17 +520,19 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         // boundary case would be computed and selected on every plane)
         auto stage_a = [&](auto edge) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge)::value;
-            auto& sx = L.sx[E0];
             const bool gnd = EDGE && K == 1, sky = EDGE && K == lp;
             T xc = xq2;
+            // the source column's neighbours
+            const T xw = LSX(E0, 1, 0), xe = LSX(E0, 1, 2), xs = LSX(E0, 0, 1), xn = LSX(E0, 2, 1);
+            T hinv;
+            if constexpr (PASS != 2 || FAST) hinv = rcp_<FAST>(hq2);
             if constexpr (PASS == 2) {
                 xa_new = xaq;
             } else {
-            T hinv = rcp_<FAST>(hq2);
-            T f1p = donor(xc, sx[saj][sai + 1], u1b1);
-            T f1 = donor(sx[saj][sai - 1], xc, u1a1);
-            T f2p = donor(xc, sx[saj + 1][sai], u2b1);
-            T f2 = donor(sx[saj - 1][sai], xc, u2a1);
+            T f1p = donor(xc, xe, u1b1);
+            T f1 = donor(xw, xc, u1a1);
+            T f2p = donor(xc, xn, u2b1);
+            T f2 = donor(xs, xc, u2a1);
             T f3p, f3;
             if (gnd) {
                 f3p = donor(xc, xq3, u3q2);
@@ -461,14 +548,16 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             else xa_new = rq2 * (xc - (f1p - f1 + f2p - f2 + f3p - f3) * hinv);
             }
             sxa[R0][pj][pi] = xa_new;
+            // FAST: r*(xant/r - s/h) = xant - (r/h)*s, to rounding
+            if constexpr (!DENS) LHI(rr, R0 * RY * RX) = FAST ? rq2 * hinv : rq2;
             // bounds of x for the limiter on plane K: the 7-point stencil,
             // where out-of-domain neighbours are edge copies of the centre
             // (cp_last_to_halo_xy) and leave max/min unchanged
             T m = xc, n = xc;
-            if (nxm) { T v = sx[pj + 1][pi]; m = max2(m, v); n = min2(n, v); }
-            if (nxp) { T v = sx[pj + 1][pi + 2]; m = max2(m, v); n = min2(n, v); }
-            if (nym) { T v = sx[pj][pi + 1]; m = max2(m, v); n = min2(n, v); }
-            if (nyp) { T v = sx[pj + 2][pi + 1]; m = max2(m, v); n = min2(n, v); }
+            { const T v = nxm ? xw : xc; m = max2(m, v); n = min2(n, v); }
+            { const T v = nxp ? xe : xc; m = max2(m, v); n = min2(n, v); }
+            { const T v = nym ? xs : xc; m = max2(m, v); n = min2(n, v); }
+            { const T v = nyp ? xn : xc; m = max2(m, v); n = min2(n, v); }
             if (!gnd) { m = max2(m, xq1); n = min2(n, xq1); }
             if (!sky) { m = max2(m, xq3); n = min2(n, xq3); }
             xmx1 = m;
@@ -478,132 +567,131 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             if (K == 1 || K == lp) stage_a(std::true_type{});
             else stage_a(std::false_type{});
         }
-        if (An_on) {
-            sx[E1][pj + 1][pi + 1] = in_dom ? xq3 : xown;
-            if (t < NRING) sx[E1][rsj][rsi] = xr;
-        }
         __syncthreads();
-// xant, cp, cn of plane K-d at tile position (a, b)
+// xant of plane K-d at tile position (a, b)
 #define XA(d, a, b) sxa[(d) == 0 ? R0 : ((d) == 1 ? R1 : R2)][(b) + 2][(a) + 2]
-#define CP(d, a, b) LMID(scp, ((d) & 1) ? E1 : E0, (b) - lj, (a) - li)
-#define CN(d, a, b) LMID(scn, ((d) & 1) ? E1 : E0, (b) - lj, (a) - li)
-        if constexpr (XJ<RX, RY>::value) {
-            if (BC_on && do_v2) {  // pj >= 1 where V2 is formed
-                nv2_h = LHI(e_h, -RX);  // element e = t - RX
-                nv2_u1a = LHI(e_u1, -RX);
-                nv2_u3a = LHI(e_u3a, -RX);
-                nv2_u3b = LHI(e_u3b, -RX);
-                // u1 on face i+1 of column j-1: the next position's face i,
-                // except on the last column, whose right neighbour is a
-                // mirrored ring position
-                if (gi < np) nv2_u1b = LHI(e_u1, -RX + 1);
-                else nv2_u1b = ldo(pl(u1, FXY, Pc) - o.fx + 1, fo);
-            }
-        }
         const int Q = K - 2;
         const bool Dq = Q >= k0 && Q <= k1;
-        // ---- B: pair sums, V1/V2 on plane P=K-1, V3 on face K --------------
-        T s1n, s2n, v3n = T(0);  // s1n/s2n read in B's z terms, where A_on holds
-        if (A_on) {
-            if (do_v1) s1n = xa_new + XA(0, li - 1, lj);
-            if (do_v2) s2n = xa_new + XA(0, li, lj - 1);
-            if (do_c && K >= 2 && K >= k0 - 1) {
-                T hmz = rcp_<FAST>(T(0.5) * (hq1 + hq2));
+        // ---- limited fluxes through the left x-face and lower y-face of this
+        //      position on plane Q: V and cp/cn of Q are from the previous
+        //      step and are replaced below; stage D reads them for both faces
+        //      a cell shares, so each face flux is formed once
+        if (Dq) {
+            const T c0 = LMID(scp, 0, 0, 0), n0 = LMID(scn, 0, 0, 0);
+            LMID(sf1, 0, 0, 0) = lflux(sv1[pj][pi], c0, LMID(scn, 0, 0, -1), LMID(scp, 0, 0, -1), n0);
+            LMID(sf2, 0, 0, 0) =
+                lflux(LMID(sv2, 0, 0, 0), c0, LMID(scn, 0, -1, 0), LMID(scp, 0, -1, 0), n0);
+        }
+        // ---- B: V1/V2 on plane P=K-1, V3 on face K, the limiter's bounds on P
+        // Straight-line on the interior planes: every lane forms every
+        // quantity and the lanes that do not own it drop it (a select, or a
+        // reader that does not look), so that the LDS reads of all of them
+        // go out together instead of one exec region after the other.
+        T v3n = T(0);
+        T mx, mn;  // bounds of x and xant on plane P, for C
+#define SB __builtin_amdgcn_sched_barrier(0);
+        auto stage_b = [&](auto edge) __attribute__((always_inline)) {
+            constexpr bool EDGE = decltype(edge)::value;
+            const bool gnd = EDGE && P == 1, sky = EDGE && P == lp;
+            const T xc = XA(1, li, lj), xw = XA(1, li - 1, lj), xe = XA(1, li + 1, lj),
+                    xs = XA(1, li, lj - 1), xn = XA(1, li, lj + 1);
+            T kw, ks, ke, kn;  // plane K
+            if (!EDGE || A_on) {
+                kw = XA(0, li - 1, lj); ks = XA(0, li, lj - 1);
+                ke = XA(0, li + 1, lj); kn = XA(0, li, lj + 1);
+            }
+            if (!EDGE || (A_on && K >= 2 && K >= k0 - 1)) {
                 T s1 = u1a0 + u1a1 + u1b1 + u1b0;
                 T s2 = u2a0 + u2b0 + u2b1 + u2a1;
-                T cr = s1 * rat4(XA(1, li - 1, lj), XA(0, li - 1, lj), XA(1, li + 1, lj),
-                                 XA(0, li + 1, lj)) +
-                       s2 * rat4(XA(1, li, lj - 1), XA(0, li, lj - 1), XA(1, li, lj + 1),
-                                 XA(0, li, lj + 1));
-                T a = u3q1;
-                v3n = vdyf(XA(1, li, lj), xa_new, a, hmz) - T(0.125) * a * hmz * (cr);
+                v3n = vface(xc, xa_new, u3q1, hq1 + hq2, s1, dif4(xw, kw, xe, ke), s2,
+                            dif4(xs, ks, xn, kn));
             }
-        }
-        if (BC_on) {
-            const bool zterms = !(P == 1 || P == lp);
-            T val1 = T(0), val2 = T(0);
-            if (do_v1) {
-                T hmx = rcp_<FAST>(T(0.5) * (nv1_h + hq1));
-                T s2 = nv1_u2a + nv1_u2b + u2b0 + u2a0;
-                T cr = s2 * rat4(XA(1, li - 1, lj - 1), XA(1, li, lj - 1), XA(1, li - 1, lj + 1),
-                                 XA(1, li, lj + 1));
-                if (zterms) {
-                    T s3 = nv1_u3a + nv1_u3b + u3q1 + u3q0;
-                    cr = cr + s3 * ((s1n - (XA(2, li, lj) + XA(2, li - 1, lj))) * T(0.25));
+            SB
+            if (!EDGE || BC_on) {
+                const T xsw = XA(1, li - 1, lj - 1), xnw = XA(1, li - 1, lj + 1),
+                        xse = XA(1, li + 1, lj - 1);
+                const T bc = XA(2, li, lj);
+                T val1, val2;
+                if (!gnd && !sky)
+                    val1 = vface(xw, xc, u1a0, hx, s2x, dif4(xsw, xs, xnw, xn), s3x,
+                                 (xa_new + kw) - (bc + XA(2, li - 1, lj)));
+                else
+                    val1 = vface(xw, xc, u1a0, hx, s2x, dif4(xsw, xs, xnw, xn));
+                SB
+                {
+                    // column (gi, gj-1): element e = t - RX
+                    const T nv2_h = LHI(e_h, -RX), nv2_u1a = LHI(e_u1, -RX),
+                            nv2_u1b = LHI(e_u1, -RX + 1), nv2_u3a = LHI(e_u3a, -RX),
+                            nv2_u3b = LHI(e_u3b, -RX);
+                    const T hy = nv2_h + hq1, s1 = nv2_u1a + u1a0 + u1b0 + nv2_u1b,
+                            s3 = nv2_u3a + u3q0 + u3q1 + nv2_u3b;
+                    if (!gnd && !sky)
+                        val2 = vface(xs, xc, u2a0, hy, s1, dif4(xsw, xw, xse, xe), s3,
+                                     (xa_new + ks) - (bc + XA(2, li, lj - 1)));
+                    else
+                        val2 = vface(xs, xc, u2a0, hy, s1, dif4(xsw, xw, xse, xe));
                 }
-                T a = u1a0;
-                val1 = vdyf(XA(1, li - 1, lj), XA(1, li, lj), a, hmx) - T(0.125) * a * hmx * (cr);
-            }
-            if (do_v2) {
-                T hmy = rcp_<FAST>(T(0.5) * (nv2_h + hq1));
-                T s1 = nv2_u1a + u1a0 + u1b0 + nv2_u1b;
-                T cr = s1 * rat4(XA(1, li - 1, lj - 1), XA(1, li - 1, lj), XA(1, li + 1, lj - 1),
-                                 XA(1, li + 1, lj));
-                if (zterms) {
-                    T s3 = nv2_u3a + u3q0 + u3q1 + nv2_u3b;
-                    cr = cr + s3 * ((s2n - (XA(2, li, lj) + XA(2, li, lj - 1))) * T(0.25));
+                val1 = do_v1 ? val1 : T(0);
+                val2 = do_v2 ? val2 : T(0);
+                sv1[pj][pi] = val1;
+                LMID(sv2, 0, 0, 0) = val2;
+                if constexpr (TAPE) {
+                    if (P >= k0 && P <= k1) {
+                        if (own_fx) sto(pl(tp->v[0], FXY, P), tfo, val1);
+                        if (own_fy) sto(pl(tp->v[1], YXY, P), tso, val2);
+                    }
                 }
-                T a = u2a0;
-                val2 = vdyf(XA(1, li, lj - 1), XA(1, li, lj), a, hmy) - T(0.125) * a * hmy * (cr);
+                mx = xw, mn = xw;
+#define ACC(v, lo, hi) { T t_ = (v); lo = min2(lo, t_); hi = max2(hi, t_); }
+                ACC(xc, mn, mx) ACC(xe, mn, mx) ACC(xs, mn, mx) ACC(xn, mn, mx)
+                if (!gnd) ACC(bc, mn, mx)
+                if (!sky) ACC(xa_new, mn, mx)
+#undef ACC
+                mx = max2(mx, xmx0);
+                mn = min2(mn, xmn0);
             }
-            sv1[E1][pj][pi] = val1;
-            LMID(sv2, E1, 0, 0) = val2;
-            if constexpr (TAPE) {
-                if (P >= k0 && P <= k1) {
-                    if (own_fx) sto(pl(tp->v[0], FXY, P), tfo, val1);
-                    if (own_fy) sto(pl(tp->v[1], YXY, P), tso, val2);
-                }
-            }
-        }
-        // ---- limited fluxes through the left x-face and lower y-face of this
-        //      position on plane Q (V and cp/cn of Q are from the previous
-        //      step); stage D reads them for both faces a cell shares, so
-        //      each face flux is formed once
-        if (Dq && do_f) {
-            LMID(sf1, 0, 0, 0) = gflux(sv1[E0][pj][pi], CP(2, li, lj), CN(2, li - 1, lj),
-                                CP(2, li - 1, lj), CN(2, li, lj));
-            LMID(sf2, 0, 0, 0) = gflux(LMID(sv2, E0, 0, 0), CP(2, li, lj), CN(2, li, lj - 1),
-                                CP(2, li, lj - 1), CN(2, li, lj));
-        }
+        };
+        if (BC_on && P != 1 && P != lp) stage_b(std::false_type{});
+        else stage_b(std::true_type{});
         if constexpr (TAPE)
             if (Dq && own_s) sto(pl(tp->psi, SXY, Q), tso, XA(2, li, lj));
         // The loaded source-column queues are not read after this point:
         // the oldest slot of each is loaded with the plane step K+1 needs;
         // the latency is covered by C, D and the next step's barrier.
         {
-            // the oldest slot of each queue becomes the newest of step K+1
+            // the oldest slot of each queue becomes the newest of step K+1;
+            // the plane pointers move by one plane until they reach the last
+            // (kept in scalar registers: formed anew from K they cost twice
+            // the scalar instructions)
             const int Kn = K + 1;
-            xq1 = ldo(pl(x, SXY, kc(Kn + 1)), so);
-            u1a0 = ldo(pl(u1, FXY, kc(Kn)), fo);
-            u1b0 = ldo(pl(u1, FXY, kc(Kn)) + 1, fo);
-            u2a0 = ldo(pl(u2, YXY, kc(Kn)), so);
-            u2b0 = ldo(pl(u2, YXY, kc(Kn)) + o.yx, so);
-            u3q0 = ldo(pl(u3, SXY, fc(Kn + 1)), so);
-            hq1 = ldo(pl(h, SXY, kc(Kn)), so);
-            if constexpr (!DENS && PASS != 2) rq2 = ldo(pl(rhr, SXY, kc(Kn)), so);
-            if constexpr (PASS == 2) xaq = ldo(pl(pio->xa, SXY, kc(Kn)), so);
+            const uint32_t dS = Kn <= lp ? SB8 : 0, dF = Kn <= lp ? FB8 : 0, dY = Kn <= lp ? YB8 : 0;
+            qx = adv(qx, Kn < lp ? SB8 : 0);
+            qu1 = adv(qu1, dF); qu2 = adv(qu2, dY); qu3 = adv(qu3, dS); qh = adv(qh, dS);
+            if constexpr (!DENS) qr = adv(qr, dS);
+            if constexpr (PASS == 2) qxa = adv(qxa, dS);
+            if (Kn + 1 <= Alast) ld_halo(Kn + 1);
+            xq1 = ldo(qx, so);
+            u1a0 = ldo(qu1, fo);
+            u1b0 = ldo(qu1 + 1, fo);
+            u2a0 = ldo(qu2, so);
+            u2b0 = ldo(qu2 + o.yx, so);
+            u3q0 = ldo(qu3, so);
+            hq1 = ldo(qh, so);
+            if constexpr (!DENS) rq2 = ldo(qr, so);
+            if constexpr (PASS == 2) xaq = ldo(qxa, so);
         }
         __syncthreads();
-        const bool D_on = do_d && Dq;
         // ---- C: cp, cn on plane P ------------------------------------------
+        // cp, cn of the own column on planes P (formed here) and P-1
+        T cpP, cnP, cpQ, cnQ;
         auto stage_c = [&](auto edge) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge)::value;
             const bool gnd = EDGE && P == 1, sky = EDGE && P == lp;
-            T rp = T(0), rn = T(0);
-            if (do_c) {
-                T mxo = xmx0, mno = xmn0;
+            T rp, rn;
+            {
                 const T xaP = XA(1, li, lj);
-                T mx = XA(1, li - 1, lj), mn = mx;
-#define ACC(v, lo, hi) { T t_ = (v); lo = min2(lo, t_); hi = max2(hi, t_); }
-                ACC(xaP, mn, mx) ACC(XA(1, li + 1, lj), mn, mx)
-                ACC(XA(1, li, lj - 1), mn, mx) ACC(XA(1, li, lj + 1), mn, mx)
-                if (!gnd) ACC(XA(2, li, lj), mn, mx)
-                if (!sky) ACC(xa_new, mn, mx)
-#undef ACC
-                mx = max2(mx, mxo);
-                mn = min2(mn, mno);
-                T a1p = sv1[E1][pj][pi + 1], a1 = sv1[E1][pj][pi];
-                T a2p = LMID(sv2, E1, 1, 0), a2 = LMID(sv2, E1, 0, 0);
+                T a1p = sv1[pj][pi + 1], a1 = sv1[pj][pi];
+                T a2p = LMID(sv2, 0, 1, 0), a2 = LMID(sv2, 0, 0, 0);
                 T a3p, a3;
                 if (gnd) { a3p = v3n; a3 = -a3p; }
                 else if (sky) { a3 = v3q2; a3p = -a3; }
@@ -614,44 +702,45 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                 rn = div_<FAST>((xaP - mn) * hc,
                                 (pp(a1p) + pn(a1) + pp(a2p) + pn(a2) + pp(a3p) + pn(a3) + ep));
             }
-            LMID(scp, E1, 0, 0) = rp;
-            LMID(scn, E1, 0, 0) = rn;
+            // capped here: every reader takes min(1, .) (the tape holds them
+            // as they are)
+            if constexpr (!TAPE) {
+                rp = min2(T(1), rp);
+                rn = min2(T(1), rn);
+            }
+            cpQ = LMID(scp, 0, 0, 0);
+            cnQ = LMID(scn, 0, 0, 0);
+            LMID(scp, 0, 0, 0) = cpP = do_c ? rp : T(0);
+            LMID(scn, 0, 0, 0) = cnP = do_c ? rn : T(0);
         };
+        // limited flux through the upper z-face of plane Q; the first output
+        // plane's lower one is formed on the step before its own
+        T F3p;
         if (BC_on) {
             if (P == 1 || P == lp) stage_c(std::true_type{});
             else stage_c(std::false_type{});
+            F3p = lflux(v3q2, cpP, cnQ, cpQ, cnP);
+        } else if constexpr (TAPE) {
+            cpQ = LMID(scp, 0, 0, 0);
+            cnQ = LMID(scn, 0, 0, 0);
         }
-        // the lower z-face flux of the first output plane of the range is
-        // the upper face of plane k0-1, formed here on the step before (the
-        // two-plane cp/cn ring no longer holds plane Q-1 once plane Q is
-        // output); later planes carry it from the previous plane
-        if (Q == k0 - 1 && Q >= 1 && do_d)
-            f3c = gflux(v3q2, CP(1, li, lj), CN(2, li, lj), CP(2, li, lj), CN(1, li, lj));
-        // ---- D: the new x on plane Q=K-2 (neighbour data of plane Q was
-        //      written in the previous step; own cp/cn of Q+1 just now) ----
-        if (D_on) {
-            const bool gnd = Q == 1, sky = Q == lp;
-            // x/y faces from stage B of this step; the lower z-face flux is
-            // the upper one of plane Q-1 (the same expression).  On the sky
-            // plane C did not run this step, so the ring still holds Q-1.
+        // ---- D: the new x on plane Q=K-2 -----------------------------------
+        const bool gnd = Q == 1, sky = Q == lp;
+        T F3 = f3c;
+        // the lid's flux is that of the face next to it, reversed
+        if (sky) F3p = T(0) - f3c;
+        if (gnd) F3 = T(0) - F3p;
+        f3c = F3p;
+        if (Dq) {
             const T F1 = LMID(sf1, 0, 0, 0), F1p = LMID(sf1, 0, 0, 1);
             const T F2 = LMID(sf2, 0, 0, 0), F2p = LMID(sf2, 0, 1, 0);
-            T F3, F3p;
-            if (gnd) {
-                const T v = v3q2;
-                F3 = gflux(-v, CP(2, li, lj), CN(1, li, lj), CP(1, li, lj), CN(2, li, lj));
-                F3p = gflux(v, CP(1, li, lj), CN(2, li, lj), CP(2, li, lj), CN(1, li, lj));
-            } else {
-                F3 = f3c;
-                if (sky) F3p = gflux(-v3q1, CP(3, li, lj), CN(2, li, lj), CP(2, li, lj), CN(3, li, lj));
-                else F3p = gflux(v3q2, CP(1, li, lj), CN(2, li, lj), CP(2, li, lj), CN(1, li, lj));
-            }
-            f3c = F3p;
-            T* const xoq = pl(xo, SXY, Q);
+            T hQ;
+            if constexpr (!FAST || DENS) hQ = LHI(hh, 0);
             if constexpr (DENS) {
                 const T xnew = (XA(2, li, lj) - div_<FAST>(F1p - F1 + F2p - F2 + F3p - F3, hQ));
-                sto(xoq, so, xnew);
+                xst = xnew;
                 const T xi = xnew * hQ;
+                if (do_d) {
                 T* const xincq = pl(dio->xinc, SXY, Q);
                 const T rho_n = ldo(xincq, so);
                 sto(xincq, so, xi);
@@ -659,14 +748,13 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                 sto(pl(dio->pexr2, SXY, Q), so, xi);
                 sto(pl(dio->rhoadv, SXY, Q), so, rho_n);
                 sto(pl(dio->rhr, SXY, Q), so, div_<FAST>(rho_n, xi));
+                }
             } else {
-                const T r = rQ;
-                if constexpr (FAST)  // r*(xant/r - s/h) = xant - r*s/h, to rounding
-                    sto(xoq, so, XA(2, li, lj) - r * ((F1p - F1 + F2p - F2 + F3p - F3) * rcp_nr(hQ)));
-                else
-                    sto(xoq, so, r * (div_<FAST>(XA(2, li, lj), r) -
-                                      div_<FAST>(F1p - F1 + F2p - F2 + F3p - F3, hQ)));
-                if constexpr (PASS == 1) {
+                const T r = LHI(rr, R2 * RY * RX);
+                const T sum = F1p - F1 + F2p - F2 + F3p - F3;
+                if constexpr (FAST) xst = XA(2, li, lj) - r * sum;
+                else xst = r * (div_<FAST>(XA(2, li, lj), r) - div_<FAST>(sum, hQ));
+                if constexpr (PASS == 1) if (do_d) {
                     // the limited velocities through the low faces of the
                     // cell, and through the wall faces n+1 at the last cells
                     T* const q1 = pl(pio->ul1, FXY, Q);
@@ -678,7 +766,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                     if (gj == mp) sto(q2 + o.yx, so, F2p);
                     if (sky) sto(pl(pio->ul3, SXY, Q + 1), so, F3p);
                 }
-                if constexpr (TAPE) {
+                if constexpr (TAPE) if (do_d) {
                     // V3 on the lower face Q of the cell (face 1 = -face 2 on
                     // the ground), and on face lp+1 = -face lp on the sky
                     // plane; cp and cn of the cell; x with the inflow values
@@ -687,8 +775,8 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                     T* const tv = pl(tp->v[2], SXY, Q);
                     sto(tv, so, gnd ? -v3q2 : v3q1);
                     if (sky) sto(tv + SXY, so, -v3q1);
-                    sto(pl(tp->cp, SXY, Q), so, CP(2, li, lj));
-                    sto(pl(tp->cn, SXY, Q), so, CN(2, li, lj));
+                    sto(pl(tp->cp, SXY, Q), so, cpQ);
+                    sto(pl(tp->cn, SXY, Q), so, cnQ);
                     const T xc = ldo(pl(x, SXY, Q), so);
                     T* const tb = pl(tp->xb, SXY, Q);
                     T* const t0 = pl(tp->x0, SXY, Q);
@@ -700,14 +788,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                     if (gj == mp) { sto(tb + o.sx, so, bcy[(gi - 1) + np * ((Q - 1) + lp)]); sto(t0 + o.sx, so, xc); }
                 }
             }
-            if (gi == 1 || gi == np || gj == 1 || gj == mp) {
-                const T xe = ldo(pl(x, SXY, Q), so);
-                if (gi == 1) sto(xoq - 1, so, xe);
-                if (gi == np) sto(xoq + 1, so, xe);
-                if (gj == 1) sto(xoq - o.sx, so, xe);
-                if (gj == mp) sto(xoq + o.sx, so, xe);
-            }
-            if constexpr (DENS) {
+            if constexpr (DENS) if (do_d) {
                 // total mass fluxes through the low faces of the cell: the
                 // upwind's donor fluxes of plane Q (x of level n, inflow
                 // values at the walls) plus the limited fluxes; the wall
@@ -730,33 +811,24 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                 sto(pl(dio->m3, SXY, Q), so, f3ns + F3);
                 if (gi == np) {
                     const T w = mpdata::donor(xc, bcx[(gj - 1) + mp * ((Q - 1) + lp)], ldo(u1q + 1, fo));
-                    const T a = sv1[E0][pj][pi + 1];
-                    sto(pl(dio->m1, FXY, Q) + 1, fo,
-                        w + mpdata::pp(a) * mpdata::min3(T(1), CP(2, li + 1, lj), CN(2, li, lj)) -
-                            mpdata::pn(a) * mpdata::min3(T(1), CP(2, li, lj), CN(2, li + 1, lj)));
+                    sto(pl(dio->m1, FXY, Q) + 1, fo, w + T(0));
                 }
                 if (gj == mp) {
                     const T w = mpdata::donor(xc, bcy[(gi - 1) + np * ((Q - 1) + lp)], ldo(u2q + o.yx, so));
-                    const T a = LMID(sv2, E0, 1, 0);
-                    sto(pl(dio->m2, YXY, Q) + o.yx, so,
-                        w + mpdata::pp(a) * mpdata::min3(T(1), CP(2, li, lj + 1), CN(2, li, lj)) -
-                            mpdata::pn(a) * mpdata::min3(T(1), CP(2, li, lj), CN(2, li, lj + 1)));
+                    sto(pl(dio->m2, YXY, Q) + o.yx, so, w + T(0));
                 }
                 if (sky) {
                     const T w = -f3ns;
-                    const T a = -v3q1;
-                    sto(pl(dio->m3, SXY, Q + 1), so,
-                        w + mpdata::pp(a) * mpdata::min3(T(1), CP(3, li, lj), CN(2, li, lj)) -
-                            mpdata::pn(a) * mpdata::min3(T(1), CP(2, li, lj), CN(3, li, lj)));
+                    sto(pl(dio->m3, SXY, Q + 1), so, w + F3p);
                 }
             }
         }
 #undef XA
-#undef CP
-#undef CN
         // ---- the computed queues move to plane K+1 by the slot rotation; V3
         //      of face K goes into the slot of face K-2 ------------------------
-        v3q1 = v3n;
+        if constexpr (!FAST || DENS) LHI(hh, 0) = hP;
+        if constexpr (TAPE) v3q1 = v3q2;
+        if (K <= lp) v3q2 = v3n;
     };
 #undef LMID
 #undef LHI
@@ -774,6 +846,118 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         step(std::integral_constant<int, 5>{}, K);
         if (++K > Ke) break;
     }
+    if (do_d) sto(pl(xo, SXY, k1), so, xst);
+}
+
+// Work of a persistent launch: which (tile, k-range) items each workgroup
+// marches, one after the other.  While there are as many tiles left as
+// workgroups, every workgroup takes a whole one (nfull of them each).  The
+// tiles that remain are laid end to end, each as `ext` = lp + lead units, of
+// which the first `lead` stand for the planes an item marches besides its
+// output (two of xant and one of V/cp/cn recomputed below a cut, two above
+// the item, and its set-up) and the others for its lp planes; this line is
+// cut into equal runs, one a workgroup, so that all of them finish together
+// whatever the numbers of tiles and planes.  Chunks of one length for all
+// tiles, in rounds, left the last round part-empty: at 256x256x128 100 tiles
+// x 2 chunks for 256 CUs, at 384x320x192 504 chunks of 64 planes.  `run` may
+// also be a fixed chunk (the tuning override): then there are more runs than
+// workgroups, and ext is the next multiple of it.
+struct March {
+    int nwg;            // workgroups that take items, a multiple of NXCD from NXCD on
+    int ntx, ntile;
+    int nfull;          // whole tiles per workgroup
+    int run, lead, ext; // see above
+    int grp;            // tiles that are cut together
+};
+
+// Calls item(tile, k0, k1) for this workgroup's items (one call site: the
+// item is inlined once).  Workgroups are dealt to the XCDs round-robin
+// (blockIdx % NXCD), each with its own L2: those of one XCD take neighbouring
+// tiles, and in the whole-tile rounds they march them through the same planes.
+template <typename F>
+__device__ __forceinline__ void march_items(const March& m, int lp, F&& item) {
+    const int nxcd = m.nwg >= NXCD ? NXCD : 1;
+    const int per_xcd = m.nwg / nxcd;
+    const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
+    const int ngrp = m.nwg / m.grp, in_grp = slot % m.grp;
+    const int g = xcd * (per_xcd / m.grp) + slot / m.grp;
+    const int base = m.nwg * m.nfull;  // first of the tiles cut into runs
+    const long long total = (long long)((m.ntile - base + m.grp - 1) / m.grp) * m.ext;
+    long long r = (long long)g * m.run, pos = r, end = min(r + m.run, total);
+    for (int f = 0;;) {
+        int tile, k0, k1;
+        if (f < m.nfull) {
+            tile = (xcd * m.nfull + f++) * per_xcd + slot;
+            k0 = 1;
+            k1 = lp;
+        } else {
+            if (pos >= end) {
+                if (pos == r || (r += (long long)ngrp * m.run) >= total) break;
+                pos = r;
+                end = min(r + m.run, total);
+            }
+            const int tt = (int)(pos / m.ext);
+            const long long t0 = (long long)tt * m.ext, stop = min(end, t0 + m.ext);
+            tile = base + tt * m.grp + in_grp;
+            k0 = max((int)(pos - t0) - m.lead, 0) + 1;
+            k1 = min((int)(stop - t0) - m.lead, lp);
+            pos = stop;
+            if (k1 < k0 || tile >= m.ntile) continue;
+        }
+        item(tile, k0, k1);
+    }
+}
+
+// What marching alone costs a workgroup over marching beside its x
+// neighbours, as a share of a plane's time (any value from 0.06 to 0.25 gives
+// the same plans; without it 256x256x128 takes 252 us instead of 233).
+constexpr double kAlone = 0.12;
+// The plan for `slots` resident workgroups (chunk > 0: runs of that length),
+// with the group of least modelled time: the planes the busiest workgroup
+// marches, dearer the fewer neighbours share their halo columns in L2.
+constexpr int kLead = 5;
+// Planes the busiest workgroup of a plan marches.
+inline long long march_cost(const Geo& g, const March& m) {
+    const long long cut = m.ntile > m.nwg * m.nfull ? m.run + m.lead : 0;
+    return (long long)m.nfull * (g.lp + m.lead) + cut;
+}
+inline double march_time(const Geo& g, const March& m) {
+    return (double)march_cost(g, m) * (1 + kAlone / m.grp);
+}
+template <int RX, int RY>
+March plan_march(const Geo& g, long long slots, int chunk) {
+    March m{};
+    m.ntx = (g.np + RX - 5) / (RX - 4);
+    m.ntile = m.ntx * ((g.mp + RY - 5) / (RY - 4));
+    m.grp = 1;
+    if (slots >= NXCD) slots = slots / NXCD * NXCD;
+    if (chunk > 0) {
+        m.run = std::min(chunk, g.lp);
+        m.ext = (g.lp + m.run - 1) / m.run * m.run;
+        m.nwg = (int)std::min(slots, (long long)m.ntile * (m.ext / m.run));
+        if (m.nwg > NXCD) m.nwg = (m.nwg + NXCD - 1) / NXCD * NXCD;
+        return m;
+    }
+    m.nfull = (int)(m.ntile / slots);
+    m.lead = kLead;
+    m.ext = g.lp + kLead;
+    const long long rest = m.ntile - m.nfull * slots;
+    March best{};
+    for (int grp = 1; grp <= 64; grp *= 2) {
+        if (grp > 1 && (grp > rest || slots % (NXCD * grp))) break;
+        const long long units = (rest + grp - 1) / grp * m.ext, ngrp = slots / grp;
+        m.grp = grp;
+        m.run = (int)std::max(1LL, (units + ngrp - 1) / ngrp);
+        long long nwg = slots;
+        if (m.nfull == 0) {  // no more workgroups than runs, whole groups on every XCD
+            const long long need = (units + m.run - 1) / m.run * grp, per = (long long)NXCD * grp;
+            if (grp > 1 || need > NXCD) nwg = std::min(slots, (need + per - 1) / per * per);
+            else nwg = need;
+        }
+        m.nwg = (int)nwg;
+        if (best.grp == 0 || march_time(g, m) < march_time(g, best)) best = m;
+    }
+    return best;
 }
 
 // Halo cells of x_out that the step does not define keep their x_in values:
@@ -810,8 +994,8 @@ __device__ __forceinline__ int untouched_halo_cell(const Geo& g, uint32_t q, uin
 // Block b of nb copies its share of them.  The step kernels are launched with
 // a few blocks more than they have places for work items (halo_blocks), which
 // do this and nothing else: they run on what the items leave idle, where a
-// kernel of its own came after them (13 us of 1.67 ms at 512x512x256, 4 us
-// and a launch of 28 us at 59^3).
+// kernel of its own came after them (2.7 of 29.8 us at 59^3, 13 us of 1.66 ms
+// at 512x512x256).
 template <typename T>
 __device__ __forceinline__ void copy_untouched_halo(const Geo& g, const T* __restrict__ x,
                                                     T* __restrict__ xo, uint32_t b, uint32_t nb) {
@@ -837,65 +1021,34 @@ inline int halo_blocks(long long cells, int nt) {
 
 template <typename T, int RX, int RY, int MINB, bool FAST = false, int PASS = 0>
 __global__ void __launch_bounds__(RX * RY, MINB)
-k_fused_gauge2(Geo g, Off o, int nitemwg, int ntx, int nty, int nchunk, int clen,
-               const T* __restrict__ x, const T* __restrict__ u1, const T* __restrict__ u2,
-               const T* __restrict__ u3, const T* __restrict__ rhr, const T* __restrict__ h,
-               const T* __restrict__ bcx, const T* __restrict__ bcy, T* __restrict__ xo,
-               PassIO<T> pio) {
+k_fused_gauge2(Geo g, Off o, March m, const T* __restrict__ x, const T* __restrict__ u1,
+               const T* __restrict__ u2, const T* __restrict__ u3, const T* __restrict__ rhr,
+               const T* __restrict__ h, const T* __restrict__ bcx, const T* __restrict__ bcy,
+               T* __restrict__ xo, PassIO<T> pio) {
     __shared__ FusedLds<T, RX, RY> L;
-    if (blockIdx.x >= (unsigned)nitemwg) {
-        copy_untouched_halo<T>(g, x, xo, blockIdx.x - nitemwg, gridDim.x - nitemwg);
+    if (blockIdx.x >= (unsigned)m.nwg) {
+        copy_untouched_halo<T>(g, x, xo, blockIdx.x - m.nwg, gridDim.x - m.nwg);
         return;
     }
-    const int ntile = ntx * nty;
-    // Work-item order: workgroups are dealt to the XCDs round-robin
-    // (blockIdx % NXCD), each with its own L2.  The workgroups of one XCD
-    // take a contiguous run of tiles, item by item in rounds, so that at any
-    // time they march neighbouring tiles through the same k-chunk and share
-    // the halo columns in that L2.  (A split into equal contiguous plane
-    // ranges per workgroup balances the tail better but loses this
-    // alignment and measured slower.)
-    const int nxcd = nitemwg >= NXCD ? NXCD : 1;
-    const int per_xcd = nitemwg / nxcd;                   // workgroups per XCD
-    const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
-    if ((int)blockIdx.x >= per_xcd * nxcd) return;
-    const int tiles_per_xcd = (ntile + nxcd - 1) / nxcd;
-    for (int r = slot; ; r += per_xcd) {
-        const int chunk = r / tiles_per_xcd, tix = r - chunk * tiles_per_xcd;
-        if (chunk >= nchunk) break;
-        const int tile = xcd * tiles_per_xcd + tix;
-        if (tile >= ntile) continue;
-        const int k0 = 1 + chunk * clen, k1 = min(g.lp, k0 + clen - 1);
-        fused_item<T, RX, RY, false, FAST, PASS>(g, o, ntx, tile, k0, k1, x, u1, u2, u3, rhr, h,
+    march_items(m, g.lp, [&](int tile, int k0, int k1) {
+        fused_item<T, RX, RY, false, FAST, PASS>(g, o, m.ntx, tile, k0, k1, x, u1, u2, u3, rhr, h,
                                                  bcx, bcy, xo, L, nullptr, &pio);
-    }
+    });
 }
 
 // The two-pass step that also records the adjoint's tape (fused_item's
 // TAPE), with the work-item order of k_fused_gauge2.
 template <typename T, int RX, int RY, int MINB>
 __global__ void __launch_bounds__(RX * RY, MINB)
-k_fused_gauge_rec(Geo g, Off o, int ntx, int nty, int nchunk, int clen, const T* __restrict__ x,
-                  const T* __restrict__ u1, const T* __restrict__ u2, const T* __restrict__ u3,
-                  const T* __restrict__ rhr, const T* __restrict__ h, const T* __restrict__ bcx,
-                  const T* __restrict__ bcy, T* __restrict__ xo, StdTape<T> tp) {
+k_fused_gauge_rec(Geo g, Off o, March m, const T* __restrict__ x, const T* __restrict__ u1,
+                  const T* __restrict__ u2, const T* __restrict__ u3, const T* __restrict__ rhr,
+                  const T* __restrict__ h, const T* __restrict__ bcx, const T* __restrict__ bcy,
+                  T* __restrict__ xo, StdTape<T> tp) {
     __shared__ FusedLds<T, RX, RY> L;
-    const int ntile = ntx * nty;
-    const int nxcd = gridDim.x >= NXCD ? NXCD : 1;
-    const int per_xcd = gridDim.x / nxcd;
-    const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
-    const int nwg = per_xcd * nxcd;
-    if (blockIdx.x >= nwg) return;
-    const int tiles_per_xcd = (ntile + nxcd - 1) / nxcd;
-    for (int r = slot; ; r += per_xcd) {
-        const int chunk = r / tiles_per_xcd, tix = r - chunk * tiles_per_xcd;
-        if (chunk >= nchunk) break;
-        const int tile = xcd * tiles_per_xcd + tix;
-        if (tile >= ntile) continue;
-        const int k0 = 1 + chunk * clen, k1 = min(g.lp, k0 + clen - 1);
-        fused_item<T, RX, RY, false, false, 0, true>(g, o, ntx, tile, k0, k1, x, u1, u2, u3, rhr,
+    march_items(m, g.lp, [&](int tile, int k0, int k1) {
+        fused_item<T, RX, RY, false, false, 0, true>(g, o, m.ntx, tile, k0, k1, x, u1, u2, u3, rhr,
                                                      h, bcx, bcy, xo, L, nullptr, nullptr, &tp);
-    }
+    });
 }
 
 // Tile configuration (0 = 32x32 lanes at 4 waves per SIMD, the fastest at
@@ -918,7 +1071,7 @@ int fused_chunk_env() {
 // workgroups per XCD than that share has items (a smaller share would
 // leave slots idle while items of the XCD wait for a second round); fewer
 // than NXCD items run without the split.
-int persistent_grid(long long nitem, long long items_per_xcd, int ncu, int per_cu) {
+[[maybe_unused]] int persistent_grid(long long nitem, long long items_per_xcd, int ncu, int per_cu) {
     if (nitem < NXCD) return (int)std::max(1LL, nitem);
     const long long slots = (long long)ncu * std::max(per_cu, 1);
     const long long per_xcd = std::max(1LL, std::min(items_per_xcd, slots / NXCD));
@@ -931,141 +1084,80 @@ long long items_of(const Geo& g, int clen) {
     return ntx * nty * ((g.lp + clen - 1) / clen);
 }
 
-// Wall time of a step, in k-march steps of one workgroup: the XCDs work in
-// parallel, each on its contiguous share of the tiles, in rounds of per_xcd
-// work items, and an item of clen output planes marches clen + kRamp planes
-// (two planes of xant and one of V/cp/cn recomputed below the chunk, two
-// above it, and the item's set-up).
-constexpr int kRamp = 5;
-[[maybe_unused]] long long step_cost(long long ntile, int lp, int clen, long long per_xcd) {
-    const long long nchunk = (lp + clen - 1) / clen;
-    const long long tiles_per_xcd = (ntile + NXCD - 1) / NXCD;
-    const long long rounds = (tiles_per_xcd * nchunk + per_xcd - 1) / per_xcd;
-    return rounds * (clen + kRamp);
-}
-
-template <typename T, int RX, int RY, int MINB>
-int per_cu_of() {
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_fused_gauge2<T, RX, RY, MINB>, RX * RY, 0) !=
-        hipSuccess)
-        return 1;
-    return n > 0 ? n : 1;
-}
-
-// Tiling and k-chunk of a single-domain step.  32x32 tiles recompute the
-// fewest ring cells but give one workgroup per CU: they are used when the
-// domain gives every CU at least two 64-plane work items, with the chunk
-// length (16 planes or more) of least wall time by step_cost (at
-// 512x512x256: 128 planes, three rounds of items per XCD against 5.75, so
-// six, with 64).  A smaller domain takes 32x16 tiles (two workgroups per
-// CU) and the longest chunk of 64 or 32 planes that gives every workgroup
-// slot two items, else 16 (measured: on smaller domains more, shorter
-// items beat fewer, longer ones; a rounds model over 64..8 planes chose
-// 64 at 256x256x128 and was 7 % slower there), and 8 or 4 planes when the
-// domain is so small that its items still fit one per CU.
-// k-chunk length of least modelled wall time for RX x RY tiles of `kernel`,
-// rounds x (clen + 7): the workgroup slots of the device take the work items
-// in rounds, and an item marches its clen output planes plus the planes
-// recomputed below and above it and its set-up.
-template <int RX, int RY, typename K>
-int chunk_by_rounds(const Geo& g, K kernel) {
+// Workgroups of `kernel` that the device holds at once, at most `want` per CU
+// (0: as many as fit).
+template <typename K>
+hipError_t resident(K kernel, int nt, int want, long long& slots) {
     int dev = 0, ncu = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        ncu < 1)
-        ncu = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, RX * RY, 0) != hipSuccess ||
-        per_cu < 1)
-        per_cu = 1;
-    (void)hipGetLastError();
-    const long long slots = (long long)ncu * per_cu;
-    long long best = -1;
-    int clen = 64;
-    for (int c : {64, 32, 16, 8, 4}) {
-        const long long rounds = (items_of<RX, RY>(g, c) + slots - 1) / slots;
-        const long long cost = rounds * (std::min(c, g.lp) + 7);
-        if (best < 0 || cost < best) {
-            best = cost;
-            clen = c;
-        }
-    }
-    return std::min(clen, g.lp);
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, nt, 0);
+    if (e != hipSuccess) return e;
+    per_cu = std::max(per_cu, 1);
+    if (want > 0) per_cu = std::min(per_cu, want);
+    slots = (long long)std::max(ncu, 1) * per_cu;
+    return e;
 }
 
+// How a step is tiled: the tile configuration, the workgroups per CU (0: as
+// many as fit) and the k-chunk if it is prescribed (0: the runs of March).
+struct Tiling {
+    int cfg = 0, per_cu = 0, chunk = 0;
+};
+
+// Modelled time of a step on RX x RY tiles with per_cu workgroups on each of
+// ncu CUs: the planes the busiest workgroup marches, times the time of a
+// plane, which a CU's march of 1024 cells sets (4.3 us in FP64) until there
+// are too few waves to hide the latency of the chain of a plane (2.95 us for
+// 512 cells, so no less than 0.69 of it).
+template <int RX, int RY>
+double tiling_time(const Geo& g, int ncu, int per_cu) {
+    const March m = plan_march<RX, RY>(g, (long long)ncu * per_cu, 0);
+    return march_time(g, m) * std::max(0.69, RX * RY * per_cu / 1024.0);
+}
+
+// Tiling of a single-domain step, the one of least modelled time.  32x32
+// tiles recompute the fewest ring cells (23 % of the lanes against 34 % with
+// 32x16) but are one workgroup a CU and cut a domain more coarsely; 32x16
+// tiles run two to a CU, or alone on it, where a domain is so small that
+// halving the planes of each workgroup no longer pays for halving its speed.
 template <typename T>
-void choose_tiling(const Geo& g, int& cfg, int& clen) {
+Tiling choose_tiling(const Geo& g) {
+    Tiling tl;
+    const int env_cfg = fused_config(), env_chunk = fused_chunk_env();
+    if (env_chunk > 0) tl.chunk = env_chunk;
+    if (env_cfg >= 0) {
+        tl.cfg = env_cfg;
+        return tl;
+    }
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         ncu < 1)
         ncu = 256;
-    const int env_cfg = fused_config(), env_clen = fused_chunk_env();
-    if (env_cfg >= 0) {
-        cfg = env_cfg;
-        clen = env_clen > 0 ? env_clen : 64;
-    } else if (items_of<32, 32>(g, 64) >= 2LL * ncu) {
-        cfg = 0;
-        clen = env_clen;
-        if (env_clen <= 0) {
-            const long long ntile = items_of<32, 32>(g, g.lp);
-            const long long per_xcd = std::max(1LL, (long long)ncu * per_cu_of<T, 32, 32, 4>() / NXCD);
-            long long best = -1;
-            for (int n = 1; n <= g.lp; n++) {
-                const int cl = (g.lp + n - 1) / n;
-                if (cl < 16) break;
-                const long long cost = step_cost(ntile, g.lp, cl, per_xcd);
-                if (best < 0 || cost < best) {
-                    best = cost;
-                    clen = cl;
-                }
-            }
-            if (best < 0) clen = g.lp;
-        }
-    } else {
-        cfg = 1;
-        clen = env_clen > 0 ? env_clen : 16;
-        if (env_clen <= 0)
-            for (int c : {64, 32}) {
-                if (items_of<32, 16>(g, c) >= 4LL * ncu) { clen = c; break; }
-            }
-        // A small domain whose items all get a CU of their own marches
-        // clen + kRamp planes in one round: shorter chunks finish sooner as
-        // long as every XCD's share still fits one workgroup per CU
-        // (measured: 32^3 68 -> 44 us, 59^3 79 -> 45 us per step).
-        if (env_clen <= 0 && clen == 16) {
-            const long long tiles_per_xcd = (items_of<32, 16>(g, g.lp) + NXCD - 1) / NXCD;
-            for (int c : {8, 4}) {
-                if (tiles_per_xcd * ((g.lp + c - 1) / c) > std::max(1, ncu / NXCD)) break;
-                clen = c;
-            }
-        }
-    }
-    if (clen > g.lp) clen = g.lp;
+    const double t32 = tiling_time<32, 32>(g, ncu, 1), t16x2 = tiling_time<32, 16>(g, ncu, 2),
+                 t16 = tiling_time<32, 16>(g, ncu, 1);
+    if (t32 <= t16x2 && t32 <= t16) return tl;
+    tl.cfg = 1;
+    tl.per_cu = t16 < t16x2 ? 1 : 2;
+    return tl;
 }
 
 // Persistent launch of the fixed-position kernel: as many workgroups as fit
-// on the device at once, each looping over (tile, k-chunk) work items.
+// on the device at once, each looping over its items.
 template <typename T, int RX, int RY, int MINB, bool FAST = false, int PASS = 0>
-hipError_t launch2(const Geo& g, const Off& o, int clen, const T* x, T* xout, const T* u1,
+hipError_t launch2(const Geo& g, const Off& o, const Tiling& tl, const T* x, T* xout, const T* u1,
                    const T* u2, const T* u3, const T* rhr, const T* h, const T* bcx, const T* bcy,
                    hipStream_t s, const PassIO<T>& pio = PassIO<T>{}) {
-    const int ntx = (g.np + RX - 5) / (RX - 4), nty = (g.mp + RY - 5) / (RY - 4);
-    const int nchunk = (g.lp + clen - 1) / clen;
-    const int nitem = ntx * nty * nchunk;
-    int dev = 0, ncu = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, k_fused_gauge2<T, RX, RY, MINB, FAST, PASS>, RX * RY, 0);
+    long long slots = 0;
+    const hipError_t e =
+        resident(k_fused_gauge2<T, RX, RY, MINB, FAST, PASS>, RX * RY, tl.per_cu, slots);
     if (e != hipSuccess) return e;
-    const int grid = persistent_grid(nitem, (long long)(ntx * nty + NXCD - 1) / NXCD * nchunk, ncu,
-                                     per_cu);
+    const March m = plan_march<RX, RY>(g, slots, tl.chunk);
     // PASS 1 writes an intermediate, whose halo nothing reads
     const int hb = PASS == 1 ? 0 : halo_blocks(halo_cells(g), RX * RY);
-    k_fused_gauge2<T, RX, RY, MINB, FAST, PASS><<<grid + hb, RX * RY, 0, s>>>(
-        g, o, grid, ntx, nty, nchunk, clen, x, u1, u2, u3, rhr, h, bcx, bcy, xout, pio);
+    k_fused_gauge2<T, RX, RY, MINB, FAST, PASS><<<m.nwg + hb, RX * RY, 0, s>>>(
+        g, o, m, x, u1, u2, u3, rhr, h, bcx, bcy, xout, pio);
     return hipGetLastError();
 }
 
@@ -1074,21 +1166,21 @@ hipError_t launch2(const Geo& g, const Off& o, int clen, const T* x, T* xout, co
 // sc.ul, then the pass kernel advances x2 with them into xout, with the
 // limiter bounds from x (time level n).  Tilings 32x32 and 32x16 lanes.
 template <typename T, bool FAST>
-hipError_t launch_three(const Geo& g, const Off& o, int cfg, int clen, const T* x, T* xout,
+hipError_t launch_three(const Geo& g, const Off& o, const Tiling& tl, const T* x, T* xout,
                         const T* u1, const T* u2, const T* u3, const T* rhr, const T* h,
                         const T* bcx, const T* bcy, const FusedScratch<T>& sc, hipStream_t s) {
     PassIO<T> p1{sc.ul[0], sc.ul[1], sc.ul[2], nullptr};
     PassIO<T> p2{nullptr, nullptr, nullptr, sc.x2};
     hipError_t e;
-    if (cfg == 0) {
-        e = launch2<T, 32, 32, 4, FAST, 1>(g, o, clen, x, sc.x2, u1, u2, u3, rhr, h, bcx, bcy, s, p1);
+    if (tl.cfg == 0) {
+        e = launch2<T, 32, 32, 4, FAST, 1>(g, o, tl, x, sc.x2, u1, u2, u3, rhr, h, bcx, bcy, s, p1);
         if (e == hipSuccess)
-            e = launch2<T, 32, 32, 4, FAST, 2>(g, o, clen, x, xout, sc.ul[0], sc.ul[1], sc.ul[2],
+            e = launch2<T, 32, 32, 4, FAST, 2>(g, o, tl, x, xout, sc.ul[0], sc.ul[1], sc.ul[2],
                                                rhr, h, bcx, bcy, s, p2);
     } else {
-        e = launch2<T, 32, 16, 4, FAST, 1>(g, o, clen, x, sc.x2, u1, u2, u3, rhr, h, bcx, bcy, s, p1);
+        e = launch2<T, 32, 16, 4, FAST, 1>(g, o, tl, x, sc.x2, u1, u2, u3, rhr, h, bcx, bcy, s, p1);
         if (e == hipSuccess)
-            e = launch2<T, 32, 16, 4, FAST, 2>(g, o, clen, x, xout, sc.ul[0], sc.ul[1], sc.ul[2],
+            e = launch2<T, 32, 16, 4, FAST, 2>(g, o, tl, x, xout, sc.ul[0], sc.ul[1], sc.ul[2],
                                                rhr, h, bcx, bcy, s, p2);
     }
     return e;
@@ -1098,48 +1190,27 @@ hipError_t launch_three(const Geo& g, const Off& o, int cfg, int clen, const T* 
 // order of k_fused_gauge2.
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
 __global__ void __launch_bounds__(RX * RY, MINB)
-k_fused_dens(Geo g, Off o, int ntx, int nty, int nchunk, int clen, const T* __restrict__ x,
-             const T* __restrict__ u1, const T* __restrict__ u2, const T* __restrict__ u3,
-             const T* __restrict__ h, const T* __restrict__ bcx, const T* __restrict__ bcy,
-             T* __restrict__ xo, DensIO<T> dio) {
+k_fused_dens(Geo g, Off o, March m, const T* __restrict__ x, const T* __restrict__ u1,
+             const T* __restrict__ u2, const T* __restrict__ u3, const T* __restrict__ h,
+             const T* __restrict__ bcx, const T* __restrict__ bcy, T* __restrict__ xo,
+             DensIO<T> dio) {
     __shared__ FusedLds<T, RX, RY> L;
-    const int ntile = ntx * nty;
-    const int nxcd = gridDim.x >= NXCD ? NXCD : 1;
-    const int per_xcd = gridDim.x / nxcd;
-    const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
-    const int nwg = per_xcd * nxcd;
-    if (blockIdx.x >= nwg) return;
-    const int tiles_per_xcd = (ntile + nxcd - 1) / nxcd;
-    for (int r = slot; ; r += per_xcd) {
-        const int chunk = r / tiles_per_xcd, tix = r - chunk * tiles_per_xcd;
-        if (chunk >= nchunk) break;
-        const int tile = xcd * tiles_per_xcd + tix;
-        if (tile >= ntile) continue;
-        const int k0 = 1 + chunk * clen, k1 = min(g.lp, k0 + clen - 1);
-        fused_item<T, RX, RY, true, FAST>(g, o, ntx, tile, k0, k1, x, u1, u2, u3, nullptr, h, bcx,
-                                          bcy, xo, L, &dio);
-    }
+    march_items(m, g.lp, [&](int tile, int k0, int k1) {
+        fused_item<T, RX, RY, true, FAST>(g, o, m.ntx, tile, k0, k1, x, u1, u2, u3, nullptr, h,
+                                          bcx, bcy, xo, L, &dio);
+    });
 }
 
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
-hipError_t launch_dens(const Geo& g, const Off& o, int clen, const T* x, T* xout, const T* u1,
-                       const T* u2, const T* u3, const T* h, const T* bcx, const T* bcy,
-                       const DensIO<T>& d, hipStream_t s) {
-    const int ntx = (g.np + RX - 5) / (RX - 4), nty = (g.mp + RY - 5) / (RY - 4);
-    const int nchunk = (g.lp + clen - 1) / clen;
-    const int nitem = ntx * nty * nchunk;
-    int dev = 0, ncu = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu,
-                                                         k_fused_dens<T, RX, RY, MINB, FAST>,
-                                                         RX * RY, 0);
+hipError_t launch_dens(const Geo& g, const Off& o, const Tiling& tl, const T* x, T* xout,
+                       const T* u1, const T* u2, const T* u3, const T* h, const T* bcx,
+                       const T* bcy, const DensIO<T>& d, hipStream_t s) {
+    long long slots = 0;
+    const hipError_t e = resident(k_fused_dens<T, RX, RY, MINB, FAST>, RX * RY, tl.per_cu, slots);
     if (e != hipSuccess) return e;
-    const int grid = persistent_grid(nitem, (long long)(ntx * nty + NXCD - 1) / NXCD * nchunk, ncu,
-                                     per_cu);
-    k_fused_dens<T, RX, RY, MINB, FAST><<<grid, RX * RY, 0, s>>>(g, o, ntx, nty, nchunk, clen, x,
-                                                                 u1, u2, u3, h, bcx, bcy, xout, d);
+    const March m = plan_march<RX, RY>(g, slots, tl.chunk);
+    k_fused_dens<T, RX, RY, MINB, FAST><<<m.nwg, RX * RY, 0, s>>>(g, o, m, x, u1, u2, u3, h, bcx,
+                                                                  bcy, xout, d);
     return hipGetLastError();
 }
 
@@ -1212,8 +1283,8 @@ k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int
         w0 = min(nitem, xcd * per);
         w1 = min(nitem, w0 + per);
     } else {
-        w0 = sc->bnd[xcd];
-        w1 = sc->bnd[xcd + 1];
+        w0 = __builtin_amdgcn_readfirstlane(sc->bnd[xcd]);
+        w1 = __builtin_amdgcn_readfirstlane(sc->bnd[xcd + 1]);
     }
     const int nrun = w1 - w0, full = nrun / per_xcd * per_xcd, rem = nrun - full;
     const int split = rem > 0 ? max(1, min(4, per_xcd / rem)) : 1;
@@ -1221,7 +1292,7 @@ k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int
     for (;;) {
         if (threadIdx.x == 0) s_w = atomicAdd(&sc->next[xcd], 1);
         __syncthreads();
-        const int i = s_w;
+        const int i = __builtin_amdgcn_readfirstlane(s_w);
         __syncthreads();  // every thread has read s_w before thread 0 writes it again
         if (i >= ntake) break;
         int w = w0 + i, part = 0, nparts = 1;
@@ -1241,19 +1312,20 @@ k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int
             int lo = 0, hi = nmem - 1;  // last member with item0 <= w
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;
-                if (mem[mid].item0 <= w) lo = mid;
+                if (__builtin_amdgcn_readfirstlane(mem[mid].item0) <= w) lo = mid;
                 else hi = mid - 1;
             }
             q = lo;
-            l = w - mem[q].item0;
+            l = w - __builtin_amdgcn_readfirstlane(mem[q].item0);
         }
-        const Member<T>& m = mem[q];
+        const Member<T> m = uniform(mem[q]);
         const int chunk = l / m.ntile, tile = l - chunk * m.ntile;
         const int c0 = 1 + chunk * m.clen, c1 = min(m.g.lp, c0 + m.clen - 1);
         const int len = c1 - c0 + 1;
-        const int k0 = c0 + len * part / nparts, k1 = c0 + len * (part + 1) / nparts - 1;
+        const int k0 = uniform(c0 + len * part / nparts),
+                  k1 = uniform(c0 + len * (part + 1) / nparts - 1);
         if (k0 > k1) continue;  // a chunk shorter than the split (uniform: every thread)
-        fused_item<T, RX, RY, false, FAST>(m.g, m.o, m.ntx, tile, k0, k1, m.x, m.u1, m.u2, m.u3,
+        fused_item<T, RX, RY, false, FAST>(m.g, m.o, m.ntx, uniform(tile), k0, k1, m.x, m.u1, m.u2, m.u3,
                                            m.rhr, m.h, m.bcx, m.bcy, m.xo, L);
     }
     if (threadIdx.x == 0 && atomicAdd(&sc->done[xcd], 1) == per_xcd - 1) {
@@ -1274,28 +1346,15 @@ Off make_off(const Geo& g) {
     return o;
 }
 
-// The density step on the build FAST selects.  32x32 tiles with 64-plane
-// chunks whenever they give at least half the CUs a work item: the step is
-// not bandwidth-bound, and these re-read the fewest inputs (measured at
-// 256x256x128: 1.60e9 B per call against 2.28e9 B with 32x16 tiles and
-// 16-plane chunks, in the same 1.12 ms); the single-domain rule otherwise
-// and for the tuning overrides.
+// The density step on the build FAST selects, with the tiling of the plain step.
 template <typename T, bool FAST>
 hipError_t dens_step(const Geo& g, const T* x, T* xout, const T* u1, const T* u2, const T* u3,
                      const T* h, const T* bcx, const T* bcy, const DensIO<T>& d, hipStream_t s) {
     const Off o = make_off(g);
-    int cfg = 0, cl = 64;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        ncu < 1)
-        ncu = 256;
-    if (fused_config() >= 0 || fused_chunk_env() > 0 || 2 * items_of<32, 32>(g, 64) < ncu)
-        choose_tiling<T>(g, cfg, cl);
-    if (cl > g.lp) cl = g.lp;
-    if (cfg == 0)
-        return launch_dens<T, 32, 32, 4, FAST>(g, o, cl, x, xout, u1, u2, u3, h, bcx, bcy, d, s);
-    return launch_dens<T, 32, 16, 4, FAST>(g, o, cl, x, xout, u1, u2, u3, h, bcx, bcy, d, s);
+    const Tiling tl = choose_tiling<T>(g);
+    if (tl.cfg == 0)
+        return launch_dens<T, 32, 32, 4, FAST>(g, o, tl, x, xout, u1, u2, u3, h, bcx, bcy, d, s);
+    return launch_dens<T, 32, 16, 4, FAST>(g, o, tl, x, xout, u1, u2, u3, h, bcx, bcy, d, s);
 }
 
 template <int RX, int RY>

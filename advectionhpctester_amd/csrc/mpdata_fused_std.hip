@@ -18,11 +18,11 @@ hipError_t FusedStd<T>::record(const Geo& g, const T* x, T* xout, const T* u1, c
                                const StdTape<T>& tp, hipStream_t s) {
     if (g.px || g.py || g.pz || g.ih != 1) return hipErrorInvalidValue;
     const Off o = make_off(g);
-    int cfg = 1, cl = 64;
-    choose_std(g, k_fused_std<T, 32, 16, 2, true, false, true>, cfg, cl);
+    Tiling tl;
+    if (const int c = fused_chunk_env(); c > 0) tl.chunk = c;
     // xout: the interior and the edge copies; the other halo cells are left
     // alone (the recorded step defines only the interior)
-    return launch_std<T, 32, 16, 2, true, false, true>(g, o, cl, x, xout, u1, u2, u3, rhr, h, bcx,
+    return launch_std<T, 32, 16, 2, true, false, true>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx,
                                                        bcy, s, tp);
 }
 

@@ -610,98 +610,81 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
 template <typename T, int RX, int RY, int MINB, bool NONOS, bool PER, bool TAPE = false,
           bool FAST = false>
 __global__ void __launch_bounds__(RX * RY, MINB)
-k_fused_std(Geo g, Off o, int nitemwg, int ntx, int nty, int nchunk, int clen, const T* __restrict__ x,
-            const T* __restrict__ u1, const T* __restrict__ u2, const T* __restrict__ u3,
-            const T* __restrict__ rhr, const T* __restrict__ h, const T* __restrict__ bcx,
-            const T* __restrict__ bcy, T* __restrict__ xo, StdTape<T> tp) {
+k_fused_std(Geo g, Off o, March m, const T* __restrict__ x, const T* __restrict__ u1,
+            const T* __restrict__ u2, const T* __restrict__ u3, const T* __restrict__ rhr,
+            const T* __restrict__ h, const T* __restrict__ bcx, const T* __restrict__ bcy,
+            T* __restrict__ xo, StdTape<T> tp) {
     __shared__ StdLds<T, RX, RY> L;
-    if (blockIdx.x >= (unsigned)nitemwg) {
-        copy_untouched_halo<T>(g, x, xo, blockIdx.x - nitemwg, gridDim.x - nitemwg);
+    if (blockIdx.x >= (unsigned)m.nwg) {
+        copy_untouched_halo<T>(g, x, xo, blockIdx.x - m.nwg, gridDim.x - m.nwg);
         return;
     }
-    // work-item order of k_fused_gauge2: contiguous tile runs per XCD
-    const int ntile = ntx * nty;
-    const int nxcd = nitemwg >= NXCD ? NXCD : 1;
-    const int per_xcd = nitemwg / nxcd;
-    const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
-    if ((int)blockIdx.x >= per_xcd * nxcd) return;
-    const int tiles_per_xcd = (ntile + nxcd - 1) / nxcd;
-    for (int r = slot; ; r += per_xcd) {
-        const int chunk = r / tiles_per_xcd, tix = r - chunk * tiles_per_xcd;
-        if (chunk >= nchunk) break;
-        const int tile = xcd * tiles_per_xcd + tix;
-        if (tile >= ntile) continue;
-        const int k0 = 1 + chunk * clen, k1 = min(g.lp, k0 + clen - 1);
-        fused_std_item<T, RX, RY, NONOS, PER, TAPE, FAST>(g, o, ntx, tile, k0, k1, x, u1, u2, u3,
+    march_items(m, g.lp, [&](int tile, int k0, int k1) {
+        fused_std_item<T, RX, RY, NONOS, PER, TAPE, FAST>(g, o, m.ntx, tile, k0, k1, x, u1, u2, u3,
                                                           rhr, h, bcx, bcy, xo, L, &tp);
-    }
+    });
 }
 
 template <typename T, int RX, int RY, int MINB, bool NONOS, bool PER, bool TAPE = false,
           bool FAST = false>
-hipError_t launch_std(const Geo& g, const Off& o, int clen, const T* x, T* xout, const T* u1,
-                      const T* u2, const T* u3, const T* rhr, const T* h, const T* bcx,
-                      const T* bcy, hipStream_t s, const StdTape<T>& tp = StdTape<T>{}) {
-    const int ntx = (g.np + RX - 5) / (RX - 4), nty = (g.mp + RY - 5) / (RY - 4);
-    const int nchunk = (g.lp + clen - 1) / clen;
-    const int nitem = ntx * nty * nchunk;
-    int dev = 0, ncu = 0, per_cu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, k_fused_std<T, RX, RY, MINB, NONOS, PER, TAPE, FAST>, RX * RY, 0);
+hipError_t launch_std(const Geo& g, const Off& o, const Tiling& tl, const T* x, T* xout,
+                      const T* u1, const T* u2, const T* u3, const T* rhr, const T* h,
+                      const T* bcx, const T* bcy, hipStream_t s,
+                      const StdTape<T>& tp = StdTape<T>{}) {
+    long long slots = 0;
+    const hipError_t e = resident(k_fused_std<T, RX, RY, MINB, NONOS, PER, TAPE, FAST>, RX * RY,
+                                  tl.per_cu, slots);
     if (e != hipSuccess) return e;
-    const int grid = persistent_grid(nitem, (long long)(ntx * nty + NXCD - 1) / NXCD * nchunk, ncu,
-                                     per_cu);
+    const March m = plan_march<RX, RY>(g, slots, tl.chunk);
     // a recorded step leaves the halo of its output alone
     const int hb = TAPE ? 0 : halo_blocks(halo_cells(g), RX * RY);
-    k_fused_std<T, RX, RY, MINB, NONOS, PER, TAPE, FAST><<<grid + hb, RX * RY, 0, s>>>(
-        g, o, grid, ntx, nty, nchunk, clen, x, u1, u2, u3, rhr, h, bcx, bcy, xout, tp);
+    k_fused_std<T, RX, RY, MINB, NONOS, PER, TAPE, FAST><<<m.nwg + hb, RX * RY, 0, s>>>(
+        g, o, m, x, u1, u2, u3, rhr, h, bcx, bcy, xout, tp);
     return hipGetLastError();
 }
 
-// Tiling and k-chunk of the standard kernel: 32x16 tiles (the 32x32 build
-// spills registers and measured slower at every size), and the chunk length
-// of least modelled wall time (chunk_by_rounds; measured: 128x128x64 78 us
-// at 8 planes against 89 at 16; 64x64x32 4 planes; 256x256x128 and
-// 512x512x256 64 planes).  MPDATA_FUSED_CFG / _CHUNK override both for
-// tests and tuning.
-template <typename K>
-void choose_std(const Geo& g, K kernel, int& cfg, int& clen) {
-    const int env_cfg = fused_config(), env_clen = fused_chunk_env();
-    cfg = env_cfg >= 0 ? env_cfg : 1;
-    clen = env_clen > 0 ? env_clen : chunk_by_rounds<32, 16>(g, kernel);
-    if (clen > g.lp) clen = g.lp;
+// Tiling of the standard kernel: 32x16 tiles (the 32x32 build spills
+// registers and measured slower at every size), two workgroups to a CU or one
+// by the modelled time.  MPDATA_FUSED_CFG / _CHUNK override them for tests
+// and tuning.
+inline Tiling choose_std(const Geo& g) {
+    Tiling tl;
+    const int env_cfg = fused_config(), env_chunk = fused_chunk_env();
+    tl.cfg = env_cfg >= 0 ? env_cfg : 1;
+    if (env_chunk > 0) tl.chunk = env_chunk;
+    if (env_cfg >= 0 || env_chunk > 0) return tl;
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        ncu < 1)
+        ncu = 256;
+    tl.per_cu = tiling_time<32, 16>(g, ncu, 1) < tiling_time<32, 16>(g, ncu, 2) ? 1 : 2;
+    return tl;
 }
 
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
-hipError_t launch_std_any(const Geo& g, const Off& o, int clen, int nonos, const T* x, T* xout,
+hipError_t launch_std_any(const Geo& g, const Off& o, const Tiling& tl, int nonos, const T* x, T* xout,
                           const T* u1, const T* u2, const T* u3, const T* rhr, const T* h,
                           const T* bcx, const T* bcy, hipStream_t s) {
     const bool per = g.px || g.py || g.pz;
     if (nonos) {
-        if (per) return launch_std<T, RX, RY, MINB, true, true, false, FAST>(g, o, clen, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
-        return launch_std<T, RX, RY, MINB, true, false, false, FAST>(g, o, clen, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+        if (per) return launch_std<T, RX, RY, MINB, true, true, false, FAST>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+        return launch_std<T, RX, RY, MINB, true, false, false, FAST>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
     }
-    if (per) return launch_std<T, RX, RY, MINB, false, true, false, FAST>(g, o, clen, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
-    return launch_std<T, RX, RY, MINB, false, false, false, FAST>(g, o, clen, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+    if (per) return launch_std<T, RX, RY, MINB, false, true, false, FAST>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
+    return launch_std<T, RX, RY, MINB, false, false, false, FAST>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
 }
 
-// One step of the standard variant on the build FAST selects: the tiling and
-// chunk of choose_std, then the halo cells the step leaves to x.
+// One step of the standard variant on the build FAST selects.
 template <typename T, bool FAST>
 hipError_t std_step(const Geo& g, int nonos, const T* x, T* xout, const T* u1, const T* u2,
                     const T* u3, const T* rhr, const T* h, const T* bcx, const T* bcy,
                     hipStream_t s) {
     const Off o = make_off(g);
-    int cfg = 1, cl = 64;
-    choose_std(g, k_fused_std<T, 32, 16, 4, true, false, false, FAST>, cfg, cl);
-    hipError_t e =
-        cfg == 0
-            ? launch_std_any<T, 32, 32, 4, FAST>(g, o, cl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
-            : launch_std_any<T, 32, 16, 4, FAST>(g, o, cl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
-    return e;
+    const Tiling tl = choose_std(g);
+    return tl.cfg == 0
+               ? launch_std_any<T, 32, 32, 4, FAST>(g, o, tl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
+               : launch_std_any<T, 32, 16, 4, FAST>(g, o, tl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
 }
 
 }  // namespace

@@ -136,3 +136,26 @@ def test_fused_rejects_unsupported(mp):
         with pytest.raises(mp.MpdataError) as e:
             d.step(x, *u, one, one)
         assert e.value.code == 4
+
+
+@pytest.mark.parametrize("variant", ["gauge", "standard"])
+@pytest.mark.parametrize("size", [(450, 460, 6), (230, 150, 41), (130, 70, 64), (61, 300, 17)])
+def test_runs_cover_the_domain(mp, size, variant):
+    """Sizes at which the equal runs of a launch cross tiles, are cut for
+    groups of tiles with a part-empty last group, and follow a round of whole
+    tiles (289 tiles of 32x32 for 256 workgroups): the stage kernels' bits,
+    every cell written."""
+    c = _case(size + (1,), sum(size), np.float64)
+    with mp.Domain(*size, 1) as d:
+        t = {k: to_dev(v) for k, v in c.items()}
+        kw = dict(variant=mp.GAUGE if variant == "gauge" else mp.STANDARD)
+        xs = t["x"].clone()
+        xo = torch.full_like(t["x"], float("nan"))
+        args = (t["u1"], t["u2"], t["u3"], t["rhr"], t["h"], t["bcx"], t["bcy"])
+        d.set_path(mp.PATH_STAGES)
+        d.step(xs, *args, **kw)
+        d.set_path(mp.PATH_FUSED)
+        print(f"runs {variant} {size}", flush=True)
+        d.step_oop(t["x"], xo, *args, **kw)
+        a, b = to_host(xs), to_host(xo)
+    assert bits_equal(a, b), describe_diff(a, b)
