@@ -482,7 +482,6 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             sx[E1][pj + 1][pi + 1] = in_dom ? xq3 : xown;
             if (t < NRING) sx[E1][rsj][rsi] = xr;
         }
-        const T hP = hq1;
         // Temporaries of a step that are read only under the condition
         // that sets them are left unset rather than zeroed: a default value
         // would cost a register move per step on every path.
@@ -588,7 +587,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         // reader that does not look), so that the LDS reads of all of them
         // go out together instead of one exec region after the other.
         T v3n = T(0);
-        T mx, mn;  // bounds of x and xant on plane P, for C
+        T up, dn;  // (bound - xant) h on plane P, for C
 #define SB __builtin_amdgcn_sched_barrier(0);
         auto stage_b = [&](auto edge) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge)::value;
@@ -641,7 +640,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                         if (own_fy) sto(pl(tp->v[1], YXY, P), tso, val2);
                     }
                 }
-                mx = xw, mn = xw;
+                T mx = xw, mn = xw;
 #define ACC(v, lo, hi) { T t_ = (v); lo = min2(lo, t_); hi = max2(hi, t_); }
                 ACC(xc, mn, mx) ACC(xe, mn, mx) ACC(xs, mn, mx) ACC(xn, mn, mx)
                 if (!gnd) ACC(bc, mn, mx)
@@ -649,12 +648,15 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
 #undef ACC
                 mx = max2(mx, xmx0);
                 mn = min2(mn, xmn0);
+                up = (mx - xc) * hq1;
+                dn = (xc - mn) * hq1;
             }
         };
         if (BC_on && P != 1 && P != lp) stage_b(std::false_type{});
         else stage_b(std::true_type{});
         if constexpr (TAPE)
             if (Dq && own_s) sto(pl(tp->psi, SXY, Q), tso, XA(2, li, lj));
+        T hP;
         // The loaded source-column queues are not read after this point:
         // the oldest slot of each is loaded with the plane step K+1 needs;
         // the latency is covered by C, D and the next step's barrier.
@@ -676,6 +678,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             u2a0 = ldo(qu2, so);
             u2b0 = ldo(qu2 + o.yx, so);
             u3q0 = ldo(qu3, so);
+            if constexpr (!FAST || DENS) hP = hq1;
             hq1 = ldo(qh, so);
             if constexpr (!DENS) rq2 = ldo(qr, so);
             if constexpr (PASS == 2) xaq = ldo(qxa, so);
@@ -689,17 +692,15 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             const bool gnd = EDGE && P == 1, sky = EDGE && P == lp;
             T rp, rn;
             {
-                const T xaP = XA(1, li, lj);
                 T a1p = sv1[pj][pi + 1], a1 = sv1[pj][pi];
                 T a2p = LMID(sv2, 0, 1, 0), a2 = LMID(sv2, 0, 0, 0);
                 T a3p, a3;
                 if (gnd) { a3p = v3n; a3 = -a3p; }
                 else if (sky) { a3 = v3q2; a3p = -a3; }
                 else { a3p = v3n; a3 = v3q2; }
-                T hc = hP;
-                rp = div_<FAST>((mx - xaP) * hc,
+                rp = div_<FAST>(up,
                                 (pn(a1p) + pp(a1) + pn(a2p) + pp(a2) + pn(a3p) + pp(a3) + ep));
-                rn = div_<FAST>((xaP - mn) * hc,
+                rn = div_<FAST>(dn,
                                 (pp(a1p) + pn(a1) + pp(a2p) + pn(a2) + pp(a3p) + pn(a3) + ep));
             }
             // capped here: every reader takes min(1, .) (the tape holds them

@@ -74,8 +74,10 @@ struct StdLds {
     T sf1[RY][RX];            // flux through the left x-face, plane Q
     T sf2[RY][RX];            // flux through the lower y-face, plane Q
     T sw2[RY][RX];            // donor flux of V2 through the lower y-face, plane P
-    T scp[2][RY][RX];         // cp, cn: planes K-2 and K-1
-    T scn[2][RY][RX];
+    T scp[RY][RX];            // cp, cn: plane K-1 from C on, K-2 until then
+    T scn[RY][RX];
+    // a thread's own V1, V2 of plane P until the next step's F
+    T sv1[RY][RX], sv2[RY][RX];
     // h, u1 (face i), u3 (faces P, P+1) of each source column on plane P,
     // read by the position above for V2
     T e_h[RY][RX], e_u1[RY][RX], e_u3a[RY][RX], e_u3b[RY][RX];
@@ -118,8 +120,6 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
     static_assert((64 % RX == 0 || RX % 64 == 0) && NT % 64 == 0, "row layout of the waves");
     static_assert(NRING <= NT, "x ring must fit one extra slot per thread");
     auto& sx = L.sx;
-    auto& sxa = L.sxa;
-    auto& src = L.src;
     const int np = g.np, mp = g.mp, lp = g.lp;
     const bool px = PER && g.px, py = PER && g.py, pz = PER && g.pz;
     const int t = threadIdx.x;
@@ -162,7 +162,6 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
     const bool do_v2 = valid && (py || gj >= 2) && li >= -1 && li <= TX && lj >= -1;
     const bool do_c = valid && li >= -1 && li <= TX && lj >= -1 && lj <= TY;
     const bool do_d = in_dom && li >= 0 && li < TX && lj >= 0 && lj < TY;
-    const bool do_f = li >= 0 && li <= TX && lj >= 0 && lj <= TY;
     // open wall faces, where the per-stage path sets the flux to zero
     // (flux_x_bcd / flux_y_bcd): the left x-face / lower y-face of this
     // position is face gi / gj of the domain
@@ -177,17 +176,17 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
     const XSrc<T> own = valid ? XSrc<T>{x, o.s(ai, aj, 0), SXY} : xsrc(gi, gj);
     const uint32_t so = uint32_t(o.s(ai, aj, 1 - o.ih)) * uint32_t(sizeof(T));
     const uint32_t fo = uint32_t(o.f1(ai, aj, 1 - o.ih)) * uint32_t(sizeof(T));
-    // faces i+1 and j+1 of the source column, and x-face i+1 of its column
-    // j-1 (wrapped in periodic directions)
-    uint32_t fob = 0, sob = 0, fjmb = 0;
+    // faces i+1 and j+1 of the source column (wrapped in periodic directions)
+    uint32_t fob = 0, sob = 0;
     if constexpr (PER) {
         const int ib = (px && ai == np) ? 1 : ai + 1;
         const int jb = (py && aj == mp) ? 1 : aj + 1;
-        const int jm = (py && aj == 1) ? mp : aj - 1;
         fob = uint32_t(o.f1(ib, aj, 1 - o.ih)) * uint32_t(sizeof(T));
         sob = uint32_t(o.f2(ai, jb, 1 - o.ih)) * uint32_t(sizeof(T));
-        fjmb = uint32_t(o.f1(ib, jm, 1 - o.ih)) * uint32_t(sizeof(T));
     }
+    // past an open x's last column a position holds a mirrored column's u1:
+    // its element of e_u1 is the last column's face n+1 instead
+    const bool wall_e = !px && gi == np + 1, last_e = !px && gi == np && pi < RX - 1;
     // tape ownership: x/y halo cells of xant and the wall faces n+1 belong to
     // the tile whose output range touches them
     bool own_fx = false, own_fy = false, own_s = false;
@@ -207,14 +206,14 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
     }
     const int ihm = o.ih - 1;
     auto pl = [&](auto* a, int stride, int k) { return a + (long long)stride * (k + ihm); };
-    // loads of the source column's faces i+1 / j+1 and of column j-1 on plane k
-    auto ld_u1b = [&](int k) -> T {
-        if constexpr (PER) return ldo(pl(u1, FXY, k), fob);
-        else return ldo(pl(u1, FXY, k) + 1, fo);
+    // loads of the source column's faces i+1 / j+1 on the plane at p
+    auto ld_u1b = [&](const T* p) -> T {
+        if constexpr (PER) return ldo(p, fob);
+        else return ldo(p + 1, fo);
     };
-    auto ld_u2b = [&](int k) -> T {
-        if constexpr (PER) return ldo(pl(u2, YXY, k), sob);
-        else return ldo(pl(u2, YXY, k) + o.yx, so);
+    auto ld_u2b = [&](const T* p) -> T {
+        if constexpr (PER) return ldo(p, sob);
+        else return ldo(p + o.yx, so);
     };
     const XSrc<T> ring = t < NRING ? xsrc(i0 + rsi - 3, j0 + rsj - 3) : XSrc<T>{nullptr, 0, 0};
     // x-neighbour availability for the in-plane max/min (edge copies on open
@@ -225,29 +224,92 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
     const int Alast = pz ? k1 + 2 : min(lp, k1 + 2);
     const int Plo = pz ? k0 - 1 : max(1, k0 - 1), Phi = pz ? k1 + 1 : min(lp, k1 + 1);
     // register queues of the source column (as in the gauge kernel) and of
-    // the position's own pseudo-velocities: v1q/v2q planes Q and P, v3q
-    // faces K-2 and K-1, w3q the donor flux of V3 on the same faces
+    // the position's own V3 and its donor flux on face K-1
     T xq[3], u1a[2], u1b[2], u2a[2], u2b[2], u3q[3], hq[2];
     xq[0] = ldo(pl(x, SXY, kc(Ks - 1)), so); xq[1] = ldo(pl(x, SXY, kc(Ks)), so);
     xq[2] = ldo(pl(x, SXY, kc(Ks + 1)), so);
     u1a[0] = ldo(pl(u1, FXY, kc(Ks - 1)), fo); u1a[1] = ldo(pl(u1, FXY, kc(Ks)), fo);
-    u1b[0] = ld_u1b(kc(Ks - 1)); u1b[1] = ld_u1b(kc(Ks));
+    u1b[0] = ld_u1b(pl(u1, FXY, kc(Ks - 1))); u1b[1] = ld_u1b(pl(u1, FXY, kc(Ks)));
     u2a[0] = ldo(pl(u2, YXY, kc(Ks - 1)), so); u2a[1] = ldo(pl(u2, YXY, kc(Ks)), so);
-    u2b[0] = ld_u2b(kc(Ks - 1)); u2b[1] = ld_u2b(kc(Ks));
+    u2b[0] = ld_u2b(pl(u2, YXY, kc(Ks - 1))); u2b[1] = ld_u2b(pl(u2, YXY, kc(Ks)));
     u3q[0] = ldo(pl(u3, SXY, fc(Ks - 1)), so); u3q[1] = ldo(pl(u3, SXY, fc(Ks)), so);
     u3q[2] = ldo(pl(u3, SXY, fc(Ks + 1)), so);
     hq[0] = ldo(pl(h, SXY, kc(Ks - 1)), so); hq[1] = ldo(pl(h, SXY, kc(Ks)), so);
     T rq2 = ldo(pl(rhr, SXY, kc(Ks)), so);
-    T v1q[2] = {T(0), T(0)}, v2q[2] = {T(0), T(0)};
-    T v3q[2] = {T(0), T(0)}, w3q[2] = {T(0), T(0)};
+    T v3 = T(0), w3 = T(0);
+    T v3q1 = T(0);  // V3 on face K-2, for the tape
     T xmx[2] = {T(0), T(0)}, xmn[2] = {T(0), T(0)};
     T f3c = T(0);  // flux through the upper z-face of the last output plane
 
     sx[0][pj + 1][pi + 1] = valid ? xq[1] : ld(own, Ks);
     if (t < NRING) sx[0][rsj][rsi] = ld(ring, Ks);
+    // x of plane K+1 for the LDS: ring cell, and the own cell where it is
+    // not in the queue; loaded a step ahead (a null source keeps the zero)
+    T xr = T(0), xown = T(0);
+    const bool ring_on = t < NRING && ring.p, own_on = !valid && own.p;
+    const uint32_t rstr = uint32_t(ring.stride) * uint32_t(sizeof(T)),
+                   ostr = uint32_t(own.stride) * uint32_t(sizeof(T));
+    const char* rp = ring_on ? (const char*)(ring.p + ring.base) : nullptr;
+    const char* op = own_on ? (const char*)(own.p + own.base) : nullptr;
+    if constexpr (!PER) {
+        rp += (uint64_t)rstr * (uint32_t)Ks;
+        op += (uint64_t)ostr * (uint32_t)Ks;
+    }
+    auto ld_halo = [&](int k) __attribute__((always_inline)) {
+        if constexpr (PER) {
+            if (ring_on) xr = ldo((const T*)(rp + (uint64_t)rstr * (uint32_t)kc(k)), 0);
+            if (own_on) xown = ldo((const T*)(op + (uint64_t)ostr * (uint32_t)kc(k)), 0);
+        } else {
+            rp += rstr;
+            op += ostr;
+            if (ring_on) xr = ldo((const T*)rp, 0);
+            if (own_on) xown = ldo((const T*)op, 0);
+        }
+    };
+    if (Ks + 1 <= Alast) ld_halo(Ks + 1);
     __syncthreads();
 
     uint32_t so_k = so, fo_k = fo;
+    // x of the source column's 3x3 neighbourhood, from one opaque address
+    using LT = StdLds<T, RX, RY>;
+    constexpr int SZ = (int)sizeof(T);
+    // and the position's own elements of the tile arrays, from three (the
+    // arrays lie beyond the reach of one immediate offset, and without this
+    // the compiler keeps a dozen address registers through the loop)
+    constexpr int PLN = RY * RX * SZ;  // one plane of a tile array
+    constexpr int MID = (int)offsetof(LT, sf1);
+    constexpr int HI = (int)offsetof(LT, e_h) - RX * SZ;  // read one row back
+    uint32_t lsx = uint32_t(offsetof(LT, sx) + ((saj - 1) * SW + (sai - 1)) * SZ);
+    uint32_t llo = uint32_t(t * SZ), lmid = uint32_t(MID + t * SZ), lhi = uint32_t(HI + t * SZ);
+    asm volatile("" : "+v"(lsx), "+v"(llo), "+v"(lmid), "+v"(lhi));
+    char* const lds0 = reinterpret_cast<char*>(&L);
+#define LSX(s, db, da) \
+    (*reinterpret_cast<T*>(lds0 + lsx + ((s) * (SW * SH) + (db) * SW + (da)) * SZ))
+// array `arr` at ring slot s, offset (db rows, da columns) from the position
+#define LLO(arr, s, db, da) \
+    (*reinterpret_cast<T*>(lds0 + llo + ((int)offsetof(LT, arr) + (s) * PLN + ((db) * RX + (da)) * SZ)))
+#define LMID(arr, db, da) \
+    (*reinterpret_cast<T*>(lds0 + lmid + ((int)offsetof(LT, arr) - MID + ((db) * RX + (da)) * SZ)))
+#define LHI(arr, r) (*reinterpret_cast<T*>(lds0 + lhi + ((int)offsetof(LT, arr) - HI + (r) * SZ)))
+    // Plane pointers of the loads of a step (in scalar registers): moved by a
+    // plane until the last one on open lids, formed anew with a periodic z.
+    // a limiter factor: min(1, a, b), where cp and cn are held as min(1, .)
+    // (the tape holds them as they are)
+    auto lmin = [](T a, T b) {
+        if constexpr (TAPE) return min3(T(1), a, b);
+        else return min2(a, b);
+    };
+    const uint32_t SB8 = SXY * SZ, FB8 = FXY * SZ, YB8 = YXY * SZ;
+    const T* qx = uniform(pl(x, SXY, kc(Ks + 1)));
+    const T* qu1 = uniform(pl(u1, FXY, kc(Ks)));
+    const T* qu2 = uniform(pl(u2, YXY, kc(Ks)));
+    const T* qu3 = uniform(pl(u3, SXY, fc(Ks + 1)));
+    const T* qh = uniform(pl(h, SXY, kc(Ks)));
+    const T* qr = uniform(pl(rhr, SXY, kc(Ks)));
+    auto adv = [](auto* p, uint32_t d) { return (decltype(p))((uintptr_t)uniform(p) + d); };
+    T* qxo = uniform(pl(xo, SXY, Ks - 4));  // plane K-3 during step K
+    T xst = T(0);                           // the new x of that plane
+    const bool edge_d = do_d && ((!px && (gi == 1 || gi == np)) || (!py && (gj == 1 || gj == mp)));
     auto step = [&](auto phase, int K) __attribute__((always_inline)) {
         constexpr int PH = decltype(phase)::value;
         asm volatile("" : "+s"(K));
@@ -259,44 +321,55 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         T& u2a0 = u2a[Q2a]; T& u2a1 = u2a[Q2b]; T& u2b0 = u2b[Q2a]; T& u2b1 = u2b[Q2b];
         T& u3q0 = u3q[Q3a]; T& u3q1 = u3q[Q3b]; T& u3q2 = u3q[Q3c];
         T& hq1 = hq[Q2a]; T& hq2 = hq[Q2b];
-        T& v1Q = v1q[Q2a]; T& v1P = v1q[Q2b]; T& v2Q = v2q[Q2a]; T& v2P = v2q[Q2b];
-        T& v3q1 = v3q[Q2a]; T& v3q2 = v3q[Q2b]; T& w3q1 = w3q[Q2a]; T& w3q2 = w3q[Q2b];
         T& xmx0 = xmx[Q2a]; T& xmn0 = xmn[Q2a]; T& xmx1 = xmx[Q2b]; T& xmn1 = xmn[Q2b];
         asm volatile("" : "+v"(so_k), "+v"(fo_k));
         const uint32_t so = so_k, fo = fo_k;
-        const bool A_on = K <= Alast, An_on = K + 1 <= Alast;
-        // h and rhr of the output plane Q=K-2 for D
-        const T hQ = ldo(pl(h, SXY, kc(K - 2)), so);
-        const T rQ = ldo(pl(rhr, SXY, kc(K - 2)), so);
-        const T hP = hq1;
-        T xr, xown;
-        if (An_on) {
-            if (t < NRING) xr = ld(ring, K + 1);
-            if (!valid) xown = ld(own, K + 1);
+        const bool A_on = K <= Alast;
+        // the one wait for the loads of the step, then the store of the last
+        // output plane and the edge copies (as in the gauge kernel)
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        qxo = adv(qxo, SB8);
+        if (do_d && K - 3 >= k0 && K - 3 <= k1) sto(qxo, so, xst);
+        if (edge_d && K >= k0 && K <= k1) {
+            T* const xok = pl(xo, SXY, K);
+            if (!px && gi == 1) sto(xok - 1, so, xq2);
+            if (!px && gi == np) sto(xok + 1, so, xq2);
+            if (!py && gj == 1) sto(xok - o.sx, so, xq2);
+            if (!py && gj == mp) sto(xok + o.sx, so, xq2);
         }
+        if (K + 1 <= Alast) {
+            sx[E1][pj + 1][pi + 1] = valid ? xq3 : xown;
+            if (t < NRING) sx[E1][rsj][rsi] = xr;
+        }
+        // V1's inputs from column i-1: the source column of the lane to the
+        // left wherever V1 is formed (gi >= 2, or a periodic x)
+        const T hx = from_left_lane(hq1) + hq1;
+        const T s2x = from_left_lane(u2a0 + u2b0) + u2b0 + u2a0;
+        const T s3x = from_left_lane(u3q0 + u3q1) + u3q1 + u3q0;
         const int P = K - 1;
         const bool BC_on = P >= Plo && P <= Phi;
         // the source column's inputs of V2 at the position above (its
         // column j-1)
         if (BC_on) {
-            L.e_h[pj][pi] = hq1;
-            L.e_u1[pj][pi] = u1a0;
-            L.e_u3a[pj][pi] = u3q0;
-            L.e_u3b[pj][pi] = u3q1;
+            LHI(e_h, 0) = hq1;
+            if (!wall_e) LHI(e_u1, 0) = u1a0;
+            if (last_e) LHI(e_u1, 1) = u1b0;
+            LHI(e_u3a, 0) = u3q0;
+            LHI(e_u3b, 0) = u3q1;
         }
 
         // ---- A: xant and xant/rhr on plane K ------------------------------
         T xa_new;
         auto stage_a = [&](auto edge) __attribute__((always_inline)) {
             constexpr bool EDGE = decltype(edge)::value;
-            auto& sx = L.sx[E0];
             const bool gnd = EDGE && !pz && K == 1, sky = EDGE && !pz && K == lp;
             const T xc = xq2;
+            const T xw = LSX(E0, 1, 0), xe = LSX(E0, 1, 2), xs = LSX(E0, 0, 1), xn = LSX(E0, 2, 1);
             const T hinv = rcp_<FAST>(hq2);
-            const T f1p = donor(xc, sx[saj][sai + 1], u1b1);
-            const T f1 = donor(sx[saj][sai - 1], xc, u1a1);
-            const T f2p = donor(xc, sx[saj + 1][sai], u2b1);
-            const T f2 = donor(sx[saj - 1][sai], xc, u2a1);
+            const T f1p = donor(xc, xe, u1b1);
+            const T f1 = donor(xw, xc, u1a1);
+            const T f2p = donor(xc, xn, u2b1);
+            const T f2 = donor(xs, xc, u2a1);
             T f3p, f3;
             if (gnd) {
                 f3p = donor(xc, xq3, u3q2);
@@ -309,14 +382,14 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
                 f3 = donor(xq1, xc, u3q1);
             }
             xa_new = rq2 * (xc - (f1p - f1 + f2p - f2 + f3p - f3) * hinv);
-            sxa[R0][pj][pi] = xa_new;
-            src[R0][pj][pi] = div_<FAST>(xa_new, rq2);
+            LLO(sxa, R0, 0, 0) = xa_new;
+            LLO(src, R0, 0, 0) = div_<FAST>(xa_new, rq2);
             if constexpr (NONOS) {
                 T m = xc, n = xc;
-                if (nxm) { T v = sx[pj + 1][pi]; m = max2(m, v); n = min2(n, v); }
-                if (nxp) { T v = sx[pj + 1][pi + 2]; m = max2(m, v); n = min2(n, v); }
-                if (nym) { T v = sx[pj][pi + 1]; m = max2(m, v); n = min2(n, v); }
-                if (nyp) { T v = sx[pj + 2][pi + 1]; m = max2(m, v); n = min2(n, v); }
+                { const T v = nxm ? xw : xc; m = max2(m, v); n = min2(n, v); }
+                { const T v = nxp ? xe : xc; m = max2(m, v); n = min2(n, v); }
+                { const T v = nym ? xs : xc; m = max2(m, v); n = min2(n, v); }
+                { const T v = nyp ? xn : xc; m = max2(m, v); n = min2(n, v); }
                 if (!gnd) { m = max2(m, xq1); n = min2(n, xq1); }
                 if (!sky) { m = max2(m, xq3); n = min2(n, xq3); }
                 xmx1 = m;
@@ -327,237 +400,230 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
             if (!pz && (K == 1 || K == lp)) stage_a(std::true_type{});
             else stage_a(std::false_type{});
         }
-        if (An_on) {
-            sx[E1][pj + 1][pi + 1] = valid ? xq3 : xown;
-            if (t < NRING) sx[E1][rsj][rsi] = xr;
-        }
         __syncthreads();
-// xant, |xant|, xant/rhr, cp, cn of plane K-d at tile position (a, b)
-#define XA(d, a, b) sxa[(d) == 0 ? R0 : ((d) == 1 ? R1 : R2)][(b) + 2][(a) + 2]
-#define AX(d, a, b) abs_(XA(d, a, b))
-#define RC(d, a, b) src[(d) == 0 ? R0 : ((d) == 1 ? R1 : R2)][(b) + 2][(a) + 2]
-#define CP(d, a, b) L.scp[((d) & 1) ? E1 : E0][(b) + 2][(a) + 2]
-#define CN(d, a, b) L.scn[((d) & 1) ? E1 : E0][(b) + 2][(a) + 2]
+// xant, xant/rhr of plane K-d at tile position (a, b)
+#define XA(d, a, b) LLO(sxa, (d) == 0 ? R0 : ((d) == 1 ? R1 : R2), (b) - lj, (a) - li)
+#define RC(d, a, b) LLO(src, (d) == 0 ? R0 : ((d) == 1 ? R1 : R2), (b) - lj, (a) - li)
+// cp, cn of plane Q until C
+#define CP(a, b) LMID(scp, (b) - lj, (a) - li)
+#define CN(a, b) LMID(scn, (b) - lj, (a) - li)
         const int Q = K - 2;
         const bool Dq = Q >= k0 && Q <= k1;
         // ---- limited fluxes through the left x-face and lower y-face of this
         //      position on plane Q (antidiff3d-standard-gpubc.f90:372-407):
         //      V of Q from the previous step, cp/cn of Q and Q-1; formed
         //      before B so that V of Q is dead before V of P is formed ------
-        if (Dq && do_f) {
-            T F1 = T(0), F2 = T(0);
-            if (!wall1) {
-                T vl = v1Q;
-                if constexpr (NONOS)
-                    vl = slim(vl, min3(T(1), CP(2, li, lj), CN(2, li - 1, lj)),
-                              min3(T(1), CP(2, li - 1, lj), CN(2, li, lj)), XA(2, li - 1, lj),
-                              XA(2, li, lj));
-                F1 = donor(RC(2, li - 1, lj), RC(2, li, lj), vl);
+        if (Dq) {
+            T vl = LMID(sv1, 0, 0), vb = LMID(sv2, 0, 0);
+            if constexpr (NONOS) {
+                const T c0 = CP(li, lj), n0 = CN(li, lj);
+                vl = slim(vl, lmin(c0, CN(li - 1, lj)), lmin(CP(li - 1, lj), n0), XA(2, li - 1, lj),
+                          XA(2, li, lj));
+                vb = slim(vb, lmin(c0, CN(li, lj - 1)), lmin(CP(li, lj - 1), n0), XA(2, li, lj - 1),
+                          XA(2, li, lj));
             }
-            if (!wall2) {
-                T vl = v2Q;
-                if constexpr (NONOS)
-                    vl = slim(vl, min3(T(1), CP(2, li, lj), CN(2, li, lj - 1)),
-                              min3(T(1), CP(2, li, lj - 1), CN(2, li, lj)), XA(2, li, lj - 1),
-                              XA(2, li, lj));
-                F2 = donor(RC(2, li, lj - 1), RC(2, li, lj), vl);
-            }
-            L.sf1[pj][pi] = F1;
-            L.sf2[pj][pi] = F2;
+            const T F1 = donor(RC(2, li - 1, lj), RC(2, li, lj), vl);
+            const T F2 = donor(RC(2, li, lj - 1), RC(2, li, lj), vb);
+            LMID(sf1, 0, 0) = wall1 ? T(0) : F1;
+            LMID(sf2, 0, 0) = wall2 ? T(0) : F2;
         }
         if constexpr (TAPE)
             if (Dq && own_s) sto(pl(tp->psi, SXY, Q), tso, XA(2, li, lj));
         // ---- B: V3 on face K, V1/V2 on plane P (antidiff3d-standard-
         //      gpubc.f90:72-202), their donor fluxes for the limiter -------
+        // Straight-line on the interior planes (see the gauge kernel).
         T v3n = T(0), w3n = T(0);
-        if (A_on && do_c && (pz || K >= 2) && K >= k0 - 1) {
-            const T hmz = rcp_<FAST>(T(0.5) * (hq1 + hq2));
-            const T s1 = u1a0 + u1a1 + u1b1 + u1b0;
-            const T s2 = u2a0 + u2b0 + u2b1 + u2a1;
-            const T a = u3q1;
-            v3n = vdyfa_<FAST>(XA(1, li, lj), xa_new, a, hmz) +
-                  vcorra_<FAST>(a, s1,
-                         (AX(1, li + 1, lj) + AX(0, li + 1, lj)) - (AX(1, li - 1, lj) + AX(0, li - 1, lj)),
-                         AX(1, li + 1, lj) + AX(0, li + 1, lj) + AX(1, li - 1, lj) + AX(0, li - 1, lj) + ep,
-                         hmz) +
-                  vcorra_<FAST>(a, s2,
-                         (AX(1, li, lj + 1) + AX(0, li, lj + 1)) - (AX(1, li, lj - 1) + AX(0, li, lj - 1)),
-                         AX(1, li, lj + 1) + AX(0, li, lj + 1) + AX(1, li, lj - 1) + AX(0, li, lj - 1) + ep,
-                         hmz);
-            if constexpr (NONOS) w3n = donor(XA(1, li, lj), xa_new, v3n);
-        }
-        // column i-1 of V1 on plane P: the source column of the lane to the
-        // left wherever V1 is formed (gi >= 2, or a periodic x)
-        const T nv1_h = from_left_lane(hq1);
-        const T nv1_u2a = from_left_lane(u2a0);
-        const T nv1_u2b = from_left_lane(u2b0);
-        const T nv1_u3a = from_left_lane(u3q0);
-        const T nv1_u3b = from_left_lane(u3q1);
         T w1 = T(0), w2 = T(0);  // donor fluxes of V1/V2 (left, lower faces of P)
-        if (BC_on) {
-            const bool zterms = pz || !(P == 1 || P == lp);
-            T val1 = T(0), val2 = T(0);
-            if (do_v1) {
-                const T hmx = rcp_<FAST>(T(0.5) * (nv1_h + hq1));
-                const T s2 = nv1_u2a + nv1_u2b + u2b0 + u2a0;
-                const T a = u1a0;
-                val1 = vdyfa_<FAST>(XA(1, li - 1, lj), XA(1, li, lj), a, hmx) +
-                       vcorra_<FAST>(a, s2,
-                              (AX(1, li - 1, lj + 1) + AX(1, li, lj + 1)) -
-                                  (AX(1, li - 1, lj - 1) + AX(1, li, lj - 1)),
-                              AX(1, li - 1, lj + 1) + AX(1, li, lj + 1) + AX(1, li - 1, lj - 1) +
-                                  AX(1, li, lj - 1) + ep,
-                              hmx);
-                if (zterms) {
-                    const T s3 = nv1_u3a + nv1_u3b + u3q1 + u3q0;
-                    val1 = val1 + vcorra_<FAST>(a, s3,
-                                         (AX(0, li - 1, lj) + AX(0, li, lj)) -
-                                             (AX(2, li - 1, lj) + AX(2, li, lj)),
-                                         AX(0, li - 1, lj) + AX(0, li, lj) + AX(2, li - 1, lj) +
-                                             AX(2, li, lj) + ep,
-                                         hmx);
-                }
-                if constexpr (NONOS) w1 = donor(XA(1, li - 1, lj), XA(1, li, lj), val1);
+        T up, dn;  // (bound - xant) h on plane P, for C
+#define SB __builtin_amdgcn_sched_barrier(0);
+        auto stage_b = [&](auto edge) __attribute__((always_inline)) {
+            constexpr bool EDGE = decltype(edge)::value;
+            const bool gnd = EDGE && !pz && P == 1, sky = EDGE && !pz && P == lp;
+            const T xc = XA(1, li, lj), xw = XA(1, li - 1, lj), xe = XA(1, li + 1, lj),
+                    xs = XA(1, li, lj - 1), xn = XA(1, li, lj + 1);
+            T kw, ks, ke, kn;  // plane K
+            if (!EDGE || A_on) {
+                kw = XA(0, li - 1, lj); ks = XA(0, li, lj - 1);
+                ke = XA(0, li + 1, lj); kn = XA(0, li, lj + 1);
             }
-            if (do_v2) {  // pj >= 1 where V2 is formed
-                // column j-1: the source column of the position below; u1 on
-                // its face i+1 is the next position's face i, except on an
-                // open x's last column, whose right neighbour is a mirrored
-                // ring position
-                const T nv2_h = L.e_h[pj - 1][pi];
-                const T nv2_u1a = L.e_u1[pj - 1][pi];
-                const T nv2_u3a = L.e_u3a[pj - 1][pi];
-                const T nv2_u3b = L.e_u3b[pj - 1][pi];
-                T nv2_u1b;
-                if (!px && gi == np) {
-                    if constexpr (PER) nv2_u1b = ldo(pl(u1, FXY, kc(P)), fjmb);
-                    else nv2_u1b = ldo(pl(u1, FXY, kc(P)) - o.fx + 1, fo);
-                } else {
-                    nv2_u1b = L.e_u1[pj - 1][pi + 1];
-                }
-                const T hmy = rcp_<FAST>(T(0.5) * (nv2_h + hq1));
-                const T s1 = nv2_u1a + u1a0 + u1b0 + nv2_u1b;
-                const T a = u2a0;
-                val2 = vdyfa_<FAST>(XA(1, li, lj - 1), XA(1, li, lj), a, hmy) +
-                       vcorra_<FAST>(a, s1,
-                              (AX(1, li + 1, lj - 1) + AX(1, li + 1, lj)) -
-                                  (AX(1, li - 1, lj - 1) + AX(1, li - 1, lj)),
-                              AX(1, li + 1, lj - 1) + AX(1, li + 1, lj) + AX(1, li - 1, lj - 1) +
-                                  AX(1, li - 1, lj) + ep,
-                              hmy);
-                if (zterms) {
-                    const T s3 = nv2_u3a + u3q0 + u3q1 + nv2_u3b;
-                    val2 = val2 + vcorra_<FAST>(a, s3,
-                                         (AX(0, li, lj - 1) + AX(0, li, lj)) -
-                                             (AX(2, li, lj - 1) + AX(2, li, lj)),
-                                         AX(0, li, lj - 1) + AX(0, li, lj) + AX(2, li, lj - 1) +
-                                             AX(2, li, lj) + ep,
-                                         hmy);
-                }
-                if constexpr (NONOS) w2 = donor(XA(1, li, lj - 1), XA(1, li, lj), val2);
+            if (!EDGE || (A_on && (pz || K >= 2) && K >= k0 - 1)) {
+                const T hmz = rcp_<FAST>(T(0.5) * (hq1 + hq2));
+                const T s1 = u1a0 + u1a1 + u1b1 + u1b0;
+                const T s2 = u2a0 + u2b0 + u2b1 + u2a1;
+                const T a = u3q1;
+                v3n = vdyfa_<FAST>(xc, xa_new, a, hmz) +
+                      vcorra_<FAST>(a, s1, (abs_(xe) + abs_(ke)) - (abs_(xw) + abs_(kw)),
+                                    abs_(xe) + abs_(ke) + abs_(xw) + abs_(kw) + ep, hmz) +
+                      vcorra_<FAST>(a, s2, (abs_(xn) + abs_(kn)) - (abs_(xs) + abs_(ks)),
+                                    abs_(xn) + abs_(kn) + abs_(xs) + abs_(ks) + ep, hmz);
+                if constexpr (NONOS) w3n = donor(xc, xa_new, v3n);
             }
-            v1P = val1;
-            v2P = val2;
-            if constexpr (NONOS) L.sw2[pj][pi] = w2;
-            if constexpr (TAPE) {
-                if (P >= k0 && P <= k1) {
-                    if (own_fx) sto(pl(tp->v[0], FXY, P), tfo, val1);
-                    if (own_fy) sto(pl(tp->v[1], YXY, P), tso, val2);
+            SB
+            if (!EDGE || BC_on) {
+                const T xsw = XA(1, li - 1, lj - 1), xnw = XA(1, li - 1, lj + 1),
+                        xse = XA(1, li + 1, lj - 1);
+                const T bc = XA(2, li, lj);
+                T val1, val2;
+                {
+                    const T hmx = rcp_<FAST>(T(0.5) * hx);
+                    const T a = u1a0;
+                    val1 = vdyfa_<FAST>(xw, xc, a, hmx) +
+                           vcorra_<FAST>(a, s2x, (abs_(xnw) + abs_(xn)) - (abs_(xsw) + abs_(xs)),
+                                         abs_(xnw) + abs_(xn) + abs_(xsw) + abs_(xs) + ep, hmx);
+                    if (!gnd && !sky) {
+                        const T bw = XA(2, li - 1, lj);
+                        val1 = val1 + vcorra_<FAST>(a, s3x,
+                                                    (abs_(kw) + abs_(xa_new)) - (abs_(bw) + abs_(bc)),
+                                                    abs_(kw) + abs_(xa_new) + abs_(bw) + abs_(bc) + ep,
+                                                    hmx);
+                    }
+                }
+                SB
+                {
+                    // column j-1: the source column of the position below
+                    const T nv2_h = LHI(e_h, -RX), nv2_u1a = LHI(e_u1, -RX),
+                            nv2_u1b = LHI(e_u1, -RX + 1), nv2_u3a = LHI(e_u3a, -RX),
+                            nv2_u3b = LHI(e_u3b, -RX);
+                    const T hmy = rcp_<FAST>(T(0.5) * (nv2_h + hq1));
+                    const T s1 = nv2_u1a + u1a0 + u1b0 + nv2_u1b;
+                    const T a = u2a0;
+                    val2 = vdyfa_<FAST>(xs, xc, a, hmy) +
+                           vcorra_<FAST>(a, s1, (abs_(xse) + abs_(xe)) - (abs_(xsw) + abs_(xw)),
+                                         abs_(xse) + abs_(xe) + abs_(xsw) + abs_(xw) + ep, hmy);
+                    if (!gnd && !sky) {
+                        const T s3 = nv2_u3a + u3q0 + u3q1 + nv2_u3b;
+                        const T bs = XA(2, li, lj - 1);
+                        val2 = val2 + vcorra_<FAST>(a, s3,
+                                                    (abs_(ks) + abs_(xa_new)) - (abs_(bs) + abs_(bc)),
+                                                    abs_(ks) + abs_(xa_new) + abs_(bs) + abs_(bc) + ep,
+                                                    hmy);
+                    }
+                }
+                const T v1 = do_v1 ? val1 : T(0), v2 = do_v2 ? val2 : T(0);
+                LMID(sv1, 0, 0) = v1;
+                LMID(sv2, 0, 0) = v2;
+                if constexpr (NONOS) {
+                    w1 = donor(xw, xc, val1);
+                    w2 = donor(xs, xc, val2);
+                    w1 = do_v1 ? w1 : T(0);
+                    w2 = do_v2 ? w2 : T(0);
+                    LMID(sw2, 0, 0) = w2;
+                    T mx = xw, mn = xw;
+#define ACC(v, lo, hi) { T t_ = (v); lo = min2(lo, t_); hi = max2(hi, t_); }
+                    ACC(xc, mn, mx) ACC(xe, mn, mx) ACC(xs, mn, mx) ACC(xn, mn, mx)
+                    if (!gnd) ACC(bc, mn, mx)
+                    if (!sky) ACC(xa_new, mn, mx)
+#undef ACC
+                    mx = max2(mx, xmx0);
+                    mn = min2(mn, xmn0);
+                    up = (mx - xc) * hq1;
+                    dn = (xc - mn) * hq1;
+                }
+                if constexpr (TAPE) {
+                    if (P >= k0 && P <= k1) {
+                        if (own_fx) sto(pl(tp->v[0], FXY, P), tfo, v1);
+                        if (own_fy) sto(pl(tp->v[1], YXY, P), tso, v2);
+                    }
                 }
             }
-        }
+        };
+        if (BC_on && (pz || (P != 1 && P != lp))) stage_b(std::false_type{});
+        else stage_b(std::true_type{});
+        // h and rhr of the output plane K-2, for D: first of the loads, so
+        // that the wait for them leaves the others in flight (two planes of
+        // registers or LDS would keep them, and there are none)
+        const T hD = ldo(pl(h, SXY, kc(Q)), so), rD = ldo(pl(rhr, SXY, kc(Q)), so);
         // the oldest slot of each queue becomes the newest of step K+1
         {
             const int Kn = K + 1;
-            xq1 = ldo(pl(x, SXY, kc(Kn + 1)), so);
-            u1a0 = ldo(pl(u1, FXY, kc(Kn)), fo);
-            u1b0 = ld_u1b(kc(Kn));
-            u2a0 = ldo(pl(u2, YXY, kc(Kn)), so);
-            u2b0 = ld_u2b(kc(Kn));
-            u3q0 = ldo(pl(u3, SXY, fc(Kn + 1)), so);
-            hq1 = ldo(pl(h, SXY, kc(Kn)), so);
-            rq2 = ldo(pl(rhr, SXY, kc(Kn)), so);
+            if (PER && pz) {
+                qx = pl(x, SXY, kc(Kn + 1));
+                qu1 = pl(u1, FXY, kc(Kn)); qu2 = pl(u2, YXY, kc(Kn)); qu3 = pl(u3, SXY, fc(Kn + 1));
+                qh = pl(h, SXY, kc(Kn)); qr = pl(rhr, SXY, kc(Kn));
+            } else {
+                const bool more = Kn <= lp;
+                const uint32_t dS = more ? SB8 : 0, dF = more ? FB8 : 0, dY = more ? YB8 : 0;
+                qx = adv(qx, Kn < lp ? SB8 : 0);
+                qu1 = adv(qu1, dF); qu2 = adv(qu2, dY); qu3 = adv(qu3, dS);
+                qh = adv(qh, dS); qr = adv(qr, dS);
+            }
+            if (Kn + 1 <= Alast) ld_halo(Kn + 1);
+            xq1 = ldo(qx, so);
+            u1a0 = ldo(qu1, fo);
+            u1b0 = ld_u1b(qu1);
+            u2a0 = ldo(qu2, so);
+            u2b0 = ld_u2b(qu2);
+            u3q0 = ldo(qu3, so);
+            hq1 = ldo(qh, so);
+            rq2 = ldo(qr, so);
         }
         // donor flux of V1 through the right x-face of P: the left face of
         // the position to the right (the lane to the right, in the same row
         // wherever the limiter runs)
         const T w1p = NONOS ? from_right_lane(w1) : T(0);
         __syncthreads();
-        const bool D_on = do_d && Dq;
         // ---- C: cp, cn on plane P (antidiff3d-standard-gpubc.f90:260-347) --
+        T cpP, cnP, cpQ, cnQ;  // of the own column on planes P (formed here) and Q
         if constexpr (NONOS) {
             auto stage_c = [&](auto edge) __attribute__((always_inline)) {
                 constexpr bool EDGE = decltype(edge)::value;
                 const bool gnd = EDGE && !pz && P == 1, sky = EDGE && !pz && P == lp;
-                T rp = T(0), rn = T(0);
-                if (do_c) {
-                    const T xaP = XA(1, li, lj);
-                    T mx = XA(1, li - 1, lj), mn = mx;
-#define ACC(v, lo, hi) { T t_ = (v); lo = min2(lo, t_); hi = max2(hi, t_); }
-                    ACC(xaP, mn, mx) ACC(XA(1, li + 1, lj), mn, mx)
-                    ACC(XA(1, li, lj - 1), mn, mx) ACC(XA(1, li, lj + 1), mn, mx)
-                    if (!gnd) ACC(XA(2, li, lj), mn, mx)
-                    if (!sky) ACC(xa_new, mn, mx)
-#undef ACC
-                    mx = max2(mx, xmx0);
-                    mn = min2(mn, xmn0);
-                    const T a1p = w1p, a1 = w1;
-                    const T a2p = L.sw2[pj + 1][pi], a2 = w2;
-                    T a3p, a3;
-                    if (gnd) { a3p = w3n; a3 = -a3p; }
-                    else if (sky) { a3 = w3q2; a3p = -a3; }
-                    else { a3p = w3n; a3 = w3q2; }
-                    rp = div_<FAST>((mx - xaP) * hP,
-                                    pn(a1p) + pp(a1) + pn(a2p) + pp(a2) + pn(a3p) + pp(a3) + ep);
-                    rn = div_<FAST>((xaP - mn) * hP,
-                                    pp(a1p) + pn(a1) + pp(a2p) + pn(a2) + pp(a3p) + pn(a3) + ep);
+                const T a1p = w1p, a1 = w1;
+                const T a2p = LMID(sw2, 1, 0), a2 = LMID(sw2, 0, 0);
+                T a3p, a3;
+                if (gnd) { a3p = w3n; a3 = -a3p; }
+                else if (sky) { a3 = w3; a3p = -a3; }
+                else { a3p = w3n; a3 = w3; }
+                T rp = div_<FAST>(up,
+                                  pn(a1p) + pp(a1) + pn(a2p) + pp(a2) + pn(a3p) + pp(a3) + ep);
+                T rn = div_<FAST>(dn,
+                                  pp(a1p) + pn(a1) + pp(a2p) + pn(a2) + pp(a3p) + pn(a3) + ep);
+                if constexpr (!TAPE) {
+                    rp = min2(T(1), rp);
+                    rn = min2(T(1), rn);
                 }
-                L.scp[E1][pj][pi] = rp;
-                L.scn[E1][pj][pi] = rn;
+                cpQ = CP(li, lj);
+                cnQ = CN(li, lj);
+                CP(li, lj) = cpP = do_c ? rp : T(0);
+                CN(li, lj) = cnP = do_c ? rn : T(0);
             };
             if (BC_on) {
                 if (!pz && (P == 1 || P == lp)) stage_c(std::true_type{});
                 else stage_c(std::false_type{});
+            } else if constexpr (TAPE) {
+                cpQ = CP(li, lj);
+                cnQ = CN(li, lj);
             }
         }
-        // limited flux through face Q+1 of the own column (cp/cn of Q from
-        // the previous step, of Q+1 from this one)
-        auto flux_up = [&]() -> T {
-            T vl = v3q2;
+        // limited flux through face Q+1 of the own column; the first output
+        // plane's lower one is formed on the step before its own
+        T F3p = T(0);
+        if (BC_on && !(!pz && Q == lp)) {
+            T vl = v3;
             if constexpr (NONOS)
-                vl = slim(vl, min3(T(1), CP(1, li, lj), CN(2, li, lj)),
-                          min3(T(1), CP(2, li, lj), CN(1, li, lj)), XA(2, li, lj), XA(1, li, lj));
-            return donor(RC(2, li, lj), RC(1, li, lj), vl);
-        };
-        // the lower z-face flux of the first output plane of the range is
-        // the upper face of plane k0-1, formed on the step before
-        if (Q == k0 - 1 && (pz || Q >= 1) && do_d) f3c = flux_up();
+                vl = slim(vl, lmin(cpP, cnQ), lmin(cpQ, cnP), XA(2, li, lj), XA(1, li, lj));
+            F3p = donor(RC(2, li, lj), RC(1, li, lj), vl);
+        }
+        const T F3 = f3c;
+        f3c = F3p;
         // ---- D: the new x on plane Q (antidiff3d-standard-gpubc.f90:431-459)
-        if (D_on) {
+        if (Dq) {
             const bool gnd = !pz && Q == 1, sky = !pz && Q == lp;
-            const T F1 = L.sf1[pj][pi], F1p = L.sf1[pj][pi + 1];
-            const T F2 = L.sf2[pj][pi], F2p = L.sf2[pj + 1][pi];
+            const T F1 = LMID(sf1, 0, 0), F1p = LMID(sf1, 0, 1);
+            const T F2 = LMID(sf2, 0, 0), F2p = LMID(sf2, 1, 0);
             T sum = F1p - F1 + F2p - F2;
-            T F3p = T(0);
-            if (gnd) {
-                F3p = flux_up();
-                sum = sum + F3p + F3p;
-            } else if (sky) {
-                sum = sum - f3c - f3c;
-            } else {
-                F3p = flux_up();
-                sum = sum + F3p - f3c;
-            }
-            f3c = F3p;
-            if constexpr (TAPE) {
+            if (gnd) sum = sum + F3p + F3p;
+            else if (sky) sum = sum - F3 - F3;
+            else sum = sum + F3p - F3;
+            if constexpr (TAPE) if (do_d) {
                 // V3 on the lower face Q of the cell (face 1 = -face 2 on
                 // the ground), and on face lp+1 = -face lp on the sky plane;
                 // cp and cn of the cell
                 T* const tv = pl(tp->v[2], SXY, Q);
-                sto(tv, so, gnd ? -v3q2 : v3q1);
+                sto(tv, so, gnd ? -v3 : v3q1);
                 if (sky) sto(tv + SXY, so, -v3q1);
-                sto(pl(tp->cp, SXY, Q), so, CP(2, li, lj));
-                sto(pl(tp->cn, SXY, Q), so, CN(2, li, lj));
+                sto(pl(tp->cp, SXY, Q), so, cpQ);
+                sto(pl(tp->cn, SXY, Q), so, cnQ);
                 // x with the inflow values on the wall halo (the upwind's
                 // input) and with edge copies there (the limiter's bounds)
                 const T xc = ldo(pl(x, SXY, Q), so);
@@ -570,26 +636,16 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
                 if (gj == 1) { sto(tb - o.sx, so, bcy[(gi - 1) + np * (Q - 1)]); sto(t0 - o.sx, so, xc); }
                 if (gj == mp) { sto(tb + o.sx, so, bcy[(gi - 1) + np * ((Q - 1) + lp)]); sto(t0 + o.sx, so, xc); }
             }
-            const T hinv = rcp_<FAST>(hQ);
-            T* const xoq = pl(xo, SXY, Q);
-            sto(xoq, so, rQ * (RC(2, li, lj) - sum * hinv));
-            // x halo on open walls: edge copies of x at level n
-            const bool ew = !px && (gi == 1 || gi == np), ns = !py && (gj == 1 || gj == mp);
-            if (ew || ns) {
-                const T xe = ldo(pl(x, SXY, Q), so);
-                if (!px && gi == 1) sto(xoq - 1, so, xe);
-                if (!px && gi == np) sto(xoq + 1, so, xe);
-                if (!py && gj == 1) sto(xoq - o.sx, so, xe);
-                if (!py && gj == mp) sto(xoq + o.sx, so, xe);
-            }
+            const T hinv = rcp_<FAST>(hD);
+            xst = rD * (RC(2, li, lj) - sum * hinv);
         }
 #undef XA
-#undef AX
 #undef RC
 #undef CP
 #undef CN
-        v3q1 = v3n;
-        w3q1 = w3n;
+        if constexpr (TAPE) v3q1 = v3;
+        v3 = v3n;
+        w3 = w3n;
     };
     for (int K = Ks;;) {
         step(std::integral_constant<int, 0>{}, K);
@@ -605,6 +661,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         step(std::integral_constant<int, 5>{}, K);
         if (++K > Ke) break;
     }
+    if (do_d) sto(pl(xo, SXY, k1), so, xst);
 }
 
 template <typename T, int RX, int RY, int MINB, bool NONOS, bool PER, bool TAPE = false,
