@@ -833,6 +833,8 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     };
 #undef LMID
 #undef LHI
+#undef LSX
+#undef SB
     for (int K = Ks;;) {
         step(std::integral_constant<int, 0>{}, K);
         if (++K > Ke) break;

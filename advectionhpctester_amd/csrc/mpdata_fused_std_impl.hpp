@@ -22,12 +22,16 @@
 //      donor fluxes of the pseudo-velocities that the limiter bounds,
 //   C  the limiter ratios cp,cn on plane P,
 //   D  the new x on plane Q.
-// A position's own V1, V2 and V3 stay in registers (the flux through its
-// left, lower and bottom faces is formed by the position itself); the
-// limiter's donor flux through the right face comes from the lane to the
-// right, the one through the upper y-face through LDS.  The inputs of V1
-// from column i-1 come from the lane to the left, those of V2 from column
-// j-1 through LDS.
+// A position's own V1, V2 (in LDS slots of its own) and V3 are used by itself
+// for the flux through its left, lower and bottom faces; the limiter's donor
+// flux through the right face comes from the lane to the right, the one
+// through the upper y-face through LDS.  The inputs of V1 from column i-1
+// come from the lane to the left, those of V2 from column j-1 through LDS.
+//
+// What bounds it is the chain of a plane, as in the gauge kernel, with more of
+// it in the divisions (thirteen a cell); the same means took 384x320x192 from
+// 743 to 687 us (fast build), 190x147x83 in place from 149 to 118 us (exact)
+// and ten steps of a periodic 64x64x32 from 323 to 235 us.
 #pragma once
 
 #include "mpdata_fused_impl.hpp"
@@ -647,6 +651,11 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         v3 = v3n;
         w3 = w3n;
     };
+#undef LSX
+#undef LLO
+#undef LMID
+#undef LHI
+#undef SB
     for (int K = Ks;;) {
         step(std::integral_constant<int, 0>{}, K);
         if (++K > Ke) break;
@@ -700,25 +709,6 @@ hipError_t launch_std(const Geo& g, const Off& o, const Tiling& tl, const T* x, 
     return hipGetLastError();
 }
 
-// Tiling of the standard kernel: 32x16 tiles (the 32x32 build spills
-// registers and measured slower at every size), two workgroups to a CU or one
-// by the modelled time.  MPDATA_FUSED_CFG / _CHUNK override them for tests
-// and tuning.
-inline Tiling choose_std(const Geo& g) {
-    Tiling tl;
-    const int env_cfg = fused_config(), env_chunk = fused_chunk_env();
-    tl.cfg = env_cfg >= 0 ? env_cfg : 1;
-    if (env_chunk > 0) tl.chunk = env_chunk;
-    if (env_cfg >= 0 || env_chunk > 0) return tl;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        ncu < 1)
-        ncu = 256;
-    tl.per_cu = tiling_time<32, 16>(g, ncu, 1) < tiling_time<32, 16>(g, ncu, 2) ? 1 : 2;
-    return tl;
-}
-
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
 hipError_t launch_std_any(const Geo& g, const Off& o, const Tiling& tl, int nonos, const T* x, T* xout,
                           const T* u1, const T* u2, const T* u3, const T* rhr, const T* h,
@@ -732,13 +722,15 @@ hipError_t launch_std_any(const Geo& g, const Off& o, const Tiling& tl, int nono
     return launch_std<T, RX, RY, MINB, false, false, false, FAST>(g, o, tl, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
 }
 
-// One step of the standard variant on the build FAST selects.
+// One step of the standard variant on the build FAST selects, with the tiling
+// rule of the gauge kernel (384x320x192, fast build: 638 us with the 32x32
+// tiles it picks, 687 with 32x16; 64x64x32 takes 32x16, 23.5 against 30 us).
 template <typename T, bool FAST>
 hipError_t std_step(const Geo& g, int nonos, const T* x, T* xout, const T* u1, const T* u2,
                     const T* u3, const T* rhr, const T* h, const T* bcx, const T* bcy,
                     hipStream_t s) {
     const Off o = make_off(g);
-    const Tiling tl = choose_std(g);
+    const Tiling tl = choose_tiling<T>(g);
     return tl.cfg == 0
                ? launch_std_any<T, 32, 32, 4, FAST>(g, o, tl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s)
                : launch_std_any<T, 32, 16, 4, FAST>(g, o, tl, nonos, x, xout, u1, u2, u3, rhr, h, bcx, bcy, s);
