@@ -221,42 +221,36 @@ __global__ void __launch_bounds__(256)
 
 // velprd_traj0's extrapolation (module_velprd.f90:55-85) followed, per cell,
 // by the time-level rotation (velprd_driver.f90:254-270): level n-1 of ox is
-// read before the rotation overwrites it with ox(.,0)*h.  The twelve level
-// stores are non-temporal: nothing reads them back before they leave L2.
+// read before the rotation overwrites it with ox(.,0)*h.  Bound by HBM (25
+// array passes): a block takes a row of one of the six fields, so that it
+// streams five arrays rather than 25 (h is read again by the blocks of oy and
+// oz, from L2), and the level stores are non-temporal, since nothing reads
+// them back before they leave L2 (row_block has the figures).
 template <typename T>
 __global__ void __launch_bounds__(256)
     k_extrap_rotate(Geo g, T* __restrict__ ox, T* __restrict__ oy, T* __restrict__ oz,
                     T* __restrict__ u, T* __restrict__ v, T* __restrict__ w,
                     const T* __restrict__ h, T gc1, T gc2, T gc3, T r) {
-    CELL_LOOP_HEAD
+    const int q = blockIdx.x % 6;
+    const int i = 1 + blockIdx.x / 6 * blockDim.x + threadIdx.x;
+    const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
+    const int k = 1 + blockIdx.z;
+    if (i > g.np || j > g.mp) return;
     const long long n = len_of<SCAL>(g);
     const long long c = off_raw<SCAL>(g, i, j, k);
-    const T hh = h[c];
-    {
-        const T a0 = ox[c] * hh, a2 = ox[c + 2 * n];
+    if (q < 3) {
+        T* const o = q == 0 ? ox : q == 1 ? oy : oz;
+        const T gc = q == 0 ? gc1 : q == 1 ? gc2 : gc3;
+        const T a0 = o[c] * h[c], a2 = o[c + 2 * n];
         const T a1 = a0 + r * (a0 - a2);
-        __builtin_nontemporal_store(T(0.5) * (a1 + a0) * gc1, &ox[c + n]);
-        __builtin_nontemporal_store(ox[c] * hh, &ox[c + 2 * n]);
+        __builtin_nontemporal_store(T(0.5) * (a1 + a0) * gc, &o[c + n]);
+        __builtin_nontemporal_store(a0, &o[c + 2 * n]);
+    } else {
+        T* const a = q == 3 ? u : q == 4 ? v : w;
+        const T a0 = a[c];
+        __builtin_nontemporal_store(a0 + r * (a0 - a[c + 2 * n]), &a[c + n]);
+        __builtin_nontemporal_store(a0, &a[c + 2 * n]);
     }
-    {
-        const T a0 = oy[c] * hh, a2 = oy[c + 2 * n];
-        const T a1 = a0 + r * (a0 - a2);
-        __builtin_nontemporal_store(T(0.5) * (a1 + a0) * gc2, &oy[c + n]);
-        __builtin_nontemporal_store(oy[c] * hh, &oy[c + 2 * n]);
-    }
-    {
-        const T a0 = oz[c] * hh, a2 = oz[c + 2 * n];
-        const T a1 = a0 + r * (a0 - a2);
-        __builtin_nontemporal_store(T(0.5) * (a1 + a0) * gc3, &oz[c + n]);
-        __builtin_nontemporal_store(oz[c] * hh, &oz[c + 2 * n]);
-    }
-    const T u0 = u[c], v0 = v[c], w0 = w[c];
-    __builtin_nontemporal_store(u0 + r * (u0 - u[c + 2 * n]), &u[c + n]);
-    __builtin_nontemporal_store(v0 + r * (v0 - v[c + 2 * n]), &v[c + n]);
-    __builtin_nontemporal_store(w0 + r * (w0 - w[c + 2 * n]), &w[c + n]);
-    __builtin_nontemporal_store(u0, &u[c + 2 * n]);
-    __builtin_nontemporal_store(v0, &v[c + 2 * n]);
-    __builtin_nontemporal_store(w0, &w[c + 2 * n]);
 }
 
 dim3 cell_block() { return dim3(64, 4, 1); }
@@ -423,9 +417,8 @@ struct Driver {
     int traj0_rotate(T dtv, T* u, T* v, T* w) {
         const Geo& g = c->g;
         const long long n = len_of<SCAL>(g);
-        dim3 grid((g.np + 63) / 64, (g.mp + 3) / 4, g.lp);
-        k_extrap_rotate<T><<<grid, dim3(64, 4, 1), 0, s>>>(g, ox, oy, oz, u, v, w, h, dtv * dxi,
-                                                           dtv * dyi, dtv * dzi, dt_ratio);
+        k_extrap_rotate<T><<<row_grid(g, 6), row_block(g.np, g.mp), 0, s>>>(
+            g, ox, oy, oz, u, v, w, h, dtv * dxi, dtv * dyi, dtv * dzi, dt_ratio);
         HIPCHK(hipGetLastError());
         HIPCHK(Stages<T>::a_to_c(g, ox + n, oy + n, oz + n, u1, u2, u3, s));
         rotated = true;

@@ -507,21 +507,19 @@ __global__ void k_extrap_halo(Geo g, T* __restrict__ a, int dir) {
 }
 
 // A->C averaging u1(i)=0.5*(ox(i)+ox(i-1)) on faces 1..n+1 (open) or 1..n
-// (periodic); launched over cells plus one extra layer.
+// (periodic): one thread per cell, that of the last cell of a direction also
+// forms its wall face, so that the blocks are whole rows (row_block).
 template <typename T>
 __global__ void k_a_to_c(Geo g, const T* __restrict__ ox, const T* __restrict__ oy,
                          const T* __restrict__ oz, T* __restrict__ u1, T* __restrict__ u2,
                          T* __restrict__ u3) {
-    const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
-    const int k = 1 + blockIdx.z;
-    const bool in_i = i <= g.np, in_j = j <= g.mp, in_k = k <= g.lp;
-    if (in_j && in_k && i <= g.np + (g.px ? 0 : 1))
-        X_(u1, i, j, k) = T(0.5) * (S_(ox, i, j, k) + S_(ox, i - 1, j, k));
-    if (in_i && in_k && j <= g.mp + (g.py ? 0 : 1))
-        Y_(u2, i, j, k) = T(0.5) * (S_(oy, i, j, k) + S_(oy, i, j - 1, k));
-    if (in_i && in_j && k <= g.lp + (g.pz ? 0 : 1))
-        Z_(u3, i, j, k) = T(0.5) * (S_(oz, i, j, k) + S_(oz, i, j, k - 1));
+    CELL_LOOP_HEAD
+    for (int q = i; q <= (i == g.np && !g.px ? i + 1 : i); q++)
+        X_(u1, q, j, k) = T(0.5) * (S_(ox, q, j, k) + S_(ox, q - 1, j, k));
+    for (int q = j; q <= (j == g.mp && !g.py ? j + 1 : j); q++)
+        Y_(u2, i, q, k) = T(0.5) * (S_(oy, i, q, k) + S_(oy, i, q - 1, k));
+    for (int q = k; q <= (k == g.lp && !g.pz ? k + 1 : k); q++)
+        Z_(u3, i, j, q) = T(0.5) * (S_(oz, i, j, q) + S_(oz, i, j, q - 1));
 }
 
 // The predictor in one pass (open walls): velprd_traj0's extrapolation of the
@@ -533,8 +531,6 @@ __global__ void k_a_to_c(Geo g, const T* __restrict__ ox, const T* __restrict__ 
 // so the caller rotates the time levels by swapping pointers; the products,
 // sums and their order are those of k_velprd_extrap, k_extrap_halo and
 // k_a_to_c, so u1..u3 are bit-identical to them as long as h is the same.
-// One thread per (i, j, k) of the face ranges; the level-n+1/2 values of the
-// neighbouring cells are recomputed from their inputs (cache hits).
 template <typename T>
 __device__ __forceinline__ T half_level(const T* __restrict__ a, const T* __restrict__ ap,
                                         const T* __restrict__ h, long long c, T gc, T r) {
@@ -544,20 +540,18 @@ __device__ __forceinline__ T half_level(const T* __restrict__ a, const T* __rest
     return T(0.5) * (a1 + a0) * gc;
 }
 
-// One thread per (i, j, k) of the face ranges; the level-n+1/2 values of the
-// neighbouring cells are recomputed from their inputs (cache hits).  (A
-// k-march with the z neighbour carried in registers measured slower: 226
-// against 188 us at 256x256x128 in FP64, its serial plane loop exposing the
-// load latency.)
+// One thread per cell, that of the last cell of a direction also forming its
+// wall face; the level-n+1/2 values of the neighbouring cells are recomputed
+// from their inputs (cache hits).  (A k-march with the z neighbour carried in
+// registers measured slower: 226 against 188 us at 256x256x128 in FP64, its
+// serial plane loop exposing the load latency.)
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_predict_ac(Geo g, const T* __restrict__ ox, const T* __restrict__ oy, const T* __restrict__ oz,
              const T* __restrict__ oxp, const T* __restrict__ oyp, const T* __restrict__ ozp,
              const T* __restrict__ h, T gc1, T gc2, T gc3, T r, T* __restrict__ u1,
              T* __restrict__ u2, T* __restrict__ u3) {
-    const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
-    const int k = 1 + blockIdx.z;
+    CELL_LOOP_HEAD
     const int np = g.np, mp = g.mp, lp = g.lp;
     auto cell = [&](int ii, int jj, int kk) { return off_raw<SCAL>(g, ii, jj, kk); };
     // level n+1/2 at cells m (upstream) and c (downstream) of a face at
@@ -580,15 +574,15 @@ k_predict_ac(Geo g, const T* __restrict__ ox, const T* __restrict__ oy, const T*
         }
         return T(0.5) * (lc + lm);
     };
-    if (i <= np + 1 && j <= mp && k <= lp)
-        u1[off_raw<FACEX>(g, i, j, k)] =
-            face(ox, oxp, gc1, i, np, [&](int q) { return cell(q, j, k); });
-    if (i <= np && j <= mp + 1 && k <= lp)
-        u2[off_raw<FACEY>(g, i, j, k)] =
-            face(oy, oyp, gc2, j, mp, [&](int q) { return cell(i, q, k); });
-    if (i <= np && j <= mp && k <= lp + 1)
-        u3[off_raw<FACEZ>(g, i, j, k)] =
-            face(oz, ozp, gc3, k, lp, [&](int q) { return cell(i, j, q); });
+    for (int q = i; q <= (i == np ? i + 1 : i); q++)
+        u1[off_raw<FACEX>(g, q, j, k)] =
+            face(ox, oxp, gc1, q, np, [&](int a) { return cell(a, j, k); });
+    for (int q = j; q <= (j == mp ? j + 1 : j); q++)
+        u2[off_raw<FACEY>(g, i, q, k)] =
+            face(oy, oyp, gc2, q, mp, [&](int a) { return cell(i, a, k); });
+    for (int q = k; q <= (k == lp ? k + 1 : k); q++)
+        u3[off_raw<FACEZ>(g, i, j, q)] =
+            face(oz, ozp, gc3, q, lp, [&](int a) { return cell(i, j, a); });
 }
 
 // Time-level rotation: velprd_driver.f90:254-270
@@ -851,7 +845,7 @@ hipError_t Stages<T>::a_to_c(const Geo& g, T* ox, T* oy, T* oz, T* u1, T* u2, T*
         dim3 grid((g.np + 63) / 64, (g.mp + 3) / 4, 2);
         k_extrap_halo<T><<<grid, wall_block(), 0, s>>>(g, oz, 2);
     }
-    k_a_to_c<T><<<cell_grid(g, 1), cell_block(), 0, s>>>(g, ox, oy, oz, u1, u2, u3);
+    k_a_to_c<T><<<row_grid(g), row_block(g.np, g.mp), 0, s>>>(g, ox, oy, oz, u1, u2, u3);
     return hipGetLastError();
 }
 
@@ -859,7 +853,7 @@ template <typename T>
 hipError_t Stages<T>::predict_ac(const Geo& g, const T* ox, const T* oy, const T* oz,
                                  const T* oxp, const T* oyp, const T* ozp, const T* h, T gc1,
                                  T gc2, T gc3, T dt_ratio, T* u1, T* u2, T* u3, hipStream_t s) {
-    k_predict_ac<T><<<cell_grid(g, 1), cell_block(), 0, s>>>(g, ox, oy, oz, oxp, oyp, ozp, h, gc1,
+    k_predict_ac<T><<<row_grid(g), row_block(g.np, g.mp), 0, s>>>(g, ox, oy, oz, oxp, oyp, ozp, h, gc1,
                                                              gc2, gc3, dt_ratio, u1, u2, u3);
     return hipGetLastError();
 }
