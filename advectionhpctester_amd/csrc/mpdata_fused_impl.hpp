@@ -435,6 +435,35 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     T* qxo = uniform(pl(xo, SXY, Ks - 4));  // plane K-3 during step K
     T xst = T(0);                           // the new x of that plane
     const bool edge_d = do_d && (gi == 1 || gi == np || gj == 1 || gj == mp);
+    // TAPE: what the last steps left for the tape, stored with it (as the new
+    // x): V1, V2 of plane K-2; V3, cp and cn of plane K-3; x of plane K with
+    // the inflow values on the wall halo (the upwind's input) and with edge
+    // copies there (the limiter's bounds)
+    T tv1 = T(0), tv2 = T(0), tv3 = T(0), tcp = T(0), tcn = T(0), tx = T(0);
+    auto store_tape = [&](int K) __attribute__((always_inline)) {
+        if (K - 2 >= k0 && K - 2 <= k1) {
+            if (own_fx) sto(pl(tp->v[0], FXY, K - 2), tfo, tv1);
+            if (own_fy) sto(pl(tp->v[1], YXY, K - 2), tso, tv2);
+        }
+        if (do_d && K - 3 >= k0 && K - 3 <= k1) {
+            const int Q = K - 3;
+            T* const tv = pl(tp->v[2], SXY, Q);
+            sto(tv, so, tv3);
+            if (Q == lp) sto(tv + SXY, so, -tv3);
+            sto(pl(tp->cp, SXY, Q), so, tcp);
+            sto(pl(tp->cn, SXY, Q), so, tcn);
+        }
+        if (do_d && K >= k0 && K <= k1) {
+            T* const tb = pl(tp->xb, SXY, K);
+            T* const t0 = pl(tp->x0, SXY, K);
+            sto(tb, so, tx);
+            sto(t0, so, tx);
+            if (gi == 1) { sto(tb - 1, so, bcx[(gj - 1) + mp * (K - 1)]); sto(t0 - 1, so, tx); }
+            if (gi == np) { sto(tb + 1, so, bcx[(gj - 1) + mp * ((K - 1) + lp)]); sto(t0 + 1, so, tx); }
+            if (gj == 1) { sto(tb - o.sx, so, bcy[(gi - 1) + np * (K - 1)]); sto(t0 - o.sx, so, tx); }
+            if (gj == mp) { sto(tb + o.sx, so, bcy[(gi - 1) + np * ((K - 1) + lp)]); sto(t0 + o.sx, so, tx); }
+        }
+    };
     auto step = [&](auto phase, int K) __attribute__((always_inline)) {
         constexpr int PH = decltype(phase)::value;
         // K opaque: every plane-dependent quantity is formed within the
@@ -470,6 +499,10 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         // n around plane K
         qxo = adv(qxo, SB8);
         if (do_d && K - 3 >= k0 && K - 3 <= k1) sto(qxo, so, xst);
+        if constexpr (TAPE) {
+            tx = xq2;
+            store_tape(K);
+        }
         if (edge_d && K >= k0 && K <= k1) {
             T* const xok = pl(xo, SXY, K);
             if (gi == 1) sto(xok - 1, so, xq2);
@@ -547,6 +580,8 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             else xa_new = rq2 * (xc - (f1p - f1 + f2p - f2 + f3p - f3) * hinv);
             }
             sxa[R0][pj][pi] = xa_new;
+            if constexpr (TAPE)
+                if (own_s && K >= k0 && K <= k1) sto(pl(tp->psi, SXY, K), tso, xa_new);
             // FAST: r*(xant/r - s/h) = xant - (r/h)*s, to rounding
             if constexpr (!DENS) LHI(rr, R0 * RY * RX) = FAST ? rq2 * hinv : rq2;
             // bounds of x for the limiter on plane K: the 7-point stencil,
@@ -634,12 +669,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                 val2 = do_v2 ? val2 : T(0);
                 sv1[pj][pi] = val1;
                 LMID(sv2, 0, 0, 0) = val2;
-                if constexpr (TAPE) {
-                    if (P >= k0 && P <= k1) {
-                        if (own_fx) sto(pl(tp->v[0], FXY, P), tfo, val1);
-                        if (own_fy) sto(pl(tp->v[1], YXY, P), tso, val2);
-                    }
-                }
+                if constexpr (TAPE) tv1 = val1, tv2 = val2;
                 T mx = xw, mn = xw;
 #define ACC(v, lo, hi) { T t_ = (v); lo = min2(lo, t_); hi = max2(hi, t_); }
                 ACC(xc, mn, mx) ACC(xe, mn, mx) ACC(xs, mn, mx) ACC(xn, mn, mx)
@@ -654,8 +684,6 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         };
         if (BC_on && P != 1 && P != lp) stage_b(std::false_type{});
         else stage_b(std::true_type{});
-        if constexpr (TAPE)
-            if (Dq && own_s) sto(pl(tp->psi, SXY, Q), tso, XA(2, li, lj));
         T hP;
         // The loaded source-column queues are not read after this point:
         // the oldest slot of each is loaded with the plane step K+1 needs;
@@ -767,26 +795,12 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                     if (gj == mp) sto(q2 + o.yx, so, F2p);
                     if (sky) sto(pl(pio->ul3, SXY, Q + 1), so, F3p);
                 }
-                if constexpr (TAPE) if (do_d) {
-                    // V3 on the lower face Q of the cell (face 1 = -face 2 on
-                    // the ground), and on face lp+1 = -face lp on the sky
-                    // plane; cp and cn of the cell; x with the inflow values
-                    // on the wall halo (the upwind's input) and with edge
-                    // copies there (the limiter's bounds)
-                    T* const tv = pl(tp->v[2], SXY, Q);
-                    sto(tv, so, gnd ? -v3q2 : v3q1);
-                    if (sky) sto(tv + SXY, so, -v3q1);
-                    sto(pl(tp->cp, SXY, Q), so, cpQ);
-                    sto(pl(tp->cn, SXY, Q), so, cnQ);
-                    const T xc = ldo(pl(x, SXY, Q), so);
-                    T* const tb = pl(tp->xb, SXY, Q);
-                    T* const t0 = pl(tp->x0, SXY, Q);
-                    sto(tb, so, xc);
-                    sto(t0, so, xc);
-                    if (gi == 1) { sto(tb - 1, so, bcx[(gj - 1) + mp * (Q - 1)]); sto(t0 - 1, so, xc); }
-                    if (gi == np) { sto(tb + 1, so, bcx[(gj - 1) + mp * ((Q - 1) + lp)]); sto(t0 + 1, so, xc); }
-                    if (gj == 1) { sto(tb - o.sx, so, bcy[(gi - 1) + np * (Q - 1)]); sto(t0 - o.sx, so, xc); }
-                    if (gj == mp) { sto(tb + o.sx, so, bcy[(gi - 1) + np * ((Q - 1) + lp)]); sto(t0 + o.sx, so, xc); }
+                if constexpr (TAPE) {
+                    // V3 on the lower face Q of the cell (face 1 = -face 2 on the ground)
+                    // and, above the sky plane, on face lp+1 = -face lp
+                    tv3 = gnd ? -v3q2 : v3q1;
+                    tcp = cpQ;
+                    tcn = cnQ;
                 }
             }
             if constexpr (DENS) if (do_d) {
@@ -850,6 +864,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         if (++K > Ke) break;
     }
     if (do_d) sto(pl(xo, SXY, k1), so, xst);
+    if constexpr (TAPE) store_tape(k1 + 3);
 }
 
 // Work of a persistent launch: which (tile, k-range) items each workgroup

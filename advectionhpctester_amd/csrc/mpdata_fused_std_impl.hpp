@@ -314,6 +314,35 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
     T* qxo = uniform(pl(xo, SXY, Ks - 4));  // plane K-3 during step K
     T xst = T(0);                           // the new x of that plane
     const bool edge_d = do_d && ((!px && (gi == 1 || gi == np)) || (!py && (gj == 1 || gj == mp)));
+    // TAPE: what the last steps left for the tape, stored with it (as the new
+    // x): V1, V2 of plane K-2; V3, cp and cn of plane K-3; x of plane K with
+    // the inflow values on the wall halo (the upwind's input) and with edge
+    // copies there (the limiter's bounds)
+    T tv1 = T(0), tv2 = T(0), tv3 = T(0), tcp = T(0), tcn = T(0), tx = T(0);
+    auto store_tape = [&](int K) __attribute__((always_inline)) {
+        if (K - 2 >= k0 && K - 2 <= k1) {
+            if (own_fx) sto(pl(tp->v[0], FXY, K - 2), tfo, tv1);
+            if (own_fy) sto(pl(tp->v[1], YXY, K - 2), tso, tv2);
+        }
+        if (do_d && K - 3 >= k0 && K - 3 <= k1) {
+            const int Q = K - 3;
+            T* const tv = pl(tp->v[2], SXY, Q);
+            sto(tv, so, tv3);
+            if (Q == lp) sto(tv + SXY, so, -tv3);
+            sto(pl(tp->cp, SXY, Q), so, tcp);
+            sto(pl(tp->cn, SXY, Q), so, tcn);
+        }
+        if (do_d && K >= k0 && K <= k1) {
+            T* const tb = pl(tp->xb, SXY, K);
+            T* const t0 = pl(tp->x0, SXY, K);
+            sto(tb, so, tx);
+            sto(t0, so, tx);
+            if (gi == 1) { sto(tb - 1, so, bcx[(gj - 1) + mp * (K - 1)]); sto(t0 - 1, so, tx); }
+            if (gi == np) { sto(tb + 1, so, bcx[(gj - 1) + mp * ((K - 1) + lp)]); sto(t0 + 1, so, tx); }
+            if (gj == 1) { sto(tb - o.sx, so, bcy[(gi - 1) + np * (K - 1)]); sto(t0 - o.sx, so, tx); }
+            if (gj == mp) { sto(tb + o.sx, so, bcy[(gi - 1) + np * ((K - 1) + lp)]); sto(t0 + o.sx, so, tx); }
+        }
+    };
     auto step = [&](auto phase, int K) __attribute__((always_inline)) {
         constexpr int PH = decltype(phase)::value;
         asm volatile("" : "+s"(K));
@@ -334,6 +363,10 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
         qxo = adv(qxo, SB8);
         if (do_d && K - 3 >= k0 && K - 3 <= k1) sto(qxo, so, xst);
+        if constexpr (TAPE) {
+            tx = xq2;
+            store_tape(K);
+        }
         if (edge_d && K >= k0 && K <= k1) {
             T* const xok = pl(xo, SXY, K);
             if (!px && gi == 1) sto(xok - 1, so, xq2);
@@ -387,6 +420,8 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
             }
             xa_new = rq2 * (xc - (f1p - f1 + f2p - f2 + f3p - f3) * hinv);
             LLO(sxa, R0, 0, 0) = xa_new;
+            if constexpr (TAPE)
+                if (own_s && K >= k0 && K <= k1) sto(pl(tp->psi, SXY, K), tso, xa_new);
             LLO(src, R0, 0, 0) = div_<FAST>(xa_new, rq2);
             if constexpr (NONOS) {
                 T m = xc, n = xc;
@@ -431,8 +466,6 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
             LMID(sf1, 0, 0) = wall1 ? T(0) : F1;
             LMID(sf2, 0, 0) = wall2 ? T(0) : F2;
         }
-        if constexpr (TAPE)
-            if (Dq && own_s) sto(pl(tp->psi, SXY, Q), tso, XA(2, li, lj));
         // ---- B: V3 on face K, V1/V2 on plane P (antidiff3d-standard-
         //      gpubc.f90:72-202), their donor fluxes for the limiter -------
         // Straight-line on the interior planes (see the gauge kernel).
@@ -523,12 +556,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
                     up = (mx - xc) * hq1;
                     dn = (xc - mn) * hq1;
                 }
-                if constexpr (TAPE) {
-                    if (P >= k0 && P <= k1) {
-                        if (own_fx) sto(pl(tp->v[0], FXY, P), tfo, v1);
-                        if (own_fy) sto(pl(tp->v[1], YXY, P), tso, v2);
-                    }
-                }
+                if constexpr (TAPE) tv1 = v1, tv2 = v2;
             }
         };
         if (BC_on && (pz || (P != 1 && P != lp))) stage_b(std::false_type{});
@@ -619,26 +647,12 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
             if (gnd) sum = sum + F3p + F3p;
             else if (sky) sum = sum - F3 - F3;
             else sum = sum + F3p - F3;
-            if constexpr (TAPE) if (do_d) {
-                // V3 on the lower face Q of the cell (face 1 = -face 2 on
-                // the ground), and on face lp+1 = -face lp on the sky plane;
-                // cp and cn of the cell
-                T* const tv = pl(tp->v[2], SXY, Q);
-                sto(tv, so, gnd ? -v3 : v3q1);
-                if (sky) sto(tv + SXY, so, -v3q1);
-                sto(pl(tp->cp, SXY, Q), so, cpQ);
-                sto(pl(tp->cn, SXY, Q), so, cnQ);
-                // x with the inflow values on the wall halo (the upwind's
-                // input) and with edge copies there (the limiter's bounds)
-                const T xc = ldo(pl(x, SXY, Q), so);
-                T* const tb = pl(tp->xb, SXY, Q);
-                T* const t0 = pl(tp->x0, SXY, Q);
-                sto(tb, so, xc);
-                sto(t0, so, xc);
-                if (gi == 1) { sto(tb - 1, so, bcx[(gj - 1) + mp * (Q - 1)]); sto(t0 - 1, so, xc); }
-                if (gi == np) { sto(tb + 1, so, bcx[(gj - 1) + mp * ((Q - 1) + lp)]); sto(t0 + 1, so, xc); }
-                if (gj == 1) { sto(tb - o.sx, so, bcy[(gi - 1) + np * (Q - 1)]); sto(t0 - o.sx, so, xc); }
-                if (gj == mp) { sto(tb + o.sx, so, bcy[(gi - 1) + np * ((Q - 1) + lp)]); sto(t0 + o.sx, so, xc); }
+            if constexpr (TAPE) {
+                // V3 on the lower face Q of the cell (face 1 = -face 2 on the ground)
+                // and, above the sky plane, on face lp+1 = -face lp
+                tv3 = gnd ? -v3 : v3q1;
+                tcp = cpQ;
+                tcn = cnQ;
             }
             const T hinv = rcp_<FAST>(hD);
             xst = rD * (RC(2, li, lj) - sum * hinv);
@@ -671,6 +685,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         if (++K > Ke) break;
     }
     if (do_d) sto(pl(xo, SXY, k1), so, xst);
+    if constexpr (TAPE) store_tape(k1 + 3);
 }
 
 template <typename T, int RX, int RY, int MINB, bool NONOS, bool PER, bool TAPE = false,
