@@ -376,9 +376,9 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     constexpr int SZ = (int)sizeof(T), PLN = RY * RX * SZ;  // one plane of a tile array
     constexpr int MID = (int)offsetof(LT, sv2);
     constexpr int HI = (int)offsetof(LT, e_h) - RX * SZ;  // e arrays are read one row back
-    uint32_t lmid = uint32_t(MID + t * SZ), lhi = uint32_t(HI + t * SZ);
+    uint32_t lmid = uint32_t(MID + t * SZ);
     uint32_t lsx = uint32_t(offsetof(LT, sx) + ((saj - 1) * SW + (sai - 1)) * SZ);
-    asm volatile("" : "+v"(lmid), "+v"(lhi), "+v"(lsx));
+    asm volatile("" : "+v"(lmid), "+v"(lsx));
     char* const lds0 = reinterpret_cast<char*>(&L);
     // array `arr` at ring slot s, offset (db rows, da columns) from the lane
 #define LMID(arr, s, db, da) \
@@ -387,6 +387,11 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
 // of the source column; for a position in the domain its own
 #define LSX(s, db, da) \
     (*reinterpret_cast<T*>(lds0 + lsx + ((s) * (SW * SH) + (db) * SW + (da)) * SZ))
+// the second offset, formed anew where a stage uses it (one add instead of a
+// register through the loop)
+#define LHI_BASE                           \
+    uint32_t lhi = lmid + (HI - MID);      \
+    asm volatile("" : "+v"(lhi));
 #define LHI(arr, r) (*reinterpret_cast<T*>(lds0 + lhi + ((int)offsetof(LT, arr) - HI + (r) * SZ)))
 
     auto dif4 = [](T z0, T z1, T z2, T z3) { return (z3 + z2) - (z1 + z0); };
@@ -515,6 +520,14 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             sx[E1][pj + 1][pi + 1] = in_dom ? xq3 : xown;
             if (t < NRING) sx[E1][rsj][rsi] = xr;
         }
+        auto load_xr = [&](int K) __attribute__((always_inline)) {
+            qx = adv(qx, K + 1 < lp ? SB8 : 0);
+            if constexpr (!DENS) qr = adv(qr, K < lp ? SB8 : 0);
+            if constexpr (PASS == 2) qxa = adv(qxa, K < lp ? SB8 : 0);
+            xq1 = ldo(qx, so);
+            if constexpr (!DENS) rq2 = ldo(qr, so);
+            if constexpr (PASS == 2) xaq = ldo(qxa, so);
+        };
         // Temporaries of a step that are read only under the condition
         // that sets them are left unset rather than zeroed: a default value
         // would cost a register move per step on every path.
@@ -537,6 +550,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         const T s2x = from_left_lane(u2a0 + u2b0) + u2b0 + u2a0;
         const T s3x = from_left_lane(u3q0 + u3q1) + u3q1 + u3q0;
         if (BC_on) {
+            LHI_BASE
             LHI(e_h, 0) = hq1;  // element e = t
             if (!wall_e) LHI(e_u1, 0) = u1a0;
             if (last_e) LHI(e_u1, 1) = u1b0;
@@ -583,7 +597,10 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             if constexpr (TAPE)
                 if (own_s && K >= k0 && K <= k1) sto(pl(tp->psi, SXY, K), tso, xa_new);
             // FAST: r*(xant/r - s/h) = xant - (r/h)*s, to rounding
-            if constexpr (!DENS) LHI(rr, R0 * RY * RX) = FAST ? rq2 * hinv : rq2;
+            if constexpr (!DENS) {
+                LHI_BASE
+                LHI(rr, R0 * RY * RX) = FAST ? rq2 * hinv : rq2;
+            }
             // bounds of x for the limiter on plane K: the 7-point stencil,
             // where out-of-domain neighbours are edge copies of the centre
             // (cp_last_to_halo_xy) and leave max/min unchanged
@@ -601,6 +618,12 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             if (K == 1 || K == lp) stage_a(std::true_type{});
             else stage_a(std::false_type{});
         }
+        // the ring of plane K+2, x of it and r of plane K+1: their registers are
+        // free already, and the loads have a stage more to arrive in (fast
+        // build, 512x512x256: 1.35 -> 1.27 ms; the exactly rounded build spills
+        // with x and r here and loses 2 % on small domains)
+        if (K + 2 <= Alast) ld_halo(K + 2);
+        if constexpr (FAST) load_xr(K);
         __syncthreads();
 // xant of plane K-d at tile position (a, b)
 #define XA(d, a, b) sxa[(d) == 0 ? R0 : ((d) == 1 ? R1 : R2)][(b) + 2][(a) + 2]
@@ -654,6 +677,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
                 SB
                 {
                     // column (gi, gj-1): element e = t - RX
+                    LHI_BASE
                     const T nv2_h = LHI(e_h, -RX), nv2_u1a = LHI(e_u1, -RX),
                             nv2_u1b = LHI(e_u1, -RX + 1), nv2_u3a = LHI(e_u3a, -RX),
                             nv2_u3b = LHI(e_u3b, -RX);
@@ -695,12 +719,8 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             // the scalar instructions)
             const int Kn = K + 1;
             const uint32_t dS = Kn <= lp ? SB8 : 0, dF = Kn <= lp ? FB8 : 0, dY = Kn <= lp ? YB8 : 0;
-            qx = adv(qx, Kn < lp ? SB8 : 0);
+            if constexpr (!FAST) load_xr(K);
             qu1 = adv(qu1, dF); qu2 = adv(qu2, dY); qu3 = adv(qu3, dS); qh = adv(qh, dS);
-            if constexpr (!DENS) qr = adv(qr, dS);
-            if constexpr (PASS == 2) qxa = adv(qxa, dS);
-            if (Kn + 1 <= Alast) ld_halo(Kn + 1);
-            xq1 = ldo(qx, so);
             u1a0 = ldo(qu1, fo);
             u1b0 = ldo(qu1 + 1, fo);
             u2a0 = ldo(qu2, so);
@@ -708,8 +728,6 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             u3q0 = ldo(qu3, so);
             if constexpr (!FAST || DENS) hP = hq1;
             hq1 = ldo(qh, so);
-            if constexpr (!DENS) rq2 = ldo(qr, so);
-            if constexpr (PASS == 2) xaq = ldo(qxa, so);
         }
         __syncthreads();
         // ---- C: cp, cn on plane P ------------------------------------------
@@ -760,6 +778,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         if (sky) F3p = T(0) - f3c;
         if (gnd) F3 = T(0) - F3p;
         f3c = F3p;
+        LHI_BASE
         if (Dq) {
             const T F1 = LMID(sf1, 0, 0, 0), F1p = LMID(sf1, 0, 0, 1);
             const T F2 = LMID(sf2, 0, 0, 0), F2p = LMID(sf2, 0, 1, 0);
@@ -847,6 +866,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     };
 #undef LMID
 #undef LHI
+#undef LHI_BASE
 #undef LSX
 #undef SB
     for (int K = Ks;;) {
@@ -933,7 +953,7 @@ constexpr double kAlone = 0.12;
 // The plan for `slots` resident workgroups (chunk > 0: runs of that length),
 // with the group of least modelled time: the planes the busiest workgroup
 // marches, dearer the fewer neighbours share their halo columns in L2.
-constexpr int kLead = 5;
+constexpr int kLead = 4;
 // Planes the busiest workgroup of a plan marches.
 inline long long march_cost(const Geo& g, const March& m) {
     const long long cut = m.ntile > m.nwg * m.nfull ? m.run + m.lead : 0;

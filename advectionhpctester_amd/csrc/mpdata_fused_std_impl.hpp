@@ -284,8 +284,16 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
     constexpr int MID = (int)offsetof(LT, sf1);
     constexpr int HI = (int)offsetof(LT, e_h) - RX * SZ;  // read one row back
     uint32_t lsx = uint32_t(offsetof(LT, sx) + ((saj - 1) * SW + (sai - 1)) * SZ);
-    uint32_t llo = uint32_t(t * SZ), lmid = uint32_t(MID + t * SZ), lhi = uint32_t(HI + t * SZ);
-    asm volatile("" : "+v"(lsx), "+v"(llo), "+v"(lmid), "+v"(lhi));
+    uint32_t llo = uint32_t(t * SZ);
+    asm volatile("" : "+v"(lsx), "+v"(llo));
+// the other two, formed anew where a stage uses them (an add instead of a
+// register through the loop)
+#define LMID_BASE                   \
+    uint32_t lmid = llo + MID;      \
+    asm volatile("" : "+v"(lmid));
+#define LHI_BASE                    \
+    uint32_t lhi = llo + HI;        \
+    asm volatile("" : "+v"(lhi));
     char* const lds0 = reinterpret_cast<char*>(&L);
 #define LSX(s, db, da) \
     (*reinterpret_cast<T*>(lds0 + lsx + ((s) * (SW * SH) + (db) * SW + (da)) * SZ))
@@ -376,7 +384,17 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         }
         if (K + 1 <= Alast) {
             sx[E1][pj + 1][pi + 1] = valid ? xq3 : xown;
-            if (t < NRING) sx[E1][rsj][rsi] = xr;
+            if (t < NRING) {
+                // the slot's address formed anew (kept, it was spilled)
+                uint32_t q = llo;
+                asm volatile("" : "+v"(q));
+                q /= (uint32_t)SZ;
+                const uint32_t r = q - 2 * SW;
+                const uint32_t c = q < SW ? q
+                                   : q < 2 * SW ? q + (SH - 2) * SW
+                                                : (1 + r / 2) * SW + ((r & 1) ? SW - 1 : 0);
+                *reinterpret_cast<T*>(lds0 + ((int)offsetof(LT, sx) + E1 * (SW * SH) * SZ) + c * SZ) = xr;
+            }
         }
         // V1's inputs from column i-1: the source column of the lane to the
         // left wherever V1 is formed (gi >= 2, or a periodic x)
@@ -388,6 +406,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         // the source column's inputs of V2 at the position above (its
         // column j-1)
         if (BC_on) {
+            LHI_BASE
             LHI(e_h, 0) = hq1;
             if (!wall_e) LHI(e_u1, 0) = u1a0;
             if (last_e) LHI(e_u1, 1) = u1b0;
@@ -439,6 +458,9 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
             if (!pz && (K == 1 || K == lp)) stage_a(std::true_type{});
             else stage_a(std::false_type{});
         }
+        // the ring of plane K+2, whose registers are free already
+        if constexpr (!PER)
+            if (K + 2 <= Alast) ld_halo(K + 2);
         __syncthreads();
 // xant, xant/rhr of plane K-d at tile position (a, b)
 #define XA(d, a, b) LLO(sxa, (d) == 0 ? R0 : ((d) == 1 ? R1 : R2), (b) - lj, (a) - li)
@@ -453,6 +475,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         //      V of Q from the previous step, cp/cn of Q and Q-1; formed
         //      before B so that V of Q is dead before V of P is formed ------
         if (Dq) {
+            LMID_BASE
             T vl = LMID(sv1, 0, 0), vb = LMID(sv2, 0, 0);
             if constexpr (NONOS) {
                 const T c0 = CP(li, lj), n0 = CN(li, lj);
@@ -518,6 +541,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
                 SB
                 {
                     // column j-1: the source column of the position below
+                    LHI_BASE
                     const T nv2_h = LHI(e_h, -RX), nv2_u1a = LHI(e_u1, -RX),
                             nv2_u1b = LHI(e_u1, -RX + 1), nv2_u3a = LHI(e_u3a, -RX),
                             nv2_u3b = LHI(e_u3b, -RX);
@@ -537,6 +561,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
                     }
                 }
                 const T v1 = do_v1 ? val1 : T(0), v2 = do_v2 ? val2 : T(0);
+                LMID_BASE
                 LMID(sv1, 0, 0) = v1;
                 LMID(sv2, 0, 0) = v2;
                 if constexpr (NONOS) {
@@ -569,25 +594,26 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         {
             const int Kn = K + 1;
             if (PER && pz) {
-                qx = pl(x, SXY, kc(Kn + 1));
+                qx = pl(x, SXY, kc(Kn + 1)); qr = pl(rhr, SXY, kc(Kn));
                 qu1 = pl(u1, FXY, kc(Kn)); qu2 = pl(u2, YXY, kc(Kn)); qu3 = pl(u3, SXY, fc(Kn + 1));
-                qh = pl(h, SXY, kc(Kn)); qr = pl(rhr, SXY, kc(Kn));
+                qh = pl(h, SXY, kc(Kn));
             } else {
                 const bool more = Kn <= lp;
                 const uint32_t dS = more ? SB8 : 0, dF = more ? FB8 : 0, dY = more ? YB8 : 0;
-                qx = adv(qx, Kn < lp ? SB8 : 0);
                 qu1 = adv(qu1, dF); qu2 = adv(qu2, dY); qu3 = adv(qu3, dS);
-                qh = adv(qh, dS); qr = adv(qr, dS);
+                qh = adv(qh, dS);
+                qx = adv(qx, Kn < lp ? SB8 : 0); qr = adv(qr, dS);
             }
-            if (Kn + 1 <= Alast) ld_halo(Kn + 1);
+            if constexpr (PER)
+                if (Kn + 1 <= Alast) ld_halo(Kn + 1);
             xq1 = ldo(qx, so);
+            rq2 = ldo(qr, so);
             u1a0 = ldo(qu1, fo);
             u1b0 = ld_u1b(qu1);
             u2a0 = ldo(qu2, so);
             u2b0 = ld_u2b(qu2);
             u3q0 = ldo(qu3, so);
             hq1 = ldo(qh, so);
-            rq2 = ldo(qr, so);
         }
         // donor flux of V1 through the right x-face of P: the left face of
         // the position to the right (the lane to the right, in the same row
@@ -595,6 +621,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         const T w1p = NONOS ? from_right_lane(w1) : T(0);
         __syncthreads();
         // ---- C: cp, cn on plane P (antidiff3d-standard-gpubc.f90:260-347) --
+        LMID_BASE
         T cpP, cnP, cpQ, cnQ;  // of the own column on planes P (formed here) and Q
         if constexpr (NONOS) {
             auto stage_c = [&](auto edge) __attribute__((always_inline)) {
@@ -669,6 +696,8 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
 #undef LLO
 #undef LMID
 #undef LHI
+#undef LMID_BASE
+#undef LHI_BASE
 #undef SB
     for (int K = Ks;;) {
         step(std::integral_constant<int, 0>{}, K);
