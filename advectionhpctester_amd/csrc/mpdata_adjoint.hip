@@ -549,8 +549,12 @@ __device__ __forceinline__ void adj_face_gauge(R* L, R vb, R x1, R x2, R a, R r,
 // GAUGE: the gauge variant's pseudo-velocities, whose adjoint a.v already
 // holds the limiter's part; else the standard variant's, with the adjoint
 // a.f of their donor fluxes.
+// Four waves a SIMD (128 VGPRs; the standard variant wants 136 and spills a
+// few): at 128x128x64 the grid is four blocks a CU, one round instead of one
+// and a third (88 -> 84 us; summing a thread's contributions in registers
+// first, 34 LDS atomics instead of 57, took 167 VGPRs and 94 us).
 template <bool GAUGE>
-__global__ void __launch_bounds__(PBX * PBY) k_adj_pseudo(Geo g, const R* __restrict__ u1,
+__global__ void __launch_bounds__(PBX * PBY, 4) k_adj_pseudo(Geo g, const R* __restrict__ u1,
                                                           const R* __restrict__ u2,
                                                           const R* __restrict__ u3,
                                                           const R* __restrict__ psi,
