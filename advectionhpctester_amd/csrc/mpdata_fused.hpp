@@ -119,8 +119,8 @@ struct DensIO {
 
 // The density step after the velocity predictor in the fused kernel: the
 // upwind divides by h and has no rhr factor, the update has none either,
-// and the update plane also writes DensIO's outputs.  x_out / m1..m3 are
-// out of place (x and u are read by neighbouring tiles' stencils); only
+// and the update plane also writes DensIO's outputs.  x_out / m1..m3 may not
+// be x / u1..u3 (neighbouring tiles' stencils read those); only
 // the cells and faces the reference defines are written (interior and
 // wall-line edge copies of x_out).
 template <typename T>

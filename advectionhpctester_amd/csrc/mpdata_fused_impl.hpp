@@ -154,7 +154,7 @@ __device__ __forceinline__ T div_(T a, T b) {
 // range of output planes [k0,k1] recomputing xant from k0-2 and cp,cn,V from
 // k0-1.  Inputs of plane K+1 are loaded while plane K is computed.
 //
-// What bounds it: not HBM (512x512x256 moves 5 GB in 1.3 ms) but the chain of
+// What bounds it: not HBM (512x512x256 moves 4.4 GB in 1.26 ms) but the chain of
 // a plane.  Four waves per SIMD, all of one workgroup and so in the same
 // stage, hide little of a wait, and the registers (128) leave no room for
 // more.  So nothing waits inside a step but the two barriers: all loads of a
@@ -162,8 +162,9 @@ __device__ __forceinline__ T div_(T a, T b) {
 // of a plane is issued right after that wait; h and rhr of the plane being
 // updated are kept, not loaded again; V, the bounds and cp/cn are formed
 // straight-line by every lane, so that their LDS reads go out together.
-// Together with the scalar plane pointers, 512x512x256 went from 1.66 to
-// 1.31 ms (fast build) and 256x256x128 from 294 to 233 us (exact build).
+// Together with the scalar plane pointers and the equal runs of March,
+// 512x512x256 went from 1.66 to 1.26 ms (fast build) and 256x256x128 from 294
+// to 232 us (exact build).
 // ---------------------------------------------------------------------------
 template <typename T>
 struct XSrc {  // where one sx cell comes from: x, bcx, bcy or nothing
@@ -1103,8 +1104,8 @@ int fused_chunk_env() {
     return c >= 1 ? c : -1;
 }
 
-// Workgroups of a persistent launch.  The kernels deal workgroups to the
-// NXCD XCDs round-robin and give XCD x the items of its contiguous share
+// Workgroups of a batched launch.  The kernel deals workgroups to the
+// NXCD XCDs round-robin and gives XCD x the items of its contiguous share
 // (items_per_xcd of them), so the grid is a multiple of NXCD with no more
 // workgroups per XCD than that share has items (a smaller share would
 // leave slots idle while items of the XCD wait for a second round); fewer
@@ -1145,9 +1146,11 @@ struct Tiling {
 
 // Modelled time of a step on RX x RY tiles with per_cu workgroups on each of
 // ncu CUs: the planes the busiest workgroup marches, times the time of a
-// plane, which a CU's march of 1024 cells sets (4.3 us in FP64) until there
-// are too few waves to hide the latency of the chain of a plane (2.95 us for
-// 512 cells, so no less than 0.69 of it).
+// plane, which a CU's march of 1024 cells sets (4.1 us in FP64) until there
+// are too few waves to hide the latency of the chain of a plane: 512 cells
+// take no less than 0.69 of it (any value from 0.62 to 0.75 gives the same
+// plans; 0.55 takes 190x147x83 standard from 113 to 130 us, 0.9 ten periodic
+// steps of 64x64x32 from 235 to 313 us).
 template <int RX, int RY>
 double tiling_time(const Geo& g, int ncu, int per_cu) {
     const March m = plan_march<RX, RY>(g, (long long)ncu * per_cu, 0);

@@ -14,9 +14,10 @@
 //
 // Kernels: the fused density step is the density mode of the tracer step's
 // fixed-position k-march kernel (FusedDens in mpdata_fused.hip), which
-// writes x and the mass fluxes out of place, followed by k_rho_copyback
-// into the reference's in-place arrays (neighbouring tiles read x and u
-// while tiles write).  For liner != 0, the context's per-stage path or
+// writes x and the mass fluxes out of place (neighbouring tiles read x and
+// the velocities while tiles write), followed by k_rho_copyback into the
+// reference's in-place arrays; after a fixed-step prediction the velocities
+// are in arrays of the context and only x is copied back.  For liner != 0, the context's per-stage path or
 // arrays too large for 32-bit offsets the stage kernels run: the density
 // upwind (k_rho_upwind: xant, the donor fluxes f*ns including the wall
 // faces, rhoadv), the gauge pseudo-velocity, face and limiter stages shared

@@ -287,7 +287,7 @@ def main():
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "alg_bytes_per_step": alg_bytes,
                      "duration": "HIP events around the timed steps on the launch stream; "
-                                 "a step is the fused kernel plus a halo-copy kernel"},
+                                 "a step is one kernel"},
         "exact_fused": exact,
         "max_rel_err_fast_vs_exact_50_steps": fast_err,
         "cpu_baseline": cpu,
