@@ -915,14 +915,14 @@ int check_adj(mpdata_ctx* c) {
     return MPDATA_OK;
 }
 
-int ensure_slot(mpdata_ctx* c, TapeSlot& t) {
+int ensure_slot(mpdata_ctx* c, TapeSlot& t, hipStream_t s) {
     int rc;
-    if ((rc = ensure(c, &t.xb, SCAL, 8)) || (rc = ensure(c, &t.x0, SCAL, 8)) ||
-        (rc = ensure(c, &t.psi, SCAL, 8)) || (rc = ensure(c, &t.cp, SCAL, 8)) ||
-        (rc = ensure(c, &t.cn, SCAL, 8)))
+    if ((rc = ensure(c, &t.xb, SCAL, 8, s)) || (rc = ensure(c, &t.x0, SCAL, 8, s)) ||
+        (rc = ensure(c, &t.psi, SCAL, 8, s)) || (rc = ensure(c, &t.cp, SCAL, 8, s)) ||
+        (rc = ensure(c, &t.cn, SCAL, 8, s)))
         return rc;
     for (int d = 0; d < 3; d++)
-        if ((rc = ensure(c, &t.v[d], FACEX + d, 8))) return rc;
+        if ((rc = ensure(c, &t.v[d], FACEX + d, 8, s))) return rc;
     return MPDATA_OK;
 }
 
@@ -935,8 +935,15 @@ int mpdata_adj_reserve(mpdata_ctx* c, int nslots) {
     if (rc) return rc;
     if (nslots < 1 || nslots > 4096) return fail(MPDATA_EINVAL, "nslots %d outside 1..4096", nslots);
     if ((int)c->tape.size() < nslots) c->tape.resize(nslots);
-    for (int q = 0; q < nslots; q++)
-        if ((rc = ensure_slot(c, c->tape[q]))) return rc;
+    // new slots are clear when the call returns, whatever stream records into
+    // them; v[2] is the last array a slot gets
+    ClearStream own;
+    for (int q = 0; q < nslots; q++) {
+        TapeSlot& t = c->tape[q];
+        if (t.v[2]) continue;
+        HIPCHK(own.open());
+        if ((rc = ensure_slot(c, t, own.s))) return rc;
+    }
     return MPDATA_OK;
 }
 
@@ -1006,8 +1013,8 @@ int mpdata_adj_record_variant_f64(mpdata_ctx* c, int slot, int variant, const do
     // scratch (the adjoint forms the first two again from the tape)
     R *fns[3], *vl[3], *f[3];
     for (int d = 0; d < 3; d++) {
-        if ((rc = ensure(c, &S.fns[d], FACEX + d, 8)) || (rc = ensure(c, &S.ul[d], FACEX + d, 8)) ||
-            (rc = ensure(c, &S.f[d], FACEX + d, 8)))
+        if ((rc = ensure(c, &S.fns[d], FACEX + d, 8, s)) || (rc = ensure(c, &S.ul[d], FACEX + d, 8, s)) ||
+            (rc = ensure(c, &S.f[d], FACEX + d, 8, s)))
             return rc;
         fns[d] = (R*)S.fns[d];
         vl[d] = (R*)S.ul[d];
@@ -1076,8 +1083,9 @@ int mpdata_adj_step_f64(mpdata_ctx* c, int slot, const double* u1, const double*
     if (!u1 || !u2 || !u3 || !rhr || !h || !xbar || !ubar1 || !ubar2 || !ubar3)
         return fail(MPDATA_EINVAL, "null pointer");
     const Geo& g = c->g;
+    hipStream_t s = (hipStream_t)stream;
     for (int q = 0; q < A_N; q++)
-        if ((rc = ensure(c, &c->adj[q], A_KIND[q], 8))) return rc;
+        if ((rc = ensure(c, &c->adj[q], A_KIND[q], 8, s))) return rc;
     // psi alternates between A_PSI and A_PSI2 from one reverse step to the
     // next (the upwind's reverse clears the other buffer)
     const int pcur = c->adj_psi ? A_PSI2 : A_PSI, pnext = c->adj_psi ? A_PSI : A_PSI2;
@@ -1085,7 +1093,6 @@ int mpdata_adj_step_f64(mpdata_ctx* c, int slot, const double* u1, const double*
           (R*)c->adj[A_CN], (R*)c->adj[A_V1], (R*)c->adj[A_V2], (R*)c->adj[A_V3],
           (R*)c->adj[A_F1], (R*)c->adj[A_F2], (R*)c->adj[A_F3], xbar, ufac};
     const TapeSlot& t = c->tape[slot];
-    hipStream_t s = (hipStream_t)stream;
     HIPCHK(hipGetLastError());
     if (t.variant == MPDATA_GAUGE)
         adj_reverse_antidiff<true>(g, t, u1, u2, u3, rhr, h, ubar1, ubar2, ubar3, a, s);

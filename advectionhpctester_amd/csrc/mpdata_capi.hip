@@ -50,7 +50,7 @@ long long field_len(const Geo& g, int kind) {
     }
 }
 
-int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes) {
+int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes, hipStream_t s) {
     if (*slot) return MPDATA_OK;
     size_t bytes = (size_t)field_len(c->g, kind) * elem_bytes;
     void* p = nullptr;
@@ -60,9 +60,23 @@ int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes) {
         return fail(MPDATA_ENOMEM, "hipMalloc(%zu bytes) for scratch failed: %s", bytes,
                     hipGetErrorString(e));
     }
-    // zero once so that halo cells never read are deterministic
-    e = hipMemset(p, 0, bytes);
-    if (e != hipSuccess) return hip_fail(e, "hipMemset(scratch)");
+    // zero once so that halo cells never read are deterministic.  On the
+    // stream that uses it: the null stream's hipMemset does not wait for the
+    // fill, and a non-blocking stream does not wait for the null stream.  Under
+    // capture the fill happens now, outside the graph.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    e = hipStreamIsCapturing(s, &cap);
+    if (e == hipSuccess && cap == hipStreamCaptureStatusNone) {
+        e = hipMemsetAsync(p, 0, bytes, s);
+    } else if (e == hipSuccess) {
+        ClearStream own;
+        e = own.open();
+        if (e == hipSuccess) e = hipMemsetAsync(p, 0, bytes, own.s);
+    }
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        return hip_fail(e, "clearing scratch");
+    }
     *slot = p;
     c->owned.push_back(p);
     c->held += (long long)bytes;
@@ -138,15 +152,15 @@ int stage_pass(mpdata_ctx* c, int variant, int nonos, const T* u1, const T* u2, 
     const bool stdv = variant == MPDATA_STANDARD;
     int rc;
     for (int d = 0; d < 3; d++)
-        if ((rc = ensure(c, &S.v[d], FACEX + d, sizeof(T)))) return rc;
+        if ((rc = ensure(c, &S.v[d], FACEX + d, sizeof(T), s))) return rc;
     if (nonos) {
-        if ((rc = ensure(c, &S.cp, SCAL, sizeof(T)))) return rc;
-        if ((rc = ensure(c, &S.cn, SCAL, sizeof(T)))) return rc;
+        if ((rc = ensure(c, &S.cp, SCAL, sizeof(T), s))) return rc;
+        if ((rc = ensure(c, &S.cn, SCAL, sizeof(T), s))) return rc;
     }
     if (stdv)
         for (int d = 0; d < 3; d++) {
-            if ((rc = ensure(c, &S.fns[d], FACEX + d, sizeof(T)))) return rc;
-            if ((rc = ensure(c, &S.f[d], FACEX + d, sizeof(T)))) return rc;
+            if ((rc = ensure(c, &S.fns[d], FACEX + d, sizeof(T), s))) return rc;
+            if ((rc = ensure(c, &S.f[d], FACEX + d, sizeof(T), s))) return rc;
         }
     T *v1 = (T*)S.v[0], *v2 = (T*)S.v[1], *v3 = (T*)S.v[2];
     T *f1ns = (T*)S.fns[0], *f2ns = (T*)S.fns[1], *f3ns = (T*)S.fns[2];
@@ -191,7 +205,7 @@ int step_stages(mpdata_ctx* c, int variant, int iters, int nonos, T* x, const T*
                 hipStream_t s) {
     Scratch& S = scr<T>(c);
     int rc;
-    if ((rc = ensure(c, &S.xant, SCAL, sizeof(T)))) return rc;
+    if ((rc = ensure(c, &S.xant, SCAL, sizeof(T), s))) return rc;
     T* xant = (T*)S.xant;
     tt_beg(16, s);  // upwind3d-gpubc.f90:87-200
     rc = upwind_impl<T>(c, u1, u2, u3, x, xant, rhr, h, bcx, bcy, s);
@@ -202,10 +216,10 @@ int step_stages(mpdata_ctx* c, int variant, int iters, int nonos, T* x, const T*
         return MPDATA_OK;
     }
     if (iters > 2) {
-        if ((rc = ensure(c, &S.psi2, SCAL, sizeof(T)))) return rc;
+        if ((rc = ensure(c, &S.psi2, SCAL, sizeof(T), s))) return rc;
         for (int d = 0; d < 3; d++) {
-            if ((rc = ensure(c, &S.ul[d], FACEX + d, sizeof(T)))) return rc;
-            if ((rc = ensure(c, &S.adv[d], FACEX + d, sizeof(T)))) return rc;
+            if ((rc = ensure(c, &S.ul[d], FACEX + d, sizeof(T), s))) return rc;
+            if ((rc = ensure(c, &S.adv[d], FACEX + d, sizeof(T), s))) return rc;
         }
     }
     T* psi = xant;
@@ -280,10 +294,10 @@ int fused_step(mpdata_ctx* c, int variant, int iters, int nonos, const T* x, T* 
     if (iters == 3) {
         Scratch& S = scr<T>(c);
         int rc;
-        if ((rc = ensure(c, &S.psi2, SCAL, sizeof(T))) ||
-            (rc = ensure(c, &S.ul[0], FACEX, sizeof(T))) ||
-            (rc = ensure(c, &S.ul[1], FACEY, sizeof(T))) ||
-            (rc = ensure(c, &S.ul[2], FACEZ, sizeof(T))))
+        if ((rc = ensure(c, &S.psi2, SCAL, sizeof(T), s)) ||
+            (rc = ensure(c, &S.ul[0], FACEX, sizeof(T), s)) ||
+            (rc = ensure(c, &S.ul[1], FACEY, sizeof(T), s)) ||
+            (rc = ensure(c, &S.ul[2], FACEZ, sizeof(T), s)))
             return rc;
         sc.x2 = (T*)S.psi2;
         for (int d = 0; d < 3; d++) sc.ul[d] = (T*)S.ul[d];
@@ -319,7 +333,7 @@ int step_impl(mpdata_ctx* c, int variant, int iters, int nonos, T* x, const T* u
     if ((rc = use_fused<T>(c, variant, iters, nonos, &fused))) return rc;
     if (!fused)
         return step_stages<T>(c, variant, iters, nonos, x, u1, u2, u3, rhr, h, bcx, bcy, s);
-    if ((rc = ensure(c, &S.xnext, SCAL, sizeof(T)))) return rc;
+    if ((rc = ensure(c, &S.xnext, SCAL, sizeof(T), s))) return rc;
     T* xn = (T*)S.xnext;
     if ((rc = fused_step<T>(c, variant, iters, nonos, x, xn, u1, u2, u3, rhr, h, bcx, bcy, s))) return rc;
     HIPCHK(hipMemcpyAsync(x, xn, (size_t)len_of<SCAL>(c->g) * sizeof(T), hipMemcpyDeviceToDevice, s));
@@ -366,7 +380,7 @@ int timeloop_impl(mpdata_ctx* c, int variant, int iters, int nonos, int nt, T* x
                 return rc;
         return MPDATA_OK;
     }
-    if ((rc = ensure(c, &S.xnext, SCAL, sizeof(T)))) return rc;
+    if ((rc = ensure(c, &S.xnext, SCAL, sizeof(T), s))) return rc;
     T* buf[2] = {x, (T*)S.xnext};
     for (int it = 0; it < nt; it++)
         if ((rc = fused_step<T>(c, variant, iters, nonos, buf[it & 1], buf[(it + 1) & 1], u1, u2,
@@ -739,9 +753,9 @@ int tl_step_impl(mpdata_ctx* c, int variant, int iters, int nonos, double* x, do
     const Geo& g = c->g;
     const int kinds[6] = {SCAL, FACEX, FACEY, FACEZ, SCAL, SCAL};
     for (int q = 0; q < 6; q++)
-        if ((rc = ensure(c, &S.in[q], kinds[q], sizeof(D64)))) return rc;
+        if ((rc = ensure(c, &S.in[q], kinds[q], sizeof(D64), s))) return rc;
     // inflow values: (2, lp, mp) and (2, lp, np) arrays, sized as x faces to fit
-    if ((rc = ensure(c, &S.in[6], FACEX, sizeof(D64))) || (rc = ensure(c, &S.in[7], FACEX, sizeof(D64))))
+    if ((rc = ensure(c, &S.in[6], FACEX, sizeof(D64), s)) || (rc = ensure(c, &S.in[7], FACEX, sizeof(D64), s)))
         return rc;
     const double* vals[6] = {x, u1, u2, u3, rhr, h};
     const double* tans[6] = {dx, du1, du2, du3, nullptr, nullptr};
@@ -790,7 +804,9 @@ int mpdata_dev_alloc(long long bytes, void** ptr) {
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, (size_t)bytes);
     if (e != hipSuccess) return fail(MPDATA_ENOMEM, "hipMalloc(%lld): %s", bytes, hipGetErrorString(e));
+    // the memory is zero when the call returns, whatever stream uses it
     e = hipMemset(p, 0, (size_t)bytes);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         (void)hipFree(p);
         return hip_fail(e, "hipMemset");

@@ -84,7 +84,19 @@ bool any_null(P... p) {
         if (!q) return true;
     return false;
 }
-// Allocates *slot (field of `kind`, elem_bytes per element) unless set.
-int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes);
+// Allocates *slot (field of `kind`, elem_bytes per element) unless set, and
+// clears it on stream s, on which it is used next.
+int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes, hipStream_t s);
+// A stream of its own to clear memory on, for a caller that has no stream or
+// one under capture; the destructor waits for what was queued on it.
+struct ClearStream {
+    hipStream_t s = nullptr;
+    hipError_t open() { return s ? hipSuccess : hipStreamCreateWithFlags(&s, hipStreamNonBlocking); }
+    ~ClearStream() {
+        if (!s) return;
+        (void)hipStreamSynchronize(s);
+        (void)hipStreamDestroy(s);
+    }
+};
 
 }  // namespace mpdata

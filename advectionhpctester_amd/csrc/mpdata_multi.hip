@@ -171,7 +171,7 @@ int ce_impl(mpdata_ctx* c, int alg_choice, int liner, int nfields, const int* ro
         const bool inplace = !oop;
         T* xo = x_out[f];
         if (inplace) {
-            int rc = ensure(c, &c->mf_out[j], SCAL, sizeof(T));
+            int rc = ensure(c, &c->mf_out[j], SCAL, sizeof(T), s);
             if (rc) return rc;
             xo = (T*)c->mf_out[j];
         }

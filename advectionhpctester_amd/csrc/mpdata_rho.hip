@@ -299,12 +299,12 @@ int rho_run(mpdata_ctx* c, int liner, T* a1, T* a2, T* a3, T* u1, T* u2, T* u3, 
     int rc;
     const bool fused = !liner && c->path != MPDATA_PATH_STAGES && rho_fusable(g);
     if (fused) {
-        if ((rc = ensure(c, &S.xnext, SCAL, sizeof(T)))) return rc;
+        if ((rc = ensure(c, &S.xnext, SCAL, sizeof(T), s))) return rc;
         T *xn = (T*)S.xnext, *m1 = u1, *m2 = u2, *m3 = u3;
         const bool faces = a1 == u1;  // not yet out of place
         if (faces) {
             for (int d = 0; d < 3; d++)
-                if ((rc = ensure(c, &S.f[d], FACEX + d, sizeof(T)))) return rc;
+                if ((rc = ensure(c, &S.f[d], FACEX + d, sizeof(T), s))) return rc;
             m1 = (T*)S.f[0], m2 = (T*)S.f[1], m3 = (T*)S.f[2];
         }
         const DensIO<T> dio{xinc, pexe, rhoadv, rhr, pexr1, pexr2, m1, m2, m3};
@@ -321,14 +321,14 @@ int rho_run(mpdata_ctx* c, int liner, T* a1, T* a2, T* a3, T* u1, T* u2, T* u3, 
         HIPCHK(hipGetLastError());
         return MPDATA_OK;
     }
-    if ((rc = ensure(c, &S.xant, SCAL, sizeof(T)))) return rc;
+    if ((rc = ensure(c, &S.xant, SCAL, sizeof(T), s))) return rc;
     for (int d = 0; d < 3; d++) {
-        if ((rc = ensure(c, &S.fns[d], FACEX + d, sizeof(T)))) return rc;
-        if (!liner && (rc = ensure(c, &S.v[d], FACEX + d, sizeof(T)))) return rc;
+        if ((rc = ensure(c, &S.fns[d], FACEX + d, sizeof(T), s))) return rc;
+        if (!liner && (rc = ensure(c, &S.v[d], FACEX + d, sizeof(T), s))) return rc;
     }
     if (!liner) {
-        if ((rc = ensure(c, &S.cp, SCAL, sizeof(T)))) return rc;
-        if ((rc = ensure(c, &S.cn, SCAL, sizeof(T)))) return rc;
+        if ((rc = ensure(c, &S.cp, SCAL, sizeof(T), s))) return rc;
+        if ((rc = ensure(c, &S.cn, SCAL, sizeof(T), s))) return rc;
     }
     T* xant = (T*)S.xant;
     T *f1ns = (T*)S.fns[0], *f2ns = (T*)S.fns[1], *f3ns = (T*)S.fns[2];
@@ -368,12 +368,13 @@ int rho_run(mpdata_ctx* c, int liner, T* a1, T* a2, T* a3, T* u1, T* u2, T* u3, 
 // u1..u3, and a vertical split also halves the halo faces of u3: they keep
 // u1..u3 as the predictor's arrays.
 template <typename T>
-int rho_velocity(mpdata_ctx* c, int liner, int lsub, int ladapt, int lvs, T** a) {
+int rho_velocity(mpdata_ctx* c, int liner, int lsub, int ladapt, int lvs, T** a,
+                 hipStream_t s) {
     const bool fused = !liner && c->path != MPDATA_PATH_STAGES && rho_fusable(c->g);
     if (!fused || lsub || ladapt || lvs) return MPDATA_OK;
     int rc;
     for (int d = 0; d < 3; d++) {
-        if ((rc = ensure(c, &c->prim.f[d], FACEX + d, sizeof(T)))) return rc;
+        if ((rc = ensure(c, &c->prim.f[d], FACEX + d, sizeof(T), s))) return rc;
         a[d] = (T*)c->prim.f[d];
     }
     return MPDATA_OK;
@@ -594,7 +595,8 @@ extern "C" {
                             pexr2, bcx, bcy)))                                                   \
             return rc;                                                                           \
         T* a[3] = {u1, u2, u3};                                                                  \
-        if ((rc = rho_velocity<T>(ctx, liner, lsubstepping, ltimeadapt, lvertsplit, a)))         \
+        if ((rc = rho_velocity<T>(ctx, liner, lsubstepping, ltimeadapt, lvertsplit, a,           \
+                                  (hipStream_t)stream)))                                        \
             return rc;                                                                           \
         if ((rc = driver_impl<T>(ctx, nsubsteps, nsubsteps_o, lsubstepping, dtn, dtnold,         \
                                  ltimeadapt, lvertsplit, lcrdiag_nphlf, crmaxlim, dtmax, ox, oy, \
