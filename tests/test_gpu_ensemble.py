@@ -294,3 +294,52 @@ def test_fast_build_equals_fast_single_domain_steps(mpd):
                 assert err <= 1e-12, f"cfg {cfg} member {q}: {err:.2e} from the exact build"
         with pytest.raises(mpd.MpdataError):
             ens.set_path(mpd.PATH_STAGES)
+
+
+def test_many_members_with_halos(mpd):
+    """More members than the launch has blocks for their halos, and one whose
+    halo is many blocks' work: every cell of every member."""
+    dtype = torch.float64
+    shapes = [(5 + q % 7, 4 + q % 5, 3 + q % 3) for q in range(330)] + [(300, 120, 4)]
+    members = _members(dtype, shapes, seed0=900)
+    want = _reference_steps(mpd, shapes, members, [m["x"] for m in members], 1, dtype)
+    ens, xa, xb = _ensemble(mpd, shapes, members, dtype)
+    with ens:
+        for cfg in (1, 5):
+            print(f"331 members cfg {cfg}", flush=True)
+            ens.set_tiling(cfg, 64)
+            for t in xb:
+                t.fill_(-1.0)
+            ens.step(0)
+            torch.cuda.synchronize()
+            for q, (got, w) in enumerate(zip(xb, want)):
+                assert torch.equal(got, w), f"cfg {cfg} member {q} {shapes[q]}"
+
+
+def test_halo_cost_of_many_small_members(mpd):
+    """1000 members of one tile each take about as long as 250 members of four
+    tiles each (as many work items and interior cells, the same kernel): their
+    halos are copied by all the blocks, not one member after the other."""
+    dtype = torch.float64
+    ms = {}
+    for n, s in ((1000, (20, 20, 10)), (250, (40, 40, 10))):
+        members = _members(dtype, [s], seed0=7) * n
+        ens = mpd.Ensemble([s] * n, dtype=dtype)
+        xb = [torch.zeros_like(m["x"]) for m in members]
+        ens.set_fields([m["x"] for m in members], xb, *[[m[k] for m in members] for k in
+                       ("u1", "u2", "u3", "rhr", "h", "bcx", "bcy")])
+        with ens:
+            ens.set_tiling(5, 64)
+            best = []
+            for _ in range(5):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                ens.step(0)
+                a.record()
+                for _ in range(20):
+                    ens.step(0)
+                b.record()
+                b.synchronize()
+                best.append(a.elapsed_time(b) / 20)
+            ms[n] = min(best)
+    print(f"1000 small members {ms[1000]:.3f} ms, 250 larger ones {ms[250]:.3f} ms", flush=True)
+    assert ms[1000] < 1.6 * ms[250], ms
