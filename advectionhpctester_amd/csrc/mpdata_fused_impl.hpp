@@ -214,8 +214,13 @@ static_assert(sizeof(FusedLds<double, 32, 32>) <= 160 * 1024, "LDS of one CU");
 // with its mirrored x/y halo ring, V on every face of the domain (zero on
 // the x/y walls, mirrored on the lids), cp and cn.  Each cell and face is
 // written by the one position that owns it.
+// EARLY: x and r of the next plane are loaded before the first barrier.  Not
+// on the batch's tilings bounded at 2 waves per SIMD: their registers then go
+// past 128 and a CU holds one workgroup instead of the two that its LDS fits
+// (32 members of 32..256 cells a side, fast build, 64x8 tiles: 3.72 ms a step
+// with it, 2.92 without; 32x16: 2.64 and 2.17).
 template <typename T, int RX, int RY, bool DENS = false, bool FAST = false, int PASS = 0,
-          bool TAPE = false>
+          bool TAPE = false, bool EARLY = FAST>
 __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, int tile, int k0,
                                            int k1, const T* __restrict__ x, const T* __restrict__ u1,
                                            const T* __restrict__ u2, const T* __restrict__ u3,
@@ -624,7 +629,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         // build, 512x512x256: 1.35 -> 1.27 ms; the exactly rounded build spills
         // with x and r here and loses 2 % on small domains)
         if (K + 2 <= Alast) ld_halo(K + 2);
-        if constexpr (FAST) load_xr(K);
+        if constexpr (EARLY) load_xr(K);
         __syncthreads();
 // xant of plane K-d at tile position (a, b)
 #define XA(d, a, b) sxa[(d) == 0 ? R0 : ((d) == 1 ? R1 : R2)][(b) + 2][(a) + 2]
@@ -720,7 +725,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
             // the scalar instructions)
             const int Kn = K + 1;
             const uint32_t dS = Kn <= lp ? SB8 : 0, dF = Kn <= lp ? FB8 : 0, dY = Kn <= lp ? YB8 : 0;
-            if constexpr (!FAST) load_xr(K);
+            if constexpr (!EARLY) load_xr(K);
             qu1 = adv(qu1, dF); qu2 = adv(qu2, dY); qu3 = adv(qu3, dS); qh = adv(qh, dS);
             u1a0 = ldo(qu1, fo);
             u1b0 = ldo(qu1 + 1, fo);
@@ -1367,8 +1372,9 @@ k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int
         const int k0 = uniform(c0 + len * part / nparts),
                   k1 = uniform(c0 + len * (part + 1) / nparts - 1);
         if (k0 > k1) continue;  // a chunk shorter than the split (uniform: every thread)
-        fused_item<T, RX, RY, false, FAST>(m.g, m.o, m.ntx, uniform(tile), k0, k1, m.x, m.u1, m.u2, m.u3,
-                                           m.rhr, m.h, m.bcx, m.bcy, m.xo, L);
+        fused_item<T, RX, RY, false, FAST, 0, false, FAST && MINB >= 4>(
+            m.g, m.o, m.ntx, uniform(tile), k0, k1, m.x, m.u1, m.u2, m.u3, m.rhr, m.h, m.bcx, m.bcy,
+            m.xo, L);
     }
     if (threadIdx.x == 0 && atomicAdd(&sc->done[xcd], 1) == per_xcd - 1) {
         atomicExch(&sc->next[xcd], 0);

@@ -343,3 +343,31 @@ def test_halo_cost_of_many_small_members(mpd):
             ms[n] = min(best)
     print(f"1000 small members {ms[1000]:.3f} ms, 250 larger ones {ms[250]:.3f} ms", flush=True)
     assert ms[1000] < 1.6 * ms[250], ms
+
+
+def test_fast_build_no_slower_on_any_tiling(mpd):
+    """The fast build of the batched step, whose divisions are cheaper, is no
+    slower than the exactly rounded one on any tile configuration (a
+    configuration whose registers leave one workgroup on a CU where two fit
+    is)."""
+    shapes = [(96 + 32 * (q % 4), 80 + 24 * (q % 5), 48 + 16 * (q % 3)) for q in range(24)]
+    members = _members(torch.float64, shapes, seed0=40)
+    ens, xa, xb = _ensemble(mpd, shapes, members, torch.float64)
+    with ens:
+        for cfg, name in enumerate(mpd.Ensemble.configs()):
+            ms = {}
+            for _ in range(4):  # in turn
+                for path in (mpd.PATH_FUSED, mpd.PATH_FAST):
+                    ens.set_path(path)
+                    ens.set_tiling(cfg, 64)
+                    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                    ens.step(0)
+                    a.record()
+                    for _ in range(5):
+                        ens.step(0)
+                    b.record()
+                    b.synchronize()
+                    ms.setdefault(path, []).append(a.elapsed_time(b) / 5)
+            exact, fast = min(ms[mpd.PATH_FUSED]), min(ms[mpd.PATH_FAST])
+            print(f"{name}: exact {exact:.3f} fast {fast:.3f} ms", flush=True)
+            assert fast < exact, (name, fast, exact)
