@@ -223,20 +223,19 @@ __global__ void __launch_bounds__(256)
 // velprd_traj0's extrapolation (module_velprd.f90:55-85) followed, per cell,
 // by the time-level rotation (velprd_driver.f90:254-270): level n-1 of ox is
 // read before the rotation overwrites it with ox(.,0)*h.  Bound by HBM (25
-// array passes): a block takes a row of one of the six fields, so that it
-// streams five arrays rather than 25 (h is read again by the blocks of oy and
-// oz, from L2), and the level stores are non-temporal, since nothing reads
-// them back before they leave L2 (row_block has the figures).
+// array passes): a block takes consecutive cells of one of the six fields, so
+// that it streams five arrays rather than 25 (h is read again by the blocks of
+// oy and oz, from L2), and the level stores are non-temporal, since nothing
+// reads them back before they leave L2 (plane_grid has the figures).
 template <typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kPlaneThreads)
     k_extrap_rotate(Geo g, T* __restrict__ ox, T* __restrict__ oy, T* __restrict__ oz,
                     T* __restrict__ u, T* __restrict__ v, T* __restrict__ w,
                     const T* __restrict__ h, T gc1, T gc2, T gc3, T r) {
     const int q = blockIdx.x % 6;
-    const int i = 1 + blockIdx.x / 6 * blockDim.x + threadIdx.x;
-    const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
+    int i, j;
     const int k = 1 + blockIdx.z;
-    if (i > g.np || j > g.mp) return;
+    if (!plane_cell(g, blockIdx.x / 6, i, j)) return;
     const long long n = len_of<SCAL>(g);
     const long long c = off_raw<SCAL>(g, i, j, k);
     if (q < 3) {
@@ -419,7 +418,7 @@ struct Driver {
     int traj0_rotate(T dtv, T* u, T* v, T* w) {
         const Geo& g = c->g;
         const long long n = len_of<SCAL>(g);
-        k_extrap_rotate<T><<<row_grid(g, 6), row_block(g.np, g.mp), 0, s>>>(
+        k_extrap_rotate<T><<<plane_grid(g, 6), kPlaneThreads, 0, s>>>(
             g, ox, oy, oz, u, v, w, h, dtv * dxi, dtv * dyi, dtv * dzi, dt_ratio);
         HIPCHK(hipGetLastError());
         HIPCHK(Stages<T>::a_to_c(g, ox + n, oy + n, oz + n, u1, u2, u3, s));

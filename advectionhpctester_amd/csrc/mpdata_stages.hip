@@ -507,19 +507,25 @@ __global__ void k_extrap_halo(Geo g, T* __restrict__ a, int dir) {
 }
 
 // A->C averaging u1(i)=0.5*(ox(i)+ox(i-1)) on faces 1..n+1 (open) or 1..n
-// (periodic): one thread per cell, that of the last cell of a direction also
-// forms its wall face, so that the blocks are whole rows (row_block).
+// (periodic): one thread per cell forms its low faces, and that of the last
+// cell of an open direction then its wall face.  (The wall faces by a second
+// turn of a loop around each face take 108 us at 256x256x128 in FP64 for 92:
+// the loads of the three faces no longer go out together.)
 template <typename T>
-__global__ void k_a_to_c(Geo g, const T* __restrict__ ox, const T* __restrict__ oy,
-                         const T* __restrict__ oz, T* __restrict__ u1, T* __restrict__ u2,
-                         T* __restrict__ u3) {
-    CELL_LOOP_HEAD
-    for (int q = i; q <= (i == g.np && !g.px ? i + 1 : i); q++)
-        X_(u1, q, j, k) = T(0.5) * (S_(ox, q, j, k) + S_(ox, q - 1, j, k));
-    for (int q = j; q <= (j == g.mp && !g.py ? j + 1 : j); q++)
-        Y_(u2, i, q, k) = T(0.5) * (S_(oy, i, q, k) + S_(oy, i, q - 1, k));
-    for (int q = k; q <= (k == g.lp && !g.pz ? k + 1 : k); q++)
-        Z_(u3, i, j, q) = T(0.5) * (S_(oz, i, j, q) + S_(oz, i, j, q - 1));
+__global__ void __launch_bounds__(kPlaneThreads)
+k_a_to_c(Geo g, const T* __restrict__ ox, const T* __restrict__ oy, const T* __restrict__ oz,
+         T* __restrict__ u1, T* __restrict__ u2, T* __restrict__ u3) {
+    int i, j;
+    const int k = 1 + blockIdx.z;
+    if (!plane_cell(g, xcd_block(), i, j)) return;
+    const T a = S_(ox, i, j, k) + S_(ox, i - 1, j, k), b = S_(oy, i, j, k) + S_(oy, i, j - 1, k),
+            c = S_(oz, i, j, k) + S_(oz, i, j, k - 1);
+    X_(u1, i, j, k) = T(0.5) * a;
+    Y_(u2, i, j, k) = T(0.5) * b;
+    Z_(u3, i, j, k) = T(0.5) * c;
+    if (i == g.np && !g.px) X_(u1, i + 1, j, k) = T(0.5) * (S_(ox, i + 1, j, k) + S_(ox, i, j, k));
+    if (j == g.mp && !g.py) Y_(u2, i, j + 1, k) = T(0.5) * (S_(oy, i, j + 1, k) + S_(oy, i, j, k));
+    if (k == g.lp && !g.pz) Z_(u3, i, j, k + 1) = T(0.5) * (S_(oz, i, j, k + 1) + S_(oz, i, j, k));
 }
 
 // The predictor in one pass (open walls): velprd_traj0's extrapolation of the
@@ -542,16 +548,19 @@ __device__ __forceinline__ T half_level(const T* __restrict__ a, const T* __rest
 
 // One thread per cell, that of the last cell of a direction also forming its
 // wall face; the level-n+1/2 values of the neighbouring cells are recomputed
-// from their inputs (cache hits).  (A k-march with the z neighbour carried in
-// registers measured slower: 226 against 188 us at 256x256x128 in FP64, its
+// from their inputs, which are in the XCD's L2 (xcd_block).  156 us at
+// 256x256x128 in FP64.  (A k-march with the z neighbour carried in registers
+// measured slower: 226 against the 188 us of a thread a face at the time, its
 // serial plane loop exposing the load latency.)
 template <typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kPlaneThreads)
 k_predict_ac(Geo g, const T* __restrict__ ox, const T* __restrict__ oy, const T* __restrict__ oz,
              const T* __restrict__ oxp, const T* __restrict__ oyp, const T* __restrict__ ozp,
              const T* __restrict__ h, T gc1, T gc2, T gc3, T r, T* __restrict__ u1,
              T* __restrict__ u2, T* __restrict__ u3) {
-    CELL_LOOP_HEAD
+    int i, j;
+    const int k = 1 + blockIdx.z;
+    if (!plane_cell(g, xcd_block(), i, j)) return;
     const int np = g.np, mp = g.mp, lp = g.lp;
     auto cell = [&](int ii, int jj, int kk) { return off_raw<SCAL>(g, ii, jj, kk); };
     // level n+1/2 at cells m (upstream) and c (downstream) of a face at
@@ -574,15 +583,24 @@ k_predict_ac(Geo g, const T* __restrict__ ox, const T* __restrict__ oy, const T*
         }
         return T(0.5) * (lc + lm);
     };
-    for (int q = i; q <= (i == np ? i + 1 : i); q++)
+    auto fx = [&](int q) {
         u1[off_raw<FACEX>(g, q, j, k)] =
             face(ox, oxp, gc1, q, np, [&](int a) { return cell(a, j, k); });
-    for (int q = j; q <= (j == mp ? j + 1 : j); q++)
+    };
+    auto fy = [&](int q) {
         u2[off_raw<FACEY>(g, i, q, k)] =
             face(oy, oyp, gc2, q, mp, [&](int a) { return cell(i, a, k); });
-    for (int q = k; q <= (k == lp ? k + 1 : k); q++)
+    };
+    auto fz = [&](int q) {
         u3[off_raw<FACEZ>(g, i, j, q)] =
             face(oz, ozp, gc3, q, lp, [&](int a) { return cell(i, j, a); });
+    };
+    fx(i);
+    fy(j);
+    fz(k);
+    if (i == np) fx(i + 1);
+    if (j == mp) fy(j + 1);
+    if (k == lp) fz(k + 1);
 }
 
 // Time-level rotation: velprd_driver.f90:254-270
@@ -845,7 +863,7 @@ hipError_t Stages<T>::a_to_c(const Geo& g, T* ox, T* oy, T* oz, T* u1, T* u2, T*
         dim3 grid((g.np + 63) / 64, (g.mp + 3) / 4, 2);
         k_extrap_halo<T><<<grid, wall_block(), 0, s>>>(g, oz, 2);
     }
-    k_a_to_c<T><<<row_grid(g), row_block(g.np, g.mp), 0, s>>>(g, ox, oy, oz, u1, u2, u3);
+    k_a_to_c<T><<<plane_grid(g), kPlaneThreads, 0, s>>>(g, ox, oy, oz, u1, u2, u3);
     return hipGetLastError();
 }
 
@@ -853,8 +871,8 @@ template <typename T>
 hipError_t Stages<T>::predict_ac(const Geo& g, const T* ox, const T* oy, const T* oz,
                                  const T* oxp, const T* oyp, const T* ozp, const T* h, T gc1,
                                  T gc2, T gc3, T dt_ratio, T* u1, T* u2, T* u3, hipStream_t s) {
-    k_predict_ac<T><<<row_grid(g), row_block(g.np, g.mp), 0, s>>>(g, ox, oy, oz, oxp, oyp, ozp, h, gc1,
-                                                             gc2, gc3, dt_ratio, u1, u2, u3);
+    k_predict_ac<T><<<plane_grid(g), kPlaneThreads, 0, s>>>(g, ox, oy, oz, oxp, oyp, ozp, h, gc1, gc2,
+                                                            gc3, dt_ratio, u1, u2, u3);
     return hipGetLastError();
 }
 

@@ -199,3 +199,76 @@ def test_three_iterations_fast_within_1e12(mpd):
     err = float((res["fast"] - res["exact"]).abs().max() / res["exact"].abs().max())
     print(f"three iterations fast vs exact after 50 steps: {err:.3e}", flush=True)
     assert err <= 1e-12
+
+
+# cells of a plane: one block exactly, one short of it, rows of one block and
+# one cell more, the smallest, nine blocks dealt to eight XCDs, long rows
+PLANES = [(16, 16, 4), (17, 15, 3), (256, 4, 3), (257, 3, 3), (3, 3, 3), (20, 103, 5), (300, 41, 4)]
+
+
+@pytest.mark.parametrize("tdt,npdt,orcname", [(torch.float64, np.float64, "orc64"),
+                                              (torch.float32, np.float32, "orc32")])
+@pytest.mark.parametrize("size", PLANES)
+@pytest.mark.parametrize("ibc", [(0, 0, 0), (1, 0, 1), (1, 1, 1)])
+def test_a_to_c_plane_blocks(mpd, request, tdt, npdt, orcname, size, ibc):
+    """The averaging to faces at the edges of its blocks: every array, cells
+    that it leaves alone included, against the oracle."""
+    orc = request.getfixturevalue(orcname)
+    dims = size + (1,)
+    rng = np.random.default_rng(sum(size))
+    a = [rng.uniform(-2, 2, shape(*dims)).astype(npdt) for _ in range(3)]
+    u = [rng.uniform(-2, 2, shape(*dims, kind=k)).astype(npdt) for k in (1, 2, 3)]
+    with mpd.Domain(*dims, ibc=ibc, dtype=tdt) as d:
+        t = [to_dev(v) for v in a + u]
+        print(f"A to C {size} ibc={ibc} {npdt.__name__}", flush=True)
+        d.velprdA_to_C(*t)
+        got = [to_host(v) for v in t]
+    orc.velprdA_to_C(*a, *u, ibc, dims)
+    for q, (x, y) in enumerate(zip(got, a + u)):
+        assert bits_equal(x, y), f"array {q}: " + describe_diff(x, y)
+
+
+@pytest.mark.parametrize("tdt,npdt,orcname", [(torch.float64, np.float64, "orc64"),
+                                              (torch.float32, np.float32, "orc32")])
+@pytest.mark.parametrize("size", PLANES)
+def test_velprd_c_plane_blocks(mpd, request, tdt, npdt, orcname, size):
+    orc = request.getfixturevalue(orcname)
+    dims = size + (1,)
+    rng = np.random.default_rng(sum(size) + 1)
+    a = [rng.uniform(-2, 2, shape(*dims)).astype(npdt) for _ in range(6)]
+    h = rng.uniform(0.8, 1.2, shape(*dims)).astype(npdt)
+    u = [rng.uniform(-2, 2, shape(*dims, kind=k)).astype(npdt) for k in (1, 2, 3)]
+    sp = (0.7, 0.9, 1.1, 0.05, 0.8)
+    with mpd.Domain(*dims, dtype=tdt) as d:
+        t = [to_dev(v) for v in a + [h]]
+        c = [to_dev(v) for v in u]
+        print(f"velprd_c {size} {npdt.__name__}", flush=True)
+        d.velprd_c(*t, *sp, *c)
+        got = [to_host(v) for v in c]
+    lev = [np.stack([x, np.zeros_like(x), p * h]) for x, p in zip(a[:3], a[3:])]
+    orc.velprd_traj0(*lev, *u, h, *sp, (0, 0, 0), dims)
+    for q, (x, y) in enumerate(zip(got, u)):
+        assert bits_equal(x, y), f"u{q + 1}: " + describe_diff(x, y)
+
+
+def test_a_to_c_cost_of_short_rows(mpd):
+    """Rows of 10 cells cost no more than rows of 372 in as many planes (a
+    block of rows rounded up to a wave idles five lanes of six)."""
+    us = {}
+    for size in ((10, 372, 114), (372, 10, 114)):
+        with mpd.Domain(*size) as d:
+            a = [d.zeros(0) + 0.1 for _ in range(3)]
+            u = [d.zeros(k) for k in (1, 2, 3)]
+            best = []
+            for _ in range(6):
+                s, e = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                d.velprdA_to_C(*a, *u)
+                s.record()
+                for _ in range(50):
+                    d.velprdA_to_C(*a, *u)
+                e.record()
+                e.synchronize()
+                best.append(s.elapsed_time(e) / 50 * 1e3)
+            us[size[0]] = min(best)
+    print(f"A to C: rows of 10 {us[10]:.1f} us, rows of 372 {us[372]:.1f} us", flush=True)
+    assert us[10] < 1.35 * us[372], us

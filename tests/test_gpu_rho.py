@@ -171,6 +171,15 @@ def test_driver_and_core_alone(mp, tdt, npdt, part, liner):
     _run_both(mp, dims, f, flags, liner, 2, tdt, npdt, part=part)
 
 
+@pytest.mark.parametrize("tdt,npdt", DTYPES)
+@pytest.mark.parametrize("size", [(16, 16, 4), (17, 15, 3), (257, 3, 3), (20, 103, 5)])
+def test_driver_plane_blocks(mp, tdt, npdt, size):
+    """The fixed-step driver's extrapolation and rotation at the edges of its
+    blocks (256 consecutive cells of a plane, nine blocks and one)."""
+    dims = size + (1,)
+    _run_both(mp, dims, _case(dims, 13, 0.4, npdt), {}, 0, 2, tdt, npdt, part="driver")
+
+
 @pytest.mark.parametrize("path", ["PATH_FUSED", "PATH_STAGES"])
 @pytest.mark.parametrize("ih", [2, 3])
 def test_rho_gauge_wide_halo(mp, path, ih):
