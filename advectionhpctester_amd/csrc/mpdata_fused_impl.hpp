@@ -903,15 +903,17 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
 // cut into equal runs, one a workgroup, so that all of them finish together
 // whatever the numbers of tiles and planes.  Chunks of one length for all
 // tiles, in rounds, left the last round part-empty: at 256x256x128 100 tiles
-// x 2 chunks for 256 CUs, at 384x320x192 504 chunks of 64 planes.  `run` may
-// also be a fixed chunk (the tuning override): then there are more runs than
-// workgroups, and ext is the next multiple of it.
+// x 2 chunks for 256 CUs, at 384x320x192 504 chunks of 64 planes.  Where they
+// fit, and with the tuning override, `run` is such a chunk all the same: then
+// lead is 0, ext the next multiple of it, and a workgroup may take several.
+// Each XCD gets an equal share of the runs.
 struct March {
     int nwg;            // workgroups that take items, a multiple of NXCD from NXCD on
     int ntx, ntile;
     int nfull;          // whole tiles per workgroup
     int run, lead, ext; // see above
     int grp;            // tiles that are cut together
+    int share;          // runs of an XCD, neighbouring ones
 };
 
 // Calls item(tile, k0, k1) for this workgroup's items (one call site: the
@@ -923,11 +925,12 @@ __device__ __forceinline__ void march_items(const March& m, int lp, F&& item) {
     const int nxcd = m.nwg >= NXCD ? NXCD : 1;
     const int per_xcd = m.nwg / nxcd;
     const int xcd = blockIdx.x % nxcd, slot = blockIdx.x / nxcd;
-    const int ngrp = m.nwg / m.grp, in_grp = slot % m.grp;
-    const int g = xcd * (per_xcd / m.grp) + slot / m.grp;
+    const int ngrp = per_xcd / m.grp, in_grp = slot % m.grp;
     const int base = m.nwg * m.nfull;  // first of the tiles cut into runs
     const long long total = (long long)((m.ntile - base + m.grp - 1) / m.grp) * m.ext;
-    long long r = (long long)g * m.run, pos = r, end = min(r + m.run, total);
+    // runs slot/grp, slot/grp + ngrp, ... of this XCD's share
+    int i = slot / m.grp - ngrp;
+    long long pos = 0, end = 0;
     for (int f = 0;;) {
         int tile, k0, k1;
         if (f < m.nfull) {
@@ -936,9 +939,10 @@ __device__ __forceinline__ void march_items(const March& m, int lp, F&& item) {
             k1 = lp;
         } else {
             if (pos >= end) {
-                if (pos == r || (r += (long long)ngrp * m.run) >= total) break;
-                pos = r;
-                end = min(r + m.run, total);
+                if ((i += ngrp) >= m.share) break;
+                pos = (long long)(xcd * m.share + i) * m.run;
+                end = min(pos + m.run, total);
+                if (pos >= end) break;
             }
             const int tt = (int)(pos / m.ext);
             const long long t0 = (long long)tt * m.ext, stop = min(end, t0 + m.ext);
@@ -956,20 +960,23 @@ __device__ __forceinline__ void march_items(const March& m, int lp, F&& item) {
 // neighbours, as a share of a plane's time (any value from 0.06 to 0.25 gives
 // the same plans; without it 256x256x128 takes 252 us instead of 233).
 constexpr double kAlone = 0.12;
-// The plan for `slots` resident workgroups (chunk > 0: runs of that length),
-// with the group of least modelled time: the planes the busiest workgroup
-// marches, dearer the fewer neighbours share their halo columns in L2.
 constexpr int kLead = 4;  // as measured: 3 to 5 the same, 2 and 7 take 59^3 from 23.1 to 25.2 us
-// Planes the busiest workgroup of a plan marches.
-inline long long march_cost(const Geo& g, const March& m) {
-    const long long cut = m.ntile > m.nwg * m.nfull ? m.run + m.lead : 0;
-    return (long long)m.nfull * (g.lp + m.lead) + cut;
-}
-inline double march_time(const Geo& g, const March& m) {
-    return (double)march_cost(g, m) * (1 + kAlone / m.grp);
-}
+// By how much chunks have to be the better plan (below 1.07 the model is no
+// longer right about which is: 1000x16x16 and 182x10x3 lose 2 to 11 % with
+// chunks that it puts 1 to 5 % ahead).
+constexpr double kChunks = 1.07;
+// The plan for `slots` resident workgroups (chunk > 0: runs of that length) of
+// least modelled time, which goes to *time: the planes the busiest workgroup
+// marches, dearer the fewer neighbours share their halo columns in L2.  The
+// tiles that remain after the whole-tile rounds are cut, in groups of any size,
+// either into equal runs of the line of tiles or each into q equal chunks.  A
+// run crosses from one tile into the next, so that its length can be anything,
+// but pays the lead planes on top; a chunk does not, and a whole tile (q = 1)
+// on open lids marches two planes less than that.  On shallow domains this
+// decides: 57x872x6, standard, 219 tiles of 32x16 for 256 CUs: 39.2 us in
+// equal runs, 25.7 with a whole tile each.
 template <int RX, int RY>
-March plan_march(const Geo& g, long long slots, int chunk) {
+March plan_march(const Geo& g, long long slots, int chunk, double* time = nullptr) {
     March m{};
     m.ntx = (g.np + RX - 5) / (RX - 4);
     m.ntile = m.ntx * ((g.mp + RY - 5) / (RY - 4));
@@ -978,30 +985,54 @@ March plan_march(const Geo& g, long long slots, int chunk) {
     if (chunk > 0) {
         m.run = std::min(chunk, g.lp);
         m.ext = (g.lp + m.run - 1) / m.run * m.run;
-        m.nwg = (int)std::min(slots, (long long)m.ntile * (m.ext / m.run));
+        const long long need = (long long)m.ntile * (m.ext / m.run);
+        m.nwg = (int)std::min(slots, need);
         if (m.nwg > NXCD) m.nwg = (m.nwg + NXCD - 1) / NXCD * NXCD;
+        m.share = (int)(m.nwg >= NXCD ? (need + NXCD - 1) / NXCD : need);
         return m;
     }
-    m.nfull = (int)(m.ntile / slots);
-    m.lead = kLead;
-    m.ext = g.lp + kLead;
-    const long long rest = m.ntile - m.nfull * slots;
+    const int nslots = (int)slots, lp = g.lp;
+    m.nfull = m.ntile / nslots;
+    const int rest = m.ntile - m.nfull * nslots;
     March best{};
+    double best_time = 0;
     for (int grp = 1; grp <= 64; grp *= 2) {
-        if (grp > 1 && (grp > rest || slots % (NXCD * grp))) break;
-        const long long units = (rest + grp - 1) / grp * m.ext, ngrp = slots / grp;
+        if (grp > 1 && (grp > rest || nslots % (NXCD * grp))) break;
+        const int groups = (rest + grp - 1) / grp, ngrp = nslots / grp;
         m.grp = grp;
-        m.run = (int)std::max(1LL, (units + ngrp - 1) / ngrp);
-        long long nwg = slots;
-        if (m.nfull == 0) {  // no more workgroups than runs, whole groups on every XCD
-            const long long need = (units + m.run - 1) / m.run * grp, per = (long long)NXCD * grp;
-            if (grp > 1 || need > NXCD) nwg = std::min(slots, (need + per - 1) / per * per);
-            else nwg = need;
+        for (int q = 0; q <= std::min(8, lp); q++) {  // q chunks a tile; 0: equal runs
+            if (q == 1 && grp > 1) continue;  // whole tiles lie side by side in any case
+            double t = m.nfull * (double)(lp + kLead);
+            if (q == 0) {
+                m.lead = kLead;
+                m.ext = lp + kLead;
+                m.run = (int)std::max(1LL, ((long long)groups * m.ext + ngrp - 1) / ngrp);
+                t = (t + (rest ? m.run + kLead : 0)) * (1 + kAlone / grp);
+            } else {
+                m.lead = 0;
+                m.run = (lp + q - 1) / q;
+                m.ext = m.run * q;
+                const int rounds = (groups * q + ngrp - 1) / ngrp;
+                t += (double)rounds * (m.run + (q == 1 && !g.pz ? 2 : kLead));
+                t *= kChunks * (1 + kAlone / (q == 1 ? std::max(rest, 1) : grp));
+            }
+            if (best.grp && t >= best_time) continue;
+            best = m;
+            best_time = t;
         }
-        m.nwg = (int)nwg;
-        if (best.grp == 0 || march_time(g, m) < march_time(g, best)) best = m;
     }
-    return best;
+    m = best;
+    const long long runs = ((long long)(rest + m.grp - 1) / m.grp * m.ext + m.run - 1) / m.run;
+    long long nwg = slots;
+    if (m.nfull == 0) {  // no more workgroups than runs, whole groups on every XCD
+        const long long need = runs * m.grp, per = (long long)NXCD * m.grp;
+        if (m.grp > 1 || need > NXCD) nwg = std::min(slots, (need + per - 1) / per * per);
+        else nwg = need;
+    }
+    m.nwg = (int)nwg;
+    m.share = (int)(nwg >= NXCD ? (runs + NXCD - 1) / NXCD : runs);
+    if (time) *time = best_time;
+    return m;
 }
 
 // Halo cells of x_out that the step does not define keep their x_in values:
@@ -1158,8 +1189,9 @@ struct Tiling {
 // steps of 64x64x32 from 235 to 313 us).
 template <int RX, int RY>
 double tiling_time(const Geo& g, int ncu, int per_cu) {
-    const March m = plan_march<RX, RY>(g, (long long)ncu * per_cu, 0);
-    return march_time(g, m) * std::max(0.69, RX * RY * per_cu / 1024.0);
+    double time = 0;
+    plan_march<RX, RY>(g, (long long)ncu * per_cu, 0, &time);
+    return time * std::max(0.69, RX * RY * per_cu / 1024.0);
 }
 
 // Tiling of a single-domain step, the one of least modelled time.  32x32

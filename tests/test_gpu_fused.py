@@ -159,3 +159,60 @@ def test_runs_cover_the_domain(mp, size, variant):
         d.step_oop(t["x"], xo, *args, **kw)
         a, b = to_host(xs), to_host(xo)
     assert bits_equal(a, b), describe_diff(a, b)
+
+
+SHALLOW = [(57, 872, 6), (256, 256, 8), (800, 40, 10), (512, 512, 3), (1500, 16, 16)]
+
+
+@pytest.mark.parametrize("variant,path", [("gauge", "PATH_FUSED"), ("standard", "PATH_FUSED")])
+@pytest.mark.parametrize("size", SHALLOW)
+def test_chunks_cover_the_domain(mp, variant, path, size):
+    """Shallow domains, whose tiles are cut into equal chunks (or not at all):
+    fewer runs than workgroups, more tiles than workgroups, several chunks a
+    tile.  The stage kernels' bits, every cell written."""
+    c = _case(size + (1,), sum(size), np.float64)
+    with mp.Domain(*size, 1) as d:
+        t = {k: to_dev(v) for k, v in c.items()}
+        kw = dict(variant=mp.GAUGE if variant == "gauge" else mp.STANDARD)
+        xs = t["x"].clone()
+        xo = torch.full_like(t["x"], float("nan"))
+        args = (t["u1"], t["u2"], t["u3"], t["rhr"], t["h"], t["bcx"], t["bcy"])
+        d.set_path(mp.PATH_STAGES)
+        d.step(xs, *args, **kw)
+        d.set_path(getattr(mp, path))
+        print(f"chunks {variant} {size}", flush=True)
+        d.step_oop(t["x"], xo, *args, **kw)
+        a, b = to_host(xs), to_host(xo)
+    assert bits_equal(a, b), describe_diff(a, b)
+
+
+@pytest.mark.parametrize("size", [(57, 872, 6), (256, 256, 8), (1500, 16, 8), (800, 40, 10)])
+def test_shallow_domains_take_whole_tiles(mp, size, monkeypatch):
+    """The standard step on shallow domains, where recomputing planes at the
+    ends of runs costs more than cutting the work evenly gains, is about as
+    fast as with a chunk prescribed: the whole depth, or half of it."""
+    c = _case(size + (1,), sum(size), np.float64)
+    with mp.Domain(*size, 1) as d:
+        t = {k: to_dev(v) for k, v in c.items()}
+        xo = torch.empty_like(t["x"])
+        args = (t["u1"], t["u2"], t["u3"], t["rhr"], t["h"], t["bcx"], t["bcy"])
+        us = {}
+        for _ in range(5):  # in turn
+            for chunk in (0, (size[2] + 1) // 2, size[2]):
+                if chunk:
+                    monkeypatch.setenv("MPDATA_FUSED_CFG", "1")
+                    monkeypatch.setenv("MPDATA_FUSED_CHUNK", str(chunk))
+                else:
+                    monkeypatch.delenv("MPDATA_FUSED_CFG", raising=False)
+                    monkeypatch.delenv("MPDATA_FUSED_CHUNK", raising=False)
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                d.step_oop(t["x"], xo, *args, variant=mp.STANDARD)
+                a.record()
+                for _ in range(100):
+                    d.step_oop(t["x"], xo, *args, variant=mp.STANDARD)
+                b.record()
+                b.synchronize()
+                us.setdefault(chunk, []).append(a.elapsed_time(b) * 10)
+    us = {k: min(v) for k, v in us.items()}
+    print(f"{size}: us by chunk (0: the rule) {us}", flush=True)
+    assert us[0] < 1.12 * min(us.values()), us
