@@ -285,9 +285,9 @@ int rho_check(mpdata_ctx* c, int liner, const void* u1, const void* u2, const vo
 // The density step after the predictor (:104-622 without the driver call),
 // arguments checked by rho_check.  a1..a3: the velocities it advects with,
 // u1..u3 themselves or, for the fused step, arrays of the context
-// (rho_velocity): then the mass fluxes go to u1..u3 directly.  ox(.,2) = ox(.,0)*h (:104-108) is not
-// repeated here: the driver's level rotation has just written the same
-// products.
+// (own_velocity): then the mass fluxes go to u1..u3 directly.  ox(.,2) =
+// ox(.,0)*h (:104-108) is not repeated here: the driver's level rotation has
+// just written the same products.
 template <typename T>
 int rho_run(mpdata_ctx* c, int liner, T* a1, T* a2, T* a3, T* u1, T* u2, T* u3, T* x, T* xinc,
             const T* h, T* rhoadv, T* rhr, const T* pexe, T* pexr1, T* pexr2, const T* bcx, const T* bcy,
@@ -359,24 +359,15 @@ int rho_run(mpdata_ctx* c, int liner, T* a1, T* a2, T* a3, T* u1, T* u2, T* u3, 
     return MPDATA_OK;
 }
 
-// Where the predictor of the whole routine puts the velocities: for the fused
-// step after a fixed-step prediction into arrays of the context, so that the
-// step's mass fluxes go to u1..u3 with no copy back (six arrays less: 119 ->
-// 30 us of copying at 256x256x128 in FP64).  With substeps or an adaptive
-// step the driver may stop with an error and leaves its last prediction in
-// u1..u3, and a vertical split also halves the halo faces of u3: they keep
-// u1..u3 as the predictor's arrays.
-template <typename T>
-int rho_velocity(mpdata_ctx* c, int liner, int lsub, int ladapt, int lvs, T** a,
-                 hipStream_t s) {
-    const bool fused = !liner && c->path != MPDATA_PATH_STAGES && rho_fusable(c->g);
-    if (!fused || lsub || ladapt || lvs) return MPDATA_OK;
-    int rc;
-    for (int d = 0; d < 3; d++) {
-        if ((rc = ensure(c, &c->prim.f[d], FACEX + d, sizeof(T), s))) return rc;
-        a[d] = (T*)c->prim.f[d];
-    }
-    return MPDATA_OK;
+// Whether the predictor of the whole routine puts the velocities into arrays
+// of the context (Driver::faces): for the fused step after a fixed-step
+// prediction, so that the step's mass fluxes go to u1..u3 with no copy back
+// (six arrays less: 119 -> 30 us of copying at 256x256x128 in FP64).  With
+// substeps or an adaptive step the driver may stop with an error and leaves
+// its last prediction in u1..u3, and a vertical split also halves the halo
+// faces of u3: they keep u1..u3 as the predictor's arrays.
+bool own_velocity(const mpdata_ctx* c, int liner, int lsub, int ladapt, int lvs) {
+    return !liner && c->path != MPDATA_PATH_STAGES && rho_fusable(c->g) && !lsub && !ladapt && !lvs;
 }
 
 constexpr int kMaxTries = 1000;
@@ -403,6 +394,20 @@ struct Driver {
     hipStream_t s;
     T dt_ratio = T(1);
     T cr[7] = {};
+    bool own = false;  // the velocities go to arrays of the context
+
+    // The arrays of the C-grid velocities.  A new context's are allocated here,
+    // with the extrapolation already queued.
+    int faces() {
+        if (!own) return MPDATA_OK;
+        T** u[3] = {&u1, &u2, &u3};
+        int rc;
+        for (int d = 0; d < 3; d++) {
+            if ((rc = ensure(c, &c->prim.f[d], FACEX + d, sizeof(T), s))) return rc;
+            *u[d] = (T*)c->prim.f[d];
+        }
+        return MPDATA_OK;
+    }
 
     int traj0(T dtv) {  // module_velprd.f90:15-89
         const Geo& g = c->g;
@@ -421,12 +426,16 @@ struct Driver {
         k_extrap_rotate<T><<<plane_grid(g, 6), kPlaneThreads, 0, s>>>(
             g, ox, oy, oz, u, v, w, h, dtv * dxi, dtv * dyi, dtv * dzi, dt_ratio);
         HIPCHK(hipGetLastError());
+        int rc;
+        if ((rc = faces())) return rc;
         HIPCHK(Stages<T>::a_to_c(g, ox + n, oy + n, oz + n, u1, u2, u3, s));
         rotated = true;
         return MPDATA_OK;
     }
     int a_to_c() {
         const long long n = len_of<SCAL>(c->g);
+        int rc;
+        if ((rc = faces())) return rc;
         HIPCHK(Stages<T>::a_to_c(c->g, ox + n, oy + n, oz + n, u1, u2, u3, s));
         return MPDATA_OK;
     }
@@ -444,7 +453,8 @@ struct Driver {
 template <typename T>
 int driver_impl(mpdata_ctx* c, int* nsub, int* nsubo, int lsub, T* dtn, T* dtnold, int ladapt,
                 int lvs, int lnph, T crmaxlim, T dtmax, T* ox, T* oy, T* oz, T* u, T* v, T* w,
-                T* u1, T* u2, T* u3, const T* h, T dxi, T dyi, T dzi, T dt, hipStream_t s) {
+                T* u1, T* u2, T* u3, const T* h, T dxi, T dyi, T dzi, T dt, hipStream_t s,
+                bool own = false) {
     if (any_null(nsub, nsubo, dtn, dtnold, ox, oy, oz, u, v, w, u1, u2, u3, h))
         return fail(MPDATA_EINVAL, "predictor driver: null argument");
     if (lsub && ladapt)
@@ -453,6 +463,7 @@ int driver_impl(mpdata_ctx* c, int* nsub, int* nsubo, int lsub, T* dtn, T* dtnol
     if (lsub && (*nsub < 1 || *nsubo < 1))
         return fail(MPDATA_EINVAL, "nsubsteps %d, nsubsteps_o %d must be >= 1", *nsub, *nsubo);
     Driver<T> d{c, ox, oy, oz, u1, u2, u3, h, dxi, dyi, dzi, s};
+    d.own = own;
     int rc;
     T dtntemp = *dtn;
     if (lsub && *nsub == 1) d.dt_ratio = (dt / T(1)) / (dt / (T)*nsubo);  // :73
@@ -593,15 +604,14 @@ extern "C" {
         if ((rc = rho_check(ctx, liner, u1, u2, u3, x_in, x_incomp, h, rhoadv, rhr, pexe, pexr1, \
                             pexr2, bcx, bcy)))                                                   \
             return rc;                                                                           \
-        T* a[3] = {u1, u2, u3};                                                                  \
-        if ((rc = rho_velocity<T>(ctx, liner, lsubstepping, ltimeadapt, lvertsplit, a,           \
-                                  (hipStream_t)stream)))                                        \
-            return rc;                                                                           \
+        const bool own = own_velocity(ctx, liner, lsubstepping, ltimeadapt, lvertsplit);         \
         if ((rc = driver_impl<T>(ctx, nsubsteps, nsubsteps_o, lsubstepping, dtn, dtnold,         \
                                  ltimeadapt, lvertsplit, lcrdiag_nphlf, crmaxlim, dtmax, ox, oy, \
-                                 oz, u, v, w, a[0], a[1], a[2], h, dxi, dyi, dzi, dt,            \
-                                 (hipStream_t)stream)))                                          \
+                                 oz, u, v, w, u1, u2, u3, h, dxi, dyi, dzi, dt,                  \
+                                 (hipStream_t)stream, own)))                                     \
             return rc;                                                                           \
+        T* a[3] = {u1, u2, u3};                                                                  \
+        for (int d = 0; d < 3 && own; d++) a[d] = (T*)ctx->prim.f[d];                            \
         return rho_run<T>(ctx, liner, a[0], a[1], a[2], u1, u2, u3, x_in, x_incomp, h, rhoadv,   \
                           rhr, pexe, pexr1, pexr2, bcx, bcy, (hipStream_t)stream);               \
     }

@@ -300,3 +300,37 @@ def test_compute_courants_equals_oracle(mp, tdt, npdt, level):
         got = d.compute_courants(to_dev(f["ox"]), to_dev(f["oy"]), to_dev(f["oz"]),
                                  to_dev(f["h"]), level, f["dxi"], f["dyi"], f["dzi"], f["dt"])
     assert [npdt(v) for v in got] == [npdt(v) for v in want], (got, want)
+
+
+def test_first_call_allocates_behind_the_predictor(mp):
+    """On a new context the whole routine takes no longer than the driver and
+    the core called one after the other, which allocate while the predictor
+    runs: its own allocations follow the extrapolation."""
+    import time
+    dims = (160, 160, 80, 1)
+    f = _case(dims, 7, 0.5, np.float64)
+    g = {k: to_dev(v) for k, v in f.items() if isinstance(v, np.ndarray)}
+    sp = (f["dxi"], f["dyi"], f["dzi"], f["dt"])
+
+    def whole(d, st):
+        d.rho_gauge_gpubc(st, *[g[k] for k in FIELDS], *sp)
+
+    def split(d, st):
+        d.velprd_driver(st, *[g[k] for k in ("ox", "oy", "oz", "u", "v", "w", "u1", "u2", "u3",
+                                             "h")], *sp)
+        d.rho_gauge_core(*[g[k] for k in ("u1", "u2", "u3", "x_in", "x_incomp", "h", "rhoadv",
+                                          "rhr", "pexe", "pexr1", "pexr2", "bcx", "bcy")])
+
+    us = {"whole": [], "split": []}
+    for _ in range(40):  # in turn, each on a context of its own
+        for name, call in (("whole", whole), ("split", split)):
+            st = dict(nsubsteps=1, nsubsteps_o=1, dtn=f["dt"], dtnold=f["dt"])
+            with mp.Domain(*dims) as d:
+                torch.cuda.synchronize()
+                t0 = time.perf_counter()
+                call(d, st)
+                torch.cuda.synchronize()
+                us[name].append((time.perf_counter() - t0) * 1e6)
+    us = {k: float(np.median(v[5:])) for k, v in us.items()}
+    print(f"first density call on a new context: {us}", flush=True)
+    assert us["whole"] <= 1.02 * us["split"], us
