@@ -19,8 +19,8 @@ bool Fused<T>::supports(const Geo& g, int variant, int iters, int nonos) {
     // 32-bit element offsets inside the kernel, and 32-bit byte offsets
     // inside one plane of every array
     const long long biggest = len_of<FACEX>(g) > len_of<FACEY>(g) ? len_of<FACEX>(g) : len_of<FACEY>(g);
-    const Off o = make_off(g);
-    const long long plane = std::max(std::max((long long)o.sxy, (long long)o.fxy), (long long)o.yxy);
+    const long long plane =
+        std::max(nx_of<FACEX>(g) * ny_of<FACEX>(g), nx_of<FACEY>(g) * ny_of<FACEY>(g));
     return biggest < (1ll << 31) - 1 && len_of<FACEZ>(g) < (1ll << 31) - 1 &&
            plane * (long long)sizeof(T) < (1ll << 32);
 }

@@ -65,6 +65,15 @@ __device__ __forceinline__ void sto(T* p, uint32_t off, T v) {
     *(__attribute__((address_space(1))) T*)((G)p + off) = v;
 }
 
+// Bytes of a plane of n elements.  Planes are below 4 GiB (Fused::supports):
+// from 2 GiB on the product does not fit an int.
+template <typename T>
+__host__ __device__ constexpr uint32_t plane_bytes(int n) {
+    return uint32_t(n) * uint32_t(sizeof(T));
+}
+// (evaluated at compile time, where a signed overflow is an error)
+static_assert(plane_bytes<double>(1 << 28) == 0x80000000u && plane_bytes<float>(1 << 29) == 0x80000000u);
+
 // A value that is the same in every lane, in scalar registers: the compiler
 // cannot tell where it comes from memory that the kernel might write.
 template <typename S>
@@ -431,7 +440,7 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
     };
     uint32_t so_k = so, fo_k = fo;
     // planes of the newest queue slots, and the planes' sizes in bytes
-    const uint32_t SB8 = SXY * SZ, FB8 = FXY * SZ, YB8 = YXY * SZ;
+    const uint32_t SB8 = plane_bytes<T>(SXY), FB8 = plane_bytes<T>(FXY), YB8 = plane_bytes<T>(YXY);
     const T* qx = uniform(pl(x, SXY, kc(Ks + 1)));
     const T* qu1 = uniform(pl(u1, FXY, kc(Ks)));
     const T* qu2 = uniform(pl(u2, YXY, kc(Ks)));

@@ -311,7 +311,7 @@ __device__ __forceinline__ void fused_std_item(const Geo& g, const Off& o, int n
         if constexpr (TAPE) return min3(T(1), a, b);
         else return min2(a, b);
     };
-    const uint32_t SB8 = SXY * SZ, FB8 = FXY * SZ, YB8 = YXY * SZ;
+    const uint32_t SB8 = plane_bytes<T>(SXY), FB8 = plane_bytes<T>(FXY), YB8 = plane_bytes<T>(YXY);
     const T* qx = uniform(pl(x, SXY, kc(Ks + 1)));
     const T* qu1 = uniform(pl(u1, FXY, kc(Ks)));
     const T* qu2 = uniform(pl(u2, YXY, kc(Ks)));

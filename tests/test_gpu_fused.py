@@ -216,3 +216,30 @@ def test_shallow_domains_take_whole_tiles(mp, size, monkeypatch):
     us = {k: min(v) for k, v in us.items()}
     print(f"{size}: us by chunk (0: the rule) {us}", flush=True)
     assert us[0] < 1.12 * min(us.values()), us
+
+
+@pytest.mark.parametrize("variant", ["gauge", "standard"])
+def test_planes_above_2_gib(mp, variant):
+    """Planes of 2.15 GB, whose size in bytes does not fit a signed int: at
+    rest (zero velocity, unit density) the step returns its input."""
+    size = (16400, 16384, 3)
+    dev = torch.device("cuda:0")
+    with mp.Domain(*size, 1) as d:
+        d.set_path(mp.PATH_FUSED)
+        x = torch.arange(1, 1 + d.zeros(0).numel(), dtype=torch.float64, device=dev)
+        x = x.remainder_(8191.0).add_(1.0).view(*d.shape(0))
+        one = torch.ones_like(x)
+        u = [d.zeros(k) for k in (1, 2, 3)]
+        bcx = torch.ones((2, 3, size[1]), dtype=torch.float64, device=dev)
+        bcy = torch.ones((2, 3, size[0]), dtype=torch.float64, device=dev)
+        xo = torch.full_like(x, float("nan"))
+        print(f"planes above 2 GiB {variant}", flush=True)
+        d.step_oop(x, xo, *u, one, one, bcx, bcy,
+                   variant=mp.GAUGE if variant == "gauge" else mp.STANDARD)
+        torch.cuda.synchronize()
+        i = (slice(1, -1),) * 3
+        assert bool((xo[i] == x[i]).all())
+        assert bool((xo[0] == x[0]).all()) and bool((xo[-1] == x[-1]).all())
+        assert bool((xo[1:-1, 1:-1, 0] == x[1:-1, 1:-1, 1]).all())
+    del x, xo, one, u
+    torch.cuda.empty_cache()
