@@ -549,12 +549,13 @@ __device__ __forceinline__ void adj_face_gauge(R* L, R vb, R x1, R x2, R a, R r,
 // GAUGE: the gauge variant's pseudo-velocities, whose adjoint a.v already
 // holds the limiter's part; else the standard variant's, with the adjoint
 // a.f of their donor fluxes.
-// Four waves a SIMD (128 VGPRs; the standard variant wants 136 and spills a
-// few): at 128x128x64 the grid is four blocks a CU, one round instead of one
-// and a third (88 -> 84 us; summing a thread's contributions in registers
-// first, 34 LDS atomics instead of 57, took 167 VGPRs and 94 us).
-template <bool GAUGE>
-__global__ void __launch_bounds__(PBX * PBY, 4) k_adj_pseudo(Geo g, const R* __restrict__ u1,
+// FOUR: bounded to four waves a SIMD, for grids of more than three and at most
+// four blocks a CU (four_blocks).  The standard variant wants 136 VGPRs, three
+// waves, and spills a few at 128; the gauge variant stays below in any case.
+// (Summing a thread's contributions in registers first, 34 LDS atomics instead
+// of 57, took 167 VGPRs and 94 us for 88.)
+template <bool GAUGE, bool FOUR>
+__global__ void __launch_bounds__(PBX * PBY, FOUR ? 4 : 1) k_adj_pseudo(Geo g, const R* __restrict__ u1,
                                                           const R* __restrict__ u2,
                                                           const R* __restrict__ u3,
                                                           const R* __restrict__ psi,
@@ -1052,6 +1053,21 @@ int mpdata_adj_record_f64(mpdata_ctx* c, int slot, const double* x_in, double* x
 
 namespace {
 
+// Whether a grid of one-wave-a-SIMD blocks runs in one round of four blocks a
+// CU but not in one of three.  There the four-waves bound pays for its spills,
+// elsewhere it does not: gradients of ten standard steps take 1 to 2 % less
+// with it from 128x128x52 to 128x128x64, at 64x256x64 and at 128x64x128, and 1
+// to 4 % more at 64x64x32, 160x100x40, 96x96x96, 128x128x68 to 128x128x128 and
+// 200x200x64.
+bool four_blocks(const dim3& grid) {
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return false;
+    const long long nb = (long long)grid.x * grid.y * grid.z;
+    return nb > 3LL * ncu && nb <= 4LL * ncu;
+}
+
 // reverse of the antidiffusive iteration (limited fluxes, limiter,
 // pseudo-velocities) of the recorded step in `t`, standard or gauge variant
 template <bool GAUGE>
@@ -1065,8 +1081,11 @@ void adj_reverse_antidiff(const Geo& g, const TapeSlot& t, const R* u1, const R*
     k_adj_flux<GAUGE><<<fgrid, dim3(BX, BY, 1), 0, s>>>(g, v0, v1, v2, cp, cn, psi, rhr, h, a);
     k_adj_limiter<GAUGE><<<fgrid, dim3(BX, BY, 1), 0, s>>>(g, (const R*)t.x0, psi, h, v0, v1, v2,
                                                             cp, cn, a);
-    k_adj_pseudo<GAUGE><<<pgrid, dim3(PBX, PBY, 1), 0, s>>>(g, u1, u2, u3, psi, h, v0, v1, v2,
-                                                             ubar1, ubar2, ubar3, a);
+    auto* pseudo = k_adj_pseudo<GAUGE, false>;
+    if constexpr (!GAUGE)
+        if (four_blocks(pgrid)) pseudo = k_adj_pseudo<GAUGE, true>;
+    pseudo<<<pgrid, dim3(PBX, PBY, 1), 0, s>>>(g, u1, u2, u3, psi, h, v0, v1, v2, ubar1, ubar2,
+                                                ubar3, a);
 }
 
 }  // namespace

@@ -412,3 +412,32 @@ def test_tape_replaced_between_forward_and_backward(mpd):
             grads.append([leaf.grad.detach().clone() for leaf in leaves])
     for g0, g1 in zip(*grads):
         assert torch.allclose(g1, g0, rtol=1e-12, atol=1e-14 * float(g0.abs().max()))
+
+
+@pytest.mark.parametrize("dims", [(130, 66, 68, 1), (128, 128, 68, 1)])
+def test_dot_product_block_counts(mpd, dims):
+    """The dot-product test on grids of 867 and 1088 blocks of the reverse
+    pseudo-velocity kernel (between three and four a CU of 256, and more)."""
+    c = _case(dims, 41)
+    d = {k: to_dev(v) for k, v in c.items()}
+    rng = np.random.default_rng(19)
+    dxn = _zero_halo(rng.standard_normal(c["x"].shape))
+    dun = [rng.standard_normal(c[k].shape) for k in ("u1", "u2", "u3")]
+    ybar = _zero_halo(rng.standard_normal(c["x"].shape))
+    with mpd.Domain(*dims) as dom:
+        x, dx = d["x"].clone(), to_dev(dxn)
+        du = [to_dev(v) for v in dun]
+        print(f"dot product at {dims}", flush=True)
+        dom.tl_step(x, dx, d["u1"], d["u2"], d["u3"], *du, d["rhr"], d["h"], d["bcx"], d["bcy"],
+                    variant=mpd.STANDARD, iters=2, nonos=1)
+        tl = to_host(dx)[I]
+        grads, _ = _adjoint_chain(mpd, dom, d, 1, ybar)
+    lhs = float((tl * ybar[I]).sum())
+    rhs = float((dxn[I] * grads[0][I]).sum()) + sum(float((a * b).sum())
+                                                    for a, b in zip(dun, grads[1:]))
+    # rounding of sums of N products: some eps * sqrt(N) of the norms' product,
+    # over N (1e6) independent terms; 1e-13 of it is a thousand times that
+    scale = float(np.linalg.norm(tl) * np.linalg.norm(ybar[I]))
+    print(f"  <TL,y>={lhs:.15e} <x,AD>={rhs:.15e} difference / norms {abs(lhs - rhs) / scale:.1e}",
+          flush=True)
+    assert abs(lhs - rhs) <= 1e-13 * scale
