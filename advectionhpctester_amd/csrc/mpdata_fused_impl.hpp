@@ -938,8 +938,9 @@ __device__ __forceinline__ void march_items(const March& m, int lp, F&& item) {
     const int base = m.nwg * m.nfull;  // first of the tiles cut into runs
     const long long total = (long long)((m.ntile - base + m.grp - 1) / m.grp) * m.ext;
     // runs slot/grp, slot/grp + ngrp, ... of this XCD's share
-    int i = slot / m.grp - ngrp;
-    long long pos = 0, end = 0;
+    int i = slot / m.grp;
+    long long pos = (long long)(xcd * m.share + i) * m.run, end = min(pos + m.run, total);
+    if (i >= m.share) end = 0;
     for (int f = 0;;) {
         int tile, k0, k1;
         if (f < m.nfull) {
