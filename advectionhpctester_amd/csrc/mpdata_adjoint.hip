@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 
 #include "../../include/mpdata_hip.h"
 #include "mpdata_ctx.hpp"
@@ -916,15 +917,29 @@ int check_adj(mpdata_ctx* c) {
     return MPDATA_OK;
 }
 
-int ensure_slot(mpdata_ctx* c, TapeSlot& t, hipStream_t s) {
+struct TapeArray {
+    void** p;
+    int kind;
+};
+std::array<TapeArray, 8> tape_arrays(TapeSlot& t) {
+    return {{{&t.xb, SCAL}, {&t.x0, SCAL}, {&t.psi, SCAL}, {&t.cp, SCAL}, {&t.cn, SCAL},
+             {&t.v[0], FACEX}, {&t.v[1], FACEY}, {&t.v[2], FACEZ}}};
+}
+int reserve_slot(mpdata_ctx* c, TapeSlot& t) {
     int rc;
-    if ((rc = ensure(c, &t.xb, SCAL, 8, s)) || (rc = ensure(c, &t.x0, SCAL, 8, s)) ||
-        (rc = ensure(c, &t.psi, SCAL, 8, s)) || (rc = ensure(c, &t.cp, SCAL, 8, s)) ||
-        (rc = ensure(c, &t.cn, SCAL, 8, s)))
-        return rc;
-    for (int d = 0; d < 3; d++)
-        if ((rc = ensure(c, &t.v[d], FACEX + d, 8, s))) return rc;
+    for (const TapeArray& a : tape_arrays(t))
+        if ((rc = ensure_memory(c, a.p, a.kind, 8))) return rc;
     return MPDATA_OK;
+}
+// A reserved slot for use on stream s: cleared by its first use, since
+// reserving it has no stream.
+hipError_t open_slot(mpdata_ctx* c, TapeSlot& t, hipStream_t s) {
+    if (t.cleared) return hipSuccess;
+    hipError_t e = hipSuccess;
+    for (const TapeArray& a : tape_arrays(t))
+        if (e == hipSuccess) e = clear_memory(*a.p, (size_t)field_len(c->g, a.kind) * 8, s);
+    t.cleared = e == hipSuccess;
+    return e;
 }
 
 }  // namespace
@@ -936,15 +951,8 @@ int mpdata_adj_reserve(mpdata_ctx* c, int nslots) {
     if (rc) return rc;
     if (nslots < 1 || nslots > 4096) return fail(MPDATA_EINVAL, "nslots %d outside 1..4096", nslots);
     if ((int)c->tape.size() < nslots) c->tape.resize(nslots);
-    // new slots are clear when the call returns, whatever stream records into
-    // them; v[2] is the last array a slot gets
-    ClearStream own;
-    for (int q = 0; q < nslots; q++) {
-        TapeSlot& t = c->tape[q];
-        if (t.v[2]) continue;
-        HIPCHK(own.open());
-        if ((rc = ensure_slot(c, t, own.s))) return rc;
-    }
+    for (int q = 0; q < nslots; q++)
+        if ((rc = reserve_slot(c, c->tape[q]))) return rc;
     return MPDATA_OK;
 }
 
@@ -969,6 +977,7 @@ int mpdata_adj_record_variant_f64(mpdata_ctx* c, int slot, int variant, const do
     Scratch& S = c->prim;
     TapeSlot& t = c->tape[slot];
     hipStream_t s = (hipStream_t)stream;
+    HIPCHK(open_slot(c, t, s));
     using St = Stages<R>;
     R *xb = (R*)t.xb, *x0 = (R*)t.x0, *psi = (R*)t.psi, *cp = (R*)t.cp, *cn = (R*)t.cn;
     R* v[3];
@@ -1111,7 +1120,8 @@ int mpdata_adj_step_f64(mpdata_ctx* c, int slot, const double* u1, const double*
     Adj a{(R*)c->adj[pcur], (R*)c->adj[pnext], (R*)c->adj[A_X0], (R*)c->adj[A_CP],
           (R*)c->adj[A_CN], (R*)c->adj[A_V1], (R*)c->adj[A_V2], (R*)c->adj[A_V3],
           (R*)c->adj[A_F1], (R*)c->adj[A_F2], (R*)c->adj[A_F3], xbar, ufac};
-    const TapeSlot& t = c->tape[slot];
+    TapeSlot& t = c->tape[slot];
+    HIPCHK(open_slot(c, t, s));
     HIPCHK(hipGetLastError());
     if (t.variant == MPDATA_GAUGE)
         adj_reverse_antidiff<true>(g, t, u1, u2, u3, rhr, h, ubar1, ubar2, ubar3, a, s);

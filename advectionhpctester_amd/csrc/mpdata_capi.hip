@@ -50,7 +50,7 @@ long long field_len(const Geo& g, int kind) {
     }
 }
 
-int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes, hipStream_t s) {
+int ensure_memory(mpdata_ctx* c, void** slot, int kind, int elem_bytes) {
     if (*slot) return MPDATA_OK;
     size_t bytes = (size_t)field_len(c->g, kind) * elem_bytes;
     void* p = nullptr;
@@ -60,29 +60,36 @@ int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes, hipStream_t s) 
         return fail(MPDATA_ENOMEM, "hipMalloc(%zu bytes) for scratch failed: %s", bytes,
                     hipGetErrorString(e));
     }
-    // zero once so that halo cells never read are deterministic.  On the
-    // stream that uses it: the null stream's hipMemset does not wait for the
-    // fill, and a non-blocking stream does not wait for the null stream.  Under
-    // capture the fill happens now, outside the graph.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    e = hipStreamIsCapturing(s, &cap);
-    if (e == hipSuccess && cap == hipStreamCaptureStatusNone) {
-        e = hipMemsetAsync(p, 0, bytes, s);
-    } else if (e == hipSuccess) {
-        ClearStream own;
-        e = own.open();
-        if (e == hipSuccess) e = hipMemsetAsync(p, 0, bytes, own.s);
-    }
-    if (e != hipSuccess) {
-        (void)hipFree(p);
-        return hip_fail(e, "clearing scratch");
-    }
     *slot = p;
     c->owned.push_back(p);
     c->held += (long long)bytes;
     return MPDATA_OK;
 }
 
+// Scratch is zeroed once so that halo cells never read are deterministic.  On
+// the stream that uses it: the null stream's hipMemset does not wait for the
+// fill, and a non-blocking stream does not wait for the null stream.  Under
+// capture the fill happens now, outside the graph.
+hipError_t clear_memory(void* p, size_t bytes, hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(s, &cap);
+    if (e != hipSuccess) return e;
+    if (cap == hipStreamCaptureStatusNone) return hipMemsetAsync(p, 0, bytes, s);
+    hipStream_t own = nullptr;
+    if ((e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking)) != hipSuccess) return e;
+    e = hipMemsetAsync(p, 0, bytes, own);
+    if (e == hipSuccess) e = hipStreamSynchronize(own);
+    (void)hipStreamDestroy(own);
+    return e;
+}
+
+int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes, hipStream_t s) {
+    if (*slot) return MPDATA_OK;
+    int rc;
+    if ((rc = ensure_memory(c, slot, kind, elem_bytes))) return rc;
+    HIPCHK(clear_memory(*slot, (size_t)field_len(c->g, kind) * elem_bytes, s));
+    return MPDATA_OK;
+}
 
 int check_ctx(const mpdata_ctx* c, int real_bytes) {
     if (!c) return fail(MPDATA_EINVAL, "null context");

@@ -33,6 +33,7 @@ struct TapeSlot {
     void* cp = nullptr;
     void* cn = nullptr;
     int variant = 2;        // MPDATA_STANDARD or MPDATA_GAUGE
+    bool cleared = false;   // on the stream of the slot's first use
 };
 
 }  // namespace mpdata
@@ -87,16 +88,8 @@ bool any_null(P... p) {
 // Allocates *slot (field of `kind`, elem_bytes per element) unless set, and
 // clears it on stream s, on which it is used next.
 int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes, hipStream_t s);
-// A stream of its own to clear memory on, for a caller that has no stream or
-// one under capture; the destructor waits for what was queued on it.
-struct ClearStream {
-    hipStream_t s = nullptr;
-    hipError_t open() { return s ? hipSuccess : hipStreamCreateWithFlags(&s, hipStreamNonBlocking); }
-    ~ClearStream() {
-        if (!s) return;
-        (void)hipStreamSynchronize(s);
-        (void)hipStreamDestroy(s);
-    }
-};
+// Its two halves, for memory that is allocated where there is no stream.
+int ensure_memory(mpdata_ctx* c, void** slot, int kind, int elem_bytes);
+hipError_t clear_memory(void* p, size_t bytes, hipStream_t s);
 
 }  // namespace mpdata
