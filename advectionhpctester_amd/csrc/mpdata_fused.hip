@@ -57,12 +57,11 @@ hipError_t Fused<T>::step(const Geo& g, const T* x, T* xout, const T* u1, const 
     }
 }
 
-// 32x16 tiles at 2 waves per SIMD (140 VGPRs, no spill), one workgroup
-// per CU, and the chunk of least modelled wall time.  Alone the kernel is
-// faster at 4 waves per SIMD (6 VGPRs spilled: 70.5 against 79.5 us per
-// step at 128x128x64); but the adjoint's backward runs it beside the
-// reverse kernels on another stream, and there the lighter occupancy
-// leaves them room (forward + backward 16.3-16.5 against 16.7-16.9 ms).
+// 32x16 tiles at 2 waves per SIMD (158 VGPRs, no spill), one workgroup per
+// CU, cut by the launch plan (March).  At 4 waves per SIMD it spills, and the
+// adjoint's backward runs it beside the reverse kernels on another stream,
+// where the lighter occupancy leaves them room (128x128x64, 50 steps, when the
+// tape was added: forward + backward 16.3-16.5 against 16.7-16.9 ms).
 template <typename T>
 hipError_t Fused<T>::record(const Geo& g, const T* x, T* xout, const T* u1, const T* u2,
                             const T* u3, const T* rhr, const T* h, const T* bcx, const T* bcy,
@@ -138,7 +137,10 @@ hipError_t FusedBatch<T>::step(const void* table, int n, int nitem, int cfg, lon
 }
 
 // Batch tiling for n members on one grid (configuration numbers of
-// MPDATA_BATCH_CONFIGS): the single-domain rule with n times the work items.
+// MPDATA_BATCH_CONFIGS): 32x32 tiles with chunks of 64 planes where they give
+// every CU two items, else 32x16 tiles with the longest chunk of 64, 32 or 16
+// planes that gives every workgroup slot two.  The batch takes its items
+// dynamically, so March's equal runs do not apply to it.
 template <typename T>
 void FusedBatch<T>::choose_shared(const Geo& g, int n, int& cfg, int& clen) {
     int dev = 0, ncu = 0;

@@ -18,12 +18,14 @@
 //      on face K (between planes K-1 and K),
 //   C  the limiter ratios cp,cn on plane K-1 (tile + 1-cell ring),
 //   D  the new x on plane K-2 (the tile),
-// keeping the last three xant planes and two V1/V2/cp/cn planes in LDS
-// rings and the V3 faces and the column's inputs in register queues.  Halo
-// values follow the reference's boundary semantics directly (inflow values
-// for the upwind, mirrored xant, zero wall velocities, edge-copied x for
-// the limiter, zero cp/cn halo), so no halo-fill kernels run.  Expressions are those of the per-stage kernels, operand for operand,
-// so the fused result is bit-identical to them.
+// keeping the last three xant planes in an LDS ring, one plane each of V1, V2,
+// cp and cn in LDS (plane K-2 until stage B or C replaces it by K-1) and the V3
+// faces and the column's inputs in register queues.  Halo values follow the
+// reference's boundary semantics directly (inflow values for the upwind,
+// mirrored xant, zero wall velocities, edge-copied x for the limiter, zero
+// cp/cn halo), so no halo-fill kernels run.  Expressions are those of the
+// per-stage kernels, operand for operand, so the fused result is bit-identical
+// to them.
 #pragma once
 #include "mpdata_fused.hpp"
 
@@ -168,9 +170,11 @@ __device__ __forceinline__ T div_(T a, T b) {
 // stage, hide little of a wait, and the registers (128) leave no room for
 // more.  So nothing waits inside a step but the two barriers: all loads of a
 // step are issued together after B and waited for once, before A; the store
-// of a plane is issued right after that wait; h and rhr of the plane being
-// updated are kept, not loaded again; V, the bounds and cp/cn are formed
-// straight-line by every lane, so that their LDS reads go out together.
+// of a plane is issued right after that wait (not so the extra outputs of PASS
+// 1 and of the density mode, and the latter's extra inputs, which stage D
+// still stores and loads: the next step's wait exposes them); h and rhr of the
+// plane being updated are kept, not loaded again; V, the bounds and cp/cn are
+// formed straight-line by every lane, so that their LDS reads go out together.
 // Together with the scalar plane pointers and the equal runs of March,
 // 512x512x256 went from 1.66 to 1.26 ms (fast build) and 256x256x128 from 294
 // to 232 us (exact build).
@@ -551,16 +555,10 @@ __device__ __forceinline__ void fused_item(const Geo& g, const Off& o, int ntx, 
         // V1 is formed (gi >= 2 in the domain, so the left position is in
         // the domain too), and its queues hold h, u2 and u3 of plane P:
         // taken across lanes.  Column (gi, gj-1) is likewise the source
-        // column of the position below wherever V2 is formed (gj >= 2): with
-        // XJ its h, u1 and u3 go through LDS (written in stage A, read in
-        // B); otherwise they are loaded, before stage A so that the latency
-        // overlaps it, by every lane on every plane (the plane clamped into
-        // the domain; the source column is in the domain, so its j-1
-        // neighbour is in the arrays), which costs nothing in a wave that
-        // loads anyway.
+        // column of the position below wherever V2 is formed (gj >= 2): its
+        // h, u1 and u3 go through LDS (written here, read in B).
         const int P = K - 1;
         const bool BC_on = P >= max(1, k0 - 1) && P <= min(lp, k1 + 1);
-        const int Pc = kc(P);
         const T hx = from_left_lane(hq1) + hq1;
         const T s2x = from_left_lane(u2a0 + u2b0) + u2b0 + u2a0;
         const T s3x = from_left_lane(u3q0 + u3q1) + u3q1 + u3q0;
@@ -1340,9 +1338,9 @@ size_t sched_offset(int n) {
 // neighbouring tiles together.  The items left after the run's whole
 // rounds (one item per workgroup of the XCD) are each split into up to four
 // k-ranges, so that the last round occupies the workgroups; a k-range of a
-// chunk gives the same planes as the whole chunk (8 fields of 256x256x128
-// on one grid: 2.02 -> 1.85 ms per step; in the statically scheduled
-// single-domain kernel the same split measured slower).
+// chunk gives the same planes as the whole chunk (8 fields of 256x256x128 on
+// one grid: 2.02 -> 1.85 ms per step when it was introduced).  The
+// single-domain kernels cut their tiles by March instead.
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
 __global__ void __launch_bounds__(RX * RY, MINB)
 k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int shared,

@@ -29,9 +29,10 @@
 // come from the lane to the left, those of V2 from column j-1 through LDS.
 //
 // What bounds it is the chain of a plane, as in the gauge kernel, with more of
-// it in the divisions (thirteen a cell); the same means took 384x320x192 from
-// 743 to 687 us (fast build), 190x147x83 in place from 149 to 118 us (exact)
-// and ten steps of a periodic 64x64x32 from 323 to 235 us.
+// it in the divisions (seventeen a cell).  The same means and the tiling rule
+// of std_step took 384x320x192 from 760 to 642 us (fast build), 190x147x83 in
+// place from 149 to 111 us (exact) and ten steps of a periodic 64x64x32 from
+// 323 to 234 us.
 #pragma once
 
 #include "mpdata_fused_impl.hpp"

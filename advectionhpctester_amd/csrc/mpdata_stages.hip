@@ -729,9 +729,7 @@ __global__ void __launch_bounds__(256) k_norm_sums(Geo g, const T* __restrict__ 
 // ---- host-side launchers ----------------------------------------------------
 namespace {
 inline dim3 cell_block() { return dim3(64, 4, 1); }
-inline dim3 cell_grid(const Geo& g, int extra = 0) {
-    return dim3((g.np + extra + 63) / 64, (g.mp + extra + 3) / 4, g.lp + extra);
-}
+inline dim3 cell_grid(const Geo& g) { return dim3((g.np + 63) / 64, (g.mp + 3) / 4, g.lp); }
 inline dim3 wall_block() { return dim3(64, 4, 1); }
 }  // namespace
 

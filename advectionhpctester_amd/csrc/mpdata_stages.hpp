@@ -15,7 +15,7 @@ namespace mpdata {
 // 300x300x100).  A plane's blocks come in multiples of NXCD; for a kernel that
 // reads neighbours, xcd_block gives each XCD a band of neighbouring rows, the
 // same band in every plane, so that rows j-1 and plane k-1 are in its L2
-// (velprd_c at 300x300x100: 182 us without, 160 with).
+// (velprd_c at 300x300x100: 182 us without, 163 with).
 constexpr unsigned kPlaneThreads = 256;
 inline dim3 plane_grid(const Geo& g, unsigned per_x = 1) {
     const unsigned nb = ((unsigned)g.np * (unsigned)g.mp + kPlaneThreads - 1) / kPlaneThreads;
