@@ -87,8 +87,14 @@ int ensure(mpdata_ctx* c, void** slot, int kind, int elem_bytes, hipStream_t s) 
     if (*slot) return MPDATA_OK;
     int rc;
     if ((rc = ensure_memory(c, slot, kind, elem_bytes))) return rc;
-    HIPCHK(clear_memory(*slot, (size_t)field_len(c->g, kind) * elem_bytes, s));
-    return MPDATA_OK;
+    const size_t bytes = (size_t)field_len(c->g, kind) * elem_bytes;
+    const hipError_t e = clear_memory(*slot, bytes, s);
+    if (e == hipSuccess) return MPDATA_OK;
+    (void)hipFree(*slot);
+    *slot = nullptr;
+    c->owned.pop_back();
+    c->held -= (long long)bytes;
+    return hip_fail(e, "clearing scratch");
 }
 
 int check_ctx(const mpdata_ctx* c, int real_bytes) {

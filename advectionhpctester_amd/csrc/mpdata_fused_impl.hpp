@@ -1096,10 +1096,14 @@ inline long long halo_cells(const Geo& g) {
     const long long ih = g.ih, nx = g.np + 2 * ih, ny = g.mp + 2 * ih;
     return 2 * ih * (nx * ny + nx * g.lp + (long long)g.mp * g.lp);
 }
-// blocks of nt threads for `cells` halo cells: four cells a thread, at most a
-// quarter of the chip's CUs
+// shares of four cells a thread for blocks of nt threads
+inline long long halo_shares(long long cells, int nt) {
+    return std::max(1LL, (cells + 4LL * nt - 1) / (4LL * nt));
+}
+// blocks of nt threads for `cells` halo cells: a share each, at most a quarter
+// of the chip's CUs
 inline int halo_blocks(long long cells, int nt) {
-    return (int)std::max(1LL, std::min(64LL, (cells + 4LL * nt - 1) / (4LL * nt)));
+    return (int)std::min(64LL, halo_shares(cells, nt));
 }
 
 template <typename T, int RX, int RY, int MINB, bool FAST = false, int PASS = 0>
@@ -1311,6 +1315,7 @@ struct Member {  // device descriptor of one member
     Geo g;
     Off o;
     int ntx, ntile, clen, item0;
+    int halo0;  // first of its shares of the halo copy
     const T *x, *u1, *u2, *u3, *rhr, *h, *bcx, *bcy;
     T* xo;
 };
@@ -1326,6 +1331,7 @@ struct BatchSched {
     int bnd[NXCD + 1];
     int next[NXCD];
     int done[NXCD];
+    int nhalo;  // shares of the members' halo copies
 };
 template <typename T>
 size_t sched_offset(int n) {
@@ -1344,14 +1350,26 @@ size_t sched_offset(int n) {
 template <typename T, int RX, int RY, int MINB, bool FAST = false>
 __global__ void __launch_bounds__(RX * RY, MINB)
 k_fused_gauge2_batch(const Member<T>* __restrict__ mem, int nmem, int nitem, int shared,
-                     BatchSched* __restrict__ sc, int nitemwg, int hparts) {
+                     BatchSched* __restrict__ sc, int nitemwg) {
     __shared__ FusedLds<T, RX, RY> L;
     __shared__ int s_w;
     if (blockIdx.x >= (unsigned)nitemwg) {
-        // the halo of every member in hparts shares, dealt to the blocks
-        for (int w = blockIdx.x - nitemwg; w < nmem * hparts; w += gridDim.x - nitemwg) {
-            const Member<T>& m = mem[w / hparts];
-            copy_untouched_halo<T>(m.g, m.x, m.xo, w % hparts, hparts);
+        // an equal run of the shares of all members' halos
+        const int total = sc->nhalo, nb = gridDim.x - nitemwg, b = blockIdx.x - nitemwg;
+        const int w1 = (int)((long long)total * (b + 1) / nb);
+        int w = (int)((long long)total * b / nb);
+        if (w >= w1) return;
+        int q = 0;  // last member with halo0 <= w
+        for (int hi = nmem - 1; q < hi;) {
+            const int mid = (q + hi + 1) >> 1;
+            if (mem[mid].halo0 <= w) q = mid;
+            else hi = mid - 1;
+        }
+        for (; w < w1; q++) {
+            const Member<T>& m = mem[q];
+            const int end = q + 1 < nmem ? mem[q + 1].halo0 : total;
+            for (const int h0 = m.halo0; w < min(w1, end); w++)
+                copy_untouched_halo<T>(m.g, m.x, m.xo, w - h0, end - h0);
         }
         return;
     }
@@ -1453,7 +1471,7 @@ void tiles_of(const Geo& g, int& ntx, int& nty) {
 
 template <typename T, int RX, int RY>
 int pack_members(const BatchMember<T>* bm, int n, int clen, Member<T>* out) {
-    long long item = 0;
+    long long item = 0, share = 0;
     for (int q = 0; q < n; q++) {
         Member<T>& m = out[q];
         m.g = bm[q].g;
@@ -1464,11 +1482,13 @@ int pack_members(const BatchMember<T>* bm, int n, int clen, Member<T>* out) {
         m.ntile = ntx * nty;
         m.clen = clen < m.g.lp ? clen : m.g.lp;
         m.item0 = (int)item;
+        m.halo0 = (int)share;
+        share += halo_shares(halo_cells(m.g), RX * RY);
         m.x = bm[q].x; m.u1 = bm[q].u1; m.u2 = bm[q].u2; m.u3 = bm[q].u3;
         m.rhr = bm[q].rhr; m.h = bm[q].h; m.bcx = bm[q].bcx; m.bcy = bm[q].bcy;
         m.xo = bm[q].xo;
         item += (long long)m.ntile * ((m.g.lp + m.clen - 1) / m.clen);
-        if (item > (1ll << 30)) return -1;
+        if (item > (1ll << 30) || share > (1ll << 30)) return -1;
     }
     // XCD runs of equal modelled cost: an item marches its chunk's planes
     // plus the two recomputed below and above it (fewer at the lids)
@@ -1499,6 +1519,7 @@ int pack_members(const BatchMember<T>* bm, int n, int clen, Member<T>* out) {
     }
     for (; x <= NXCD; x++) sc->bnd[x] = (int)item;
     for (int d = 0; d < NXCD; d++) sc->next[d] = sc->done[d] = 0;
+    sc->nhalo = (int)share;
     return (int)item;
 }
 
@@ -1525,14 +1546,13 @@ hipError_t launch_batch(const void* table, int n, int nitem, int shared, long lo
     const int grid = persistent_grid(nitem, ((long long)nitem + NXCD - 1) / NXCD, ncu, per_cu);
     BatchSched* sc = reinterpret_cast<BatchSched*>(
         reinterpret_cast<char*>(const_cast<void*>(table)) + sched_offset<T>(n));
-    // Shares of four cells a thread of the largest member's halo, over at most
-    // a block a CU.  (Every block walking all members took 1000 members of
-    // 20x20x10 from 207 to 1190 us a step: their halos were copied one after
-    // the other by the few blocks that one halo fills.)
-    const int hparts = (int)std::max(1LL, (max_halo + 4LL * RX * RY - 1) / (4LL * RX * RY));
-    const int hb = (int)std::min<long long>(std::max(ncu, 1), (long long)n * hparts);
+    // Blocks for the halo shares (pack_members), at most one a CU.  (Every block
+    // walking all members took 1000 members of 20x20x10 from 207 to 1190 us a
+    // step: their halos were copied one after the other by the few blocks that
+    // one halo fills.)
+    const int hb = (int)std::min<long long>(std::max(ncu, 1), n * halo_shares(max_halo, RX * RY));
     k_fused_gauge2_batch<T, RX, RY, MINB, FAST><<<grid + hb, RX * RY, 0, s>>>(
-        (const Member<T>*)table, n, nitem, shared, sc, grid, hparts);
+        (const Member<T>*)table, n, nitem, shared, sc, grid);
     return hipGetLastError();
 }
 

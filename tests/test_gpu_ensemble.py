@@ -371,3 +371,35 @@ def test_fast_build_no_slower_on_any_tiling(mpd):
             exact, fast = min(ms[mpd.PATH_FUSED]), min(ms[mpd.PATH_FAST])
             print(f"{name}: exact {exact:.3f} fast {fast:.3f} ms", flush=True)
             assert fast < exact, (name, fast, exact)
+
+
+def test_halo_cost_beside_a_large_member(mpd):
+    """One large member and 1000 of one tile each in one ensemble take about as
+    long as the two ensembles one after the other: a small member's halo is one
+    share of the copy, whatever the largest member's is."""
+    dtype = torch.float64
+    small, large = (20, 20, 10), (512, 512, 64)
+    ms = {}
+    for name, shapes in (("small", [small] * 1000), ("large", [large]),
+                         ("both", [large] + [small] * 1000)):
+        made = {s: _members(dtype, [s], seed0=7)[0] for s in set(shapes)}
+        members = [made[s] for s in shapes]
+        ens = mpd.Ensemble(shapes, dtype=dtype)
+        xb = [torch.zeros_like(m["x"]) for m in members]
+        ens.set_fields([m["x"] for m in members], xb, *[[m[k] for m in members] for k in
+                       ("u1", "u2", "u3", "rhr", "h", "bcx", "bcy")])
+        with ens:
+            ens.set_tiling(5, 64)
+            best = []
+            for _ in range(5):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                ens.step(0)
+                a.record()
+                for _ in range(20):
+                    ens.step(0)
+                b.record()
+                b.synchronize()
+                best.append(a.elapsed_time(b) / 20)
+            ms[name] = min(best)
+    print(f"1000 small and a large member: {ms}", flush=True)
+    assert ms["both"] < 1.2 * (ms["small"] + ms["large"]), ms
